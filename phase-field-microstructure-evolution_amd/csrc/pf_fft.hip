@@ -14,7 +14,7 @@
 
 #include "../../include/pf.h"
 #include "pf_internal.hpp"
-#include "pf_kernels.hpp"
+#include "pf_passes.hpp"
 
 namespace pf {
 
@@ -233,7 +233,7 @@ template const c2<double>* twiddle_table<double>(int);
 static inline unsigned ceil_div(long a, long b) { return (unsigned)((a + b - 1) / b); }
 
 template <typename R>
-int x_r2c(int nx, c2<R>* data, c2<R>* nyq, long nlines, R scale, hipStream_t s) {
+int x_r2c(int nx, const c2<R>* src, c2<R>* dst, c2<R>* nyq, long nlines, R scale, hipStream_t s) {
   const c2<R>* tw = twiddle_table<R>(nx);
   if (!tw) return fail(PF_EHIP, "twiddle table set-up failed");
   switch (nx) {
@@ -241,7 +241,7 @@ int x_r2c(int nx, c2<R>* data, c2<R>* nyq, long nlines, R scale, hipStream_t s) 
   case N: {                                                                             \
     constexpr int LPB = x_lines<R>(N / 2);                                              \
     hipLaunchKernelGGL((k_x_r2c<R, N>), dim3(ceil_div(nlines, LPB)),                    \
-                       dim3(LPB * plan_T(N / 2)), 0, s, data, nyq, nlines, tw, scale); \
+                       dim3(LPB * plan_T(N / 2)), 0, s, src, dst, nyq, nlines, tw, scale); \
     break;                                                                              \
   }
     PF_GRID_SIZES(PF_CASE)
@@ -252,7 +252,7 @@ int x_r2c(int nx, c2<R>* data, c2<R>* nyq, long nlines, R scale, hipStream_t s) 
 }
 
 template <typename R>
-int x_c2r(int nx, c2<R>* data, const c2<R>* nyq, long nlines, hipStream_t s) {
+int x_c2r(int nx, const c2<R>* src, c2<R>* dst, const c2<R>* nyq, long nlines, hipStream_t s) {
   const c2<R>* tw = twiddle_table<R>(nx);
   if (!tw) return fail(PF_EHIP, "twiddle table set-up failed");
   switch (nx) {
@@ -260,7 +260,7 @@ int x_c2r(int nx, c2<R>* data, const c2<R>* nyq, long nlines, hipStream_t s) {
   case N: {                                                                          \
     constexpr int LPB = x_lines<R>(N / 2);                                           \
     hipLaunchKernelGGL((k_x_c2r<R, N>), dim3(ceil_div(nlines, LPB)),                 \
-                       dim3(LPB * plan_T(N / 2)), 0, s, data, nyq, nlines, tw); \
+                       dim3(LPB * plan_T(N / 2)), 0, s, src, dst, nyq, nlines, tw); \
     break;                                                                           \
   }
     PF_GRID_SIZES(PF_CASE)
@@ -271,164 +271,91 @@ int x_c2r(int nx, c2<R>* data, const c2<R>* nyq, long nlines, hipStream_t s) {
 }
 
 template <typename R>
-int x_c2r_sumsq(int nx, const c2<R>* data, const c2<R>* nyq, long nlines, long lines_per_field, double w0,
-                double w1, double* part, long max_blocks, long* nblocks, hipStream_t s) {
-  const c2<R>* tw = twiddle_table<R>(nx);
+int y_pass(int ny, bool inv, c2<R>* main, c2<R>* nyq, long M, long nlines, hipStream_t s) {
+  const c2<R>* tw = twiddle_table<R>(ny);
   if (!tw) return fail(PF_EHIP, "twiddle table set-up failed");
-  switch (nx) {
-#define PF_CASE(N)                                                                                   \
-  case N: {                                                                                          \
-    constexpr int LPB = x_lines<R>(N / 2);                                                           \
-    const long grid = std::max<long>(1, std::min<long>((nlines + LPB - 1) / LPB, max_blocks));       \
-    hipLaunchKernelGGL((k_x_c2r_sumsq<R, N>), dim3((unsigned)grid), dim3(LPB * plan_T(N / 2)), 0, s, \
-                       data, nyq, nlines, lines_per_field, w0, w1, tw, part);                        \
-    *nblocks = grid;                                                                                 \
-    break;                                                                                           \
+  switch (ny) {
+#define PF_CASE(N)                                                                                     \
+  case N: {                                                                                            \
+    constexpr int TX = col_tile(N, sizeof(c2<R>));                                                     \
+    /* a multiple of 8 blocks for the XCD order (xcd_block); the extra blocks fall on Nyquist lines  */ \
+    /* past the last one and touch no memory                                                         */ \
+    const unsigned tiles = ceil_div(M * nlines, TX) + ceil_div(nlines, TX);                            \
+    dim3 grid((tiles + 7) / 8 * 8), block(TX * plan_T(N));                                             \
+    if (inv)                                                                                           \
+      hipLaunchKernelGGL((k_ypass<R, N, true>), grid, block, 0, s, main, nyq, M, nlines, nlines, tw,   \
+                         (const Member<R>*)nullptr, 0L);                                               \
+    else                                                                                               \
+      hipLaunchKernelGGL((k_ypass<R, N, false>), grid, block, 0, s, main, nyq, M, nlines, nlines, tw,  \
+                         (const Member<R>*)nullptr, 0L);                                               \
+    break;                                                                                             \
   }
     PF_GRID_SIZES(PF_CASE)
 #undef PF_CASE
-    default: return fail(PF_EINVAL, "unsupported nx " + std::to_string(nx));
+    default: return fail(PF_EINVAL, "unsupported ny " + std::to_string(ny));
   }
   return 0;
 }
 
-template <typename R>
-int col_pass(int n, bool inv, c2<R>* data, long W, long npanels, hipStream_t s) {
-  const c2<R>* tw = twiddle_table<R>(n);
+template <typename R, bool INV, int FAR>
+int z_pass(int nz, c2<R>* near, c2<R>* nearn, c2<R>* far, c2<R>* farn, int M, int ny, int nf, hipStream_t s) {
+  const c2<R>* tw = twiddle_table<R>(nz);
   if (!tw) return fail(PF_EHIP, "twiddle table set-up failed");
-  switch (n) {
-#define PF_CASE(N)                                                                          \
-  case N: {                                                                                 \
-    constexpr int TX = col_tile(N, sizeof(c2<R>));                                          \
-    const long tpp = (W + TX - 1) / TX;                                                     \
-    dim3 grid((unsigned)(tpp * npanels)), block(TX * plan_T(N));                       \
-    if (inv)                                                                                \
-      hipLaunchKernelGGL((k_col_fft<R, N, true>), grid, block, 0, s, data, W, tpp, tw);    \
-    else                                                                                    \
-      hipLaunchKernelGGL((k_col_fft<R, N, false>), grid, block, 0, s, data, W, tpp, tw);   \
-    break;                                                                                  \
+  switch (nz) {
+#define PF_CASE(N)                                                                                         \
+  case N: {                                                                                                \
+    constexpr int TX = col_tile(N, sizeof(c2<R>));                                                         \
+    const unsigned tm = ceil_div((long)M * ny, TX), tn = ceil_div(ny, TX), run = ceil_div(M, TX);          \
+    const unsigned tiles = (tm + tn) * (unsigned)nf;                                                       \
+    hipLaunchKernelGGL((k_zpass<R, N, INV, FAR>), dim3(ceil_div(tiles, 8 * run) * 8 * run),                \
+                       dim3(TX * plan_T(N)), 0, s, near, nearn, far, farn, (unsigned)M, (unsigned)ny,      \
+                       (unsigned)nf, tm, tn, run, tw);                                                     \
+    break;                                                                                                 \
   }
     PF_GRID_SIZES(PF_CASE)
 #undef PF_CASE
-    default: return fail(PF_EINVAL, "unsupported axis length " + std::to_string(n));
-  }
-  return 0;
-}
-
-template <typename R>
-int row_pass(int n, bool inv, c2<R>* data, long nlines, hipStream_t s) {
-  const c2<R>* tw = twiddle_table<R>(n);
-  if (!tw) return fail(PF_EHIP, "twiddle table set-up failed");
-  switch (n) {
-#define PF_CASE(N)                                                                      \
-  case N: {                                                                             \
-    constexpr int LPB = lines_per_block(N);                                             \
-    dim3 grid(ceil_div(nlines, LPB)), block(LPB * plan_T(N));                      \
-    if (inv)                                                                            \
-      hipLaunchKernelGGL((k_row_fft<R, N, true>), grid, block, 0, s, data, nlines, tw);  \
-    else                                                                                \
-      hipLaunchKernelGGL((k_row_fft<R, N, false>), grid, block, 0, s, data, nlines, tw); \
-    break;                                                                              \
-  }
-    PF_GRID_SIZES(PF_CASE)
-#undef PF_CASE
-    default: return fail(PF_EINVAL, "unsupported axis length " + std::to_string(n));
+    default: return fail(PF_EINVAL, "unsupported nz " + std::to_string(nz));
   }
   return 0;
 }
 
 #define PF_INST(R)                                                                \
-  template int x_r2c<R>(int, c2<R>*, c2<R>*, long, R, hipStream_t);               \
-  template int x_c2r<R>(int, c2<R>*, const c2<R>*, long, hipStream_t);            \
-  template int x_c2r_sumsq<R>(int, const c2<R>*, const c2<R>*, long, long, double, double, double*, long, \
-                              long*, hipStream_t);                                 \
-  template int col_pass<R>(int, bool, c2<R>*, long, long, hipStream_t);           \
-  template int row_pass<R>(int, bool, c2<R>*, long, hipStream_t);
+  template int x_r2c<R>(int, const c2<R>*, c2<R>*, c2<R>*, long, R, hipStream_t); \
+  template int x_c2r<R>(int, const c2<R>*, c2<R>*, const c2<R>*, long, hipStream_t); \
+  template int y_pass<R>(int, bool, c2<R>*, c2<R>*, long, long, hipStream_t);
 PF_INST(float)
 PF_INST(double)
 #undef PF_INST
 
 // ---------------------------------------------------------------------------
-// Whole 3-D transforms (P3DFFT order: forward x, y, z; inverse z, y, x).
+// Whole 3-D transforms (P3DFFT order: forward x, y, z; inverse z, y, x), three
+// launches each: the x pass takes the caller's real fields into the split
+// layout, the z pass leaves it for the requested one (FAR_*), so neither end
+// needs a copy.
 // ---------------------------------------------------------------------------
-template <typename R>
-int fwd3d(c2<R>* data, c2<R>* nyq, int nx, int ny, int nz, int batch, R scale, hipStream_t s) {
-  const long M = nx / 2;
-  int rc;
-  if ((rc = x_r2c<R>(nx, data, nyq, (long)ny * nz * batch, scale, s))) return rc;
-  if ((rc = col_pass<R>(ny, false, data, M, (long)nz * batch, s))) return rc;
-  if ((rc = row_pass<R>(ny, false, nyq, (long)nz * batch, s))) return rc;
-  if ((rc = col_pass<R>(nz, false, data, M * ny, batch, s))) return rc;
-  if ((rc = col_pass<R>(nz, false, nyq, ny, batch, s))) return rc;
-  return 0;
-}
-
-template <typename R>
-int inv3d(c2<R>* data, c2<R>* nyq, int nx, int ny, int nz, int batch, hipStream_t s) {
-  const long M = nx / 2;
-  int rc;
-  if ((rc = col_pass<R>(nz, true, data, M * ny, batch, s))) return rc;
-  if ((rc = col_pass<R>(nz, true, nyq, ny, batch, s))) return rc;
-  if ((rc = col_pass<R>(ny, true, data, M, (long)nz * batch, s))) return rc;
-  if ((rc = row_pass<R>(ny, true, nyq, (long)nz * batch, s))) return rc;
-  if ((rc = x_c2r<R>(nx, data, nyq, (long)ny * nz * batch, s))) return rc;
-  return 0;
-}
-template int fwd3d<float>(c2<float>*, c2<float>*, int, int, int, int, float, hipStream_t);
-template int fwd3d<double>(c2<double>*, c2<double>*, int, int, int, int, double, hipStream_t);
-template int inv3d<float>(c2<float>*, c2<float>*, int, int, int, int, hipStream_t);
-template int inv3d<double>(c2<double>*, c2<double>*, int, int, int, int, hipStream_t);
-
-// ---------------------------------------------------------------------------
-// Split <-> dense half-spectrum layouts.
-//   XFAST: kx + (M+1)*(ky + ny*(kz + nz*f))     (numpy rfftn of a (nz,ny,nx) array)
-//   ZFAST: kz + nz*(ky + ny*(kx + (M+1)*f))     (P3DFFT STRIDE1 Z-pencil, as f_trans)
-// ---------------------------------------------------------------------------
-template <typename R, bool PACK>
-__global__ void k_layout(const c2<R>* __restrict__ a, c2<R>* __restrict__ b, c2<R>* __restrict__ nq,
-                         int M, int ny, int nz, long total, int layout) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= total) return;
-  const long mx = M + 1;
-  long kx, ky, kz, f;
-  if (layout == LAYOUT_XFAST) {
-    kx = i % mx; long r = i / mx; ky = r % ny; r /= ny; kz = r % nz; f = r / nz;
-  } else {
-    kz = i % nz; long r = i / nz; ky = r % ny; r /= ny; kx = r % mx; f = r / mx;
-  }
-  const long plane = (long)ny * nz;
-  if (PACK) {
-    // a = main (split), nq = nyquist, b = dense
-    const c2<R> v = (kx < M) ? a[kx + M * (ky + ny * (kz + nz * f))] : nq[ky + ny * kz + plane * f];
-    b[i] = v;
-  } else {
-    // a = dense, b = main, nq = nyquist
-    const c2<R> v = a[i];
-    if (kx < M) b[kx + M * (ky + ny * (kz + nz * f))] = v;
-    else nq[ky + ny * kz + plane * f] = v;
-  }
-}
-
-template <typename R>
-int pack_spec(const c2<R>* main, const c2<R>* nyq, c2<R>* dense, int nx, int ny, int nz,
-              int batch, int layout, hipStream_t s) {
-  const long total = (long)(nx / 2 + 1) * ny * nz * batch;
-  hipLaunchKernelGGL((k_layout<R, true>), dim3(ceil_div(total, 256)), dim3(256), 0, s, main, dense,
-                     const_cast<c2<R>*>(nyq), nx / 2, ny, nz, total, layout);
-  return 0;
+template <typename R, int FAR>
+int fwd3d(const c2<R>* src, c2<R>* main, c2<R>* nyq, c2<R>* far, c2<R>* farn, int nx, int ny, int nz, int batch,
+          R scale, hipStream_t s) {
+  const int M = nx / 2;
+  int rc = x_r2c<R>(nx, src, main, nyq, (long)ny * nz * batch, scale, s);
+  if (!rc) rc = y_pass<R>(ny, false, main, nyq, M, (long)nz * batch, s);
+  if (!rc) rc = z_pass<R, false, FAR>(nz, main, nyq, far, farn, M, ny, batch, s);
+  return rc;
 }
 template <typename R>
-int unpack_spec(const c2<R>* dense, c2<R>* main, c2<R>* nyq, int nx, int ny, int nz, int batch,
-                int layout, hipStream_t s) {
-  const long total = (long)(nx / 2 + 1) * ny * nz * batch;
-  hipLaunchKernelGGL((k_layout<R, false>), dim3(ceil_div(total, 256)), dim3(256), 0, s, dense, main,
-                     nyq, nx / 2, ny, nz, total, layout);
-  return 0;
+int fwd3d_split(const c2<R>* src, c2<R>* main, c2<R>* nyq, int nx, int ny, int nz, int batch, R scale, hipStream_t s) {
+  return fwd3d<R, FAR_SPLIT>(src, main, nyq, main, nyq, nx, ny, nz, batch, scale, s);
 }
-template int pack_spec<float>(const c2<float>*, const c2<float>*, c2<float>*, int, int, int, int, int, hipStream_t);
-template int pack_spec<double>(const c2<double>*, const c2<double>*, c2<double>*, int, int, int, int, int, hipStream_t);
-template int unpack_spec<float>(const c2<float>*, c2<float>*, c2<float>*, int, int, int, int, int, hipStream_t);
-template int unpack_spec<double>(const c2<double>*, c2<double>*, c2<double>*, int, int, int, int, int, hipStream_t);
+template <typename R>
+int fwd3d_tiled(const c2<R>* src, c2<R>* main, c2<R>* nyq, c2<R>* tiled, int nx, int ny, int nz, int batch, R scale,
+                hipStream_t s) {
+  return fwd3d<R, FAR_TILED>(src, main, nyq, tiled, nullptr, nx, ny, nz, batch, scale, s);
+}
+template int fwd3d_split<double>(const c2<double>*, c2<double>*, c2<double>*, int, int, int, int, double, hipStream_t);
+template int fwd3d_tiled<float>(const c2<float>*, c2<float>*, c2<float>*, c2<float>*, int, int, int, int, float,
+                                hipStream_t);
+template int fwd3d_tiled<double>(const c2<double>*, c2<double>*, c2<double>*, c2<double>*, int, int, int, int, double,
+                                 hipStream_t);
 
 }  // namespace pf
 
@@ -520,7 +447,12 @@ template <typename R> size_t r2c_scratch_bytes(int nx, int ny, int nz, int batch
   return sizeof(R) * (size_t)nx * ny * nz * batch + sizeof(c2<R>) * (size_t)ny * nz * batch;
 }
 
-// The forward transform with its scratch at ws.
+// Whether complex accesses at p are aligned (a caller's real array need only be
+// aligned for its reals).
+template <typename R> bool complex_aligned(const void* p) { return reinterpret_cast<uintptr_t>(p) % sizeof(c2<R>) == 0; }
+
+// The forward transform with its scratch at ws.  A real array that is not aligned
+// for complex accesses is copied into the scratch first.
 template <typename R>
 int r2c_core(int nx, int ny, int nz, int batch, const void* in, void* out, int layout, double scale,
              void* wsp, hipStream_t s) {
@@ -528,10 +460,14 @@ int r2c_core(int nx, int ny, int nz, int batch, const void* in, void* out, int l
   char* ws = (char*)wsp;
   c2<R>* main = (c2<R>*)ws;
   c2<R>* nyq = (c2<R>*)(ws + sizeof(R) * P * batch);
-  PF_HIP(hipMemcpyAsync(main, in, sizeof(R) * P * batch, hipMemcpyDeviceToDevice, s));
-  int rc = fwd3d<R>(main, nyq, nx, ny, nz, batch, (R)scale, s);
-  if (rc) return rc;
-  rc = pack_spec<R>(main, nyq, (c2<R>*)out, nx, ny, nz, batch, layout, s);
+  const c2<R>* src = (const c2<R>*)in;
+  if (!complex_aligned<R>(in)) {
+    PF_HIP(hipMemcpyAsync(main, in, sizeof(R) * P * batch, hipMemcpyDeviceToDevice, s));
+    src = main;
+  }
+  const int rc = layout == PF_LAYOUT_XFAST
+                     ? fwd3d<R, FAR_XFAST>(src, main, nyq, (c2<R>*)out, nullptr, nx, ny, nz, batch, (R)scale, s)
+                     : fwd3d<R, FAR_ZFAST>(src, main, nyq, (c2<R>*)out, nullptr, nx, ny, nz, batch, (R)scale, s);
   if (rc) return rc;
   PF_HIP(hipGetLastError());
   return 0;
@@ -553,11 +489,15 @@ int c2r_dev(int nx, int ny, int nz, int batch, const void* in, void* out, int la
   char* ws = (char*)lease.p;
   c2<R>* main = (c2<R>*)ws;
   c2<R>* nyq = (c2<R>*)(ws + sizeof(R) * P * batch);
-  int rc = unpack_spec<R>((const c2<R>*)in, main, nyq, nx, ny, nz, batch, layout, s);
+  c2<R>* spec = (c2<R>*)const_cast<void*>(in);  // read only
+  int rc = layout == PF_LAYOUT_XFAST ? z_pass<R, true, FAR_XFAST>(nz, main, nyq, spec, nullptr, nx / 2, ny, batch, s)
+                                     : z_pass<R, true, FAR_ZFAST>(nz, main, nyq, spec, nullptr, nx / 2, ny, batch, s);
+  if (!rc) rc = y_pass<R>(ny, true, main, nyq, nx / 2, (long)nz * batch, s);
+  // a real array not aligned for complex stores is filled by a copy
+  const bool direct = complex_aligned<R>(out);
+  if (!rc) rc = x_c2r<R>(nx, main, direct ? (c2<R>*)out : main, nyq, (long)ny * nz * batch, s);
   if (rc) return rc;
-  rc = inv3d<R>(main, nyq, nx, ny, nz, batch, s);
-  if (rc) return rc;
-  PF_HIP(hipMemcpyAsync(out, main, sizeof(R) * P * batch, hipMemcpyDeviceToDevice, s));
+  if (!direct) PF_HIP(hipMemcpyAsync(out, main, sizeof(R) * P * batch, hipMemcpyDeviceToDevice, s));
   PF_HIP(hipGetLastError());
   return 0;
 }

@@ -11,26 +11,9 @@
 // so each field's half spectrum crosses HBM 10 times per step (x: 2, y: 2+2,
 // z: 4 including S), against 17 for separate transform and pointwise passes.
 #pragma once
-#include "pf_kernels.hpp"
-#include "pf_step_kernels.hpp"
+#include "pf_passes.hpp"
 
 namespace pf {
-
-struct UPar {
-  double dt, kphi, kc, D, L, Dgb, am, ap, cm, cp, s1g, s2g, invP;
-};
-
-// One simulation of a batched ensemble (a device table of these drives the
-// BATCH forms of the step kernels: one launch per stage covers every member of
-// one grid shape): its carried spectrum S (column-tile layout, below), work
-// bank W, FP64 k = 0 modes and parameters.
-template <typename R> struct Member {
-  c2<R>* Wm;
-  c2<R>* Wn;
-  c2<R>* S;
-  double* dc64;
-  UPar u;
-};
 
 // Deterministic block reductions for any blockDim (multiple of 64).
 __device__ __forceinline__ double wave_sum(double v) {
@@ -642,67 +625,6 @@ k_xline(Geo g, UPar u, c2<R>* __restrict__ wm, c2<R>* __restrict__ wn, R* __rest
       double* o = part + (long)blockIdx.x * 6;
       o[0] = s0; o[1] = s1; o[2] = e0; o[3] = e1; o[4] = e2; o[5] = e3;
     }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// k_ypass: y transform of the main block (column tiles of W = M, panels (z, f))
-// and of the Nyquist planes (contiguous lines of length NY), one launch.
-// ---------------------------------------------------------------------------
-// BATCH: the W banks of every member in mt, ppm panels (and Nyquist lines) per
-// member (fields x nz); main and nyq are unused.
-template <typename R, int NY, bool INV, bool BATCH = false>
-__global__ void __launch_bounds__(col_tile(NY, sizeof(c2<R>)) * plan_T(NY))
-k_ypass(c2<R>* __restrict__ main, c2<R>* __restrict__ nyq, long M, long npanels, long nlines,
-        const c2<R>* __restrict__ tw, const Member<R>* __restrict__ mt, long ppm) {
-  constexpr int T = plan_T(NY), E = plan_E(NY);
-  constexpr int TX = col_tile(NY, sizeof(c2<R>));
-  __shared__ c2<R> sh[(plan_np(NY) > 1) ? NY * TX : 1];
-  const long tpp = (M + TX - 1) / TX;
-  const long nmain = tpp * npanels;
-  const long b = xcd_block(blockIdx.x, gridDim.x);
-  c2<R> v[E];
-  if (b < nmain) {
-    const long pl = b / tpp;
-    long pnl = pl;
-    c2<R>* mb = main;
-    if constexpr (BATCH) {
-      const long m = pl / ppm;
-      pnl = pl - m * ppm;
-      mb = mt[m].Wm;
-    }
-    const long col0 = (b - pl * tpp) * TX;
-    const int ncol = (int)((M - col0) < TX ? (M - col0) : TX);
-    const int c = threadIdx.x % TX, t = threadIdx.x / TX;
-    const bool act = c < ncol;
-    c2<R>* gp = mb + pnl * NY * M + col0 + c;
-#pragma unroll
-    for (int s = 0; s < kInSlots<NY>; ++s)
-      if (act && rfft_in_valid<NY>(t, s)) v[s] = ld_nt<R>(gp + (long)rfft_in_idx<NY>(t, s) * M);
-    rfft<R, NY, INV, TX>(v, t, act, sh + c, tw);
-#pragma unroll
-    for (int s = 0; s < kOutSlots<NY>; ++s)
-      if (act && rfft_out_valid<NY>(t, s)) st_nt<R>(gp + (long)rfft_out_idx<NY>(t, s) * M, v[s]);
-  } else {
-    const int l = threadIdx.x / T, t = threadIdx.x % T;
-    const long line = (b - nmain) * TX + l;
-    const bool act = line < nlines;
-    long gl = line;
-    c2<R>* nb = nyq;
-    if constexpr (BATCH) {
-      const long ln = act ? line : 0;
-      const long m = ln / ppm;
-      gl = ln - m * ppm;
-      nb = mt[m].Wn;
-    }
-    c2<R>* gp = nb + (act ? gl : 0) * NY;
-#pragma unroll
-    for (int s = 0; s < kInSlots<NY>; ++s)
-      if (act && rfft_in_valid<NY>(t, s)) v[s] = ld_nt<R>(gp + rfft_in_idx<NY>(t, s));
-    rfft<R, NY, INV, 1>(v, t, act, sh + ((plan_np(NY) > 1) ? l * NY : 0), tw);
-#pragma unroll
-    for (int s = 0; s < kOutSlots<NY>; ++s)
-      if (act && rfft_out_valid<NY>(t, s)) st_nt<R>(gp + rfft_out_idx<NY>(t, s), v[s]);
   }
 }
 

@@ -28,30 +28,27 @@ const char* supported_sizes_text();
 // Device table of exp(-2 pi i q/n), q in [0, n), in precision R (cached per device).
 template <typename R> const c2<R>* twiddle_table(int n);
 
-// Whole-axis transforms over a batch of fields in the split-Nyquist layout.
-//   data: batch * (nx/2)*ny*nz complex == batch * nx*ny*nz reals (in place)
+// Whole 3-D forward transforms of a batch of real fields at src: the passes run in
+// the split-Nyquist layout at main, nyq
+//   main: batch * (nx/2)*ny*nz complex == batch * nx*ny*nz reals (may be src)
 //   nyq : batch * ny*nz complex
+// and leave the spectrum there (fwd3d_split), or in the column-tile layout of the
+// carried spectrum at tiled (fwd3d_tiled).
 template <typename R>
-int fwd3d(c2<R>* data, c2<R>* nyq, int nx, int ny, int nz, int batch, R scale, hipStream_t s);
+int fwd3d_split(const c2<R>* src, c2<R>* main, c2<R>* nyq, int nx, int ny, int nz, int batch, R scale, hipStream_t s);
 template <typename R>
-int inv3d(c2<R>* data, c2<R>* nyq, int nx, int ny, int nz, int batch, hipStream_t s);
+int fwd3d_tiled(const c2<R>* src, c2<R>* main, c2<R>* nyq, c2<R>* tiled, int nx, int ny, int nz, int batch, R scale,
+                hipStream_t s);
 
-// Individual passes (used by the step pipelines).
+// Individual passes (used by the step pipelines).  x: real lines at src to half
+// lines at dst and back (src == dst in place); y: nlines = panels of M columns,
+// and as many Nyquist-plane lines, in one launch.
 template <typename R>
-int x_r2c(int nx, c2<R>* data, c2<R>* nyq, long nlines, R scale, hipStream_t s);
+int x_r2c(int nx, const c2<R>* src, c2<R>* dst, c2<R>* nyq, long nlines, R scale, hipStream_t s);
 template <typename R>
-int x_c2r(int nx, c2<R>* data, const c2<R>* nyq, long nlines, hipStream_t s);
+int x_c2r(int nx, const c2<R>* src, c2<R>* dst, const c2<R>* nyq, long nlines, hipStream_t s);
 template <typename R>
-int col_pass(int n, bool inv, c2<R>* data, long W, long npanels, hipStream_t s);
-// Inverse x pass of a batch of gradient fields reduced to
-// sum_lines w * sum_points out^2 (w = w0 for the lines of gradient fields 0-2,
-// w1 after), one partial per block (at most max_blocks) in part.
-template <typename R>
-int x_c2r_sumsq(int nx, const c2<R>* data, const c2<R>* nyq, long nlines, long lines_per_field, double w0,
-                double w1, double* part, long max_blocks, long* nblocks, hipStream_t s);
-template <typename R>
-int row_pass(int n, bool inv, c2<R>* data, long nlines, hipStream_t s);
-
+int y_pass(int ny, bool inv, c2<R>* main, c2<R>* nyq, long M, long nlines, hipStream_t s);
 // Copies between device memory and the caller's (pageable) host arrays on
 // stream s; both return once the copy has finished.  Copies of 128 MiB and more
 // go through two pinned bounce buffers of 64 MiB (process-wide, made on first
@@ -59,14 +56,5 @@ int row_pass(int n, bool inv, c2<R>* data, long nlines, hipStream_t s);
 // between the other buffer and the caller's array.
 int to_host(void* dst, const void* src, size_t bytes, hipStream_t s);
 int to_device(void* dst, const void* src, size_t bytes, hipStream_t s);
-
-// Dense half-spectrum layouts at the C-ABI.
-enum { LAYOUT_XFAST = 0, LAYOUT_ZFAST = 1 };
-template <typename R>
-int pack_spec(const c2<R>* main, const c2<R>* nyq, c2<R>* dense, int nx, int ny, int nz,
-              int batch, int layout, hipStream_t s);
-template <typename R>
-int unpack_spec(const c2<R>* dense, c2<R>* main, c2<R>* nyq, int nx, int ny, int nz,
-                int batch, int layout, hipStream_t s);
 
 }  // namespace pf

@@ -63,58 +63,7 @@ __device__ __forceinline__ long xcd_runs(long b, long nb, long G) {
   return (i / G) * (8 * G) + x * G + i % G;
 }
 
-// ---------------------------------------------------------------------------
-// Column pass: FFT along the rows of row-major panels (N rows x W columns),
-// batch of panels at stride N*W.  Used for y (W = M, one panel per (z, field))
-// and z (W = M*NY, one panel per field; W = NY for the Nyquist planes).
-// ---------------------------------------------------------------------------
-template <typename R, int N, bool INV>
-__global__ void __launch_bounds__(col_tile(N, sizeof(c2<R>)) * plan_T(N))
-k_col_fft(c2<R>* __restrict__ data, long W, long tiles_per_panel, const c2<R>* __restrict__ tw) {
-  constexpr int E = plan_E(N);
-  constexpr int TX = col_tile(N, sizeof(c2<R>));
-  __shared__ c2<R> sh[(plan_np(N) > 1) ? N * TX : 1];
-  const long bid = xcd_block(blockIdx.x, gridDim.x);
-  const long b = bid / tiles_per_panel;
-  const long col0 = (bid - b * tiles_per_panel) * TX;
-  const int ncol = (int)((W - col0) < TX ? (W - col0) : TX);
-  const int c = threadIdx.x % TX, t = threadIdx.x / TX;
-  const bool act = c < ncol;
-  c2<R>* g = data + b * N * W + col0 + c;
-  c2<R> v[E];
-#pragma unroll
-  for (int s = 0; s < kInSlots<N>; ++s)
-    if (act && rfft_in_valid<N>(t, s)) v[s] = ld_nt<R>(g + (long)rfft_in_idx<N>(t, s) * W);
-  rfft<R, N, INV, TX>(v, t, act, sh + c, tw);
-#pragma unroll
-  for (int s = 0; s < kOutSlots<N>; ++s)
-    if (act && rfft_out_valid<N>(t, s)) st_nt<R>(g + (long)rfft_out_idx<N>(t, s) * W, v[s]);
-}
-
-// ---------------------------------------------------------------------------
-// Row pass: FFT of contiguous complex lines of length N (Nyquist-plane y pass).
-// ---------------------------------------------------------------------------
-template <typename R, int N, bool INV>
-__global__ void __launch_bounds__(lines_per_block(N) * plan_T(N))
-k_row_fft(c2<R>* __restrict__ data, long nlines, const c2<R>* __restrict__ tw) {
-  constexpr int T = plan_T(N), E = plan_E(N);
-  constexpr int LPB = lines_per_block(N);
-  __shared__ c2<R> sh[(plan_np(N) > 1) ? LPB * N : 1];
-  const int l = threadIdx.x / T, t = threadIdx.x % T;
-  const long line = (long)blockIdx.x * LPB + l;
-  const bool act = line < nlines;
-  c2<R>* g = data + (act ? line : 0) * N;
-  c2<R> v[E];
-#pragma unroll
-  for (int s = 0; s < kInSlots<N>; ++s)
-    if (act && rfft_in_valid<N>(t, s)) v[s] = ld_nt<R>(g + rfft_in_idx<N>(t, s));
-  rfft<R, N, INV, 1>(v, t, act, sh + ((plan_np(N) > 1) ? l * N : 0), tw);
-#pragma unroll
-  for (int s = 0; s < kOutSlots<N>; ++s)
-    if (act && rfft_out_valid<N>(t, s)) st_nt<R>(g + rfft_out_idx<N>(t, s), v[s]);
-}
-
-// Lines per block of the x passes (k_x_r2c, k_x_c2r, k_x_c2r_sumsq).  FP64:
+// Lines per block of the x passes (k_x_r2c, k_x_c2r).  FP64:
 // blocks of one wave (e.g. 8 lines of 8 threads at NX = 256), a 16 KiB tile
 // instead of 64 KiB, which held blocks to two per CU; measured for 17 fields at
 // 256^3: R2C 0.90 -> 0.85 ms, C2R 1.19 -> 1.13 ms.  FP32: lines_per_block.
@@ -155,12 +104,14 @@ __device__ __forceinline__ c2<R> c2r_z(const c2<R>* x, R xn, int k, const c2<R>*
 
 // ---------------------------------------------------------------------------
 // x pass, forward: real lines (NX) -> half spectrum lines (M main + 1 Nyquist).
-// data: in/out (real lines == main block); nyq: Nyquist entries, one per line.
-// tw:   table of exp(-2 pi i q/NX), q in [0, NX).
+// src: real lines; dst: main block (the same memory for an in-place pass: a line
+// is read whole, through LDS, before any of it is written); nyq: Nyquist
+// entries, one per line.
+// tw:  table of exp(-2 pi i q/NX), q in [0, NX).
 // ---------------------------------------------------------------------------
 template <typename R, int NX>
 __global__ void __launch_bounds__(x_lines<R>(NX / 2) * plan_T(NX / 2))
-k_x_r2c(c2<R>* __restrict__ data, c2<R>* __restrict__ nyq, long nlines,
+k_x_r2c(const c2<R>* src, c2<R>* dst, c2<R>* __restrict__ nyq, long nlines,
         const c2<R>* __restrict__ tw, R scale) {
   constexpr int M = NX / 2, T = plan_T(M), E = plan_E(M);
   constexpr int LPB = x_lines<R>(M), NT = LPB * T;
@@ -169,11 +120,12 @@ k_x_r2c(c2<R>* __restrict__ data, c2<R>* __restrict__ nyq, long nlines,
   const int nl = (int)((nlines - l0) < LPB ? (nlines - l0) : LPB);
   const int l = threadIdx.x / T, t = threadIdx.x % T;
   const bool act = l < nl;
-  c2<R>* g = data + l0 * M;
+  const c2<R>* gs = src + l0 * M;
+  c2<R>* g = dst + l0 * M;
   c2<R> v[E];
 #pragma unroll
   for (int s = 0; s < kInSlots<M>; ++s)
-    if (act && rfft_in_valid<M>(t, s)) v[s] = ld_nt<R>(g + (long)l * M + rfft_in_idx<M>(t, s));
+    if (act && rfft_in_valid<M>(t, s)) v[s] = ld_nt<R>(gs + (long)l * M + rfft_in_idx<M>(t, s));
   c2<R>* line = sh + l * M;
   rfft<R, M, false, 1>(v, t, act, line, tw, 2);
   __syncthreads();
@@ -194,11 +146,13 @@ k_x_r2c(c2<R>* __restrict__ data, c2<R>* __restrict__ nyq, long nlines,
 }
 
 // ---------------------------------------------------------------------------
-// x pass, inverse: half spectrum lines -> real lines (unnormalised).
+// x pass, inverse: half spectrum lines -> real lines (unnormalised); src and dst
+// may be the same memory (one-pass lengths hold a line in one thread, the others
+// pass a barrier between a block's reads and its writes).
 // ---------------------------------------------------------------------------
 template <typename R, int NX>
 __global__ void __launch_bounds__(x_lines<R>(NX / 2) * plan_T(NX / 2))
-k_x_c2r(c2<R>* __restrict__ data, const c2<R>* __restrict__ nyq, long nlines,
+k_x_c2r(const c2<R>* src, c2<R>* dst, const c2<R>* __restrict__ nyq, long nlines,
         const c2<R>* __restrict__ tw) {
   constexpr int M = NX / 2, T = plan_T(M), E = plan_E(M);
   constexpr int LPB = x_lines<R>(M);
@@ -206,7 +160,8 @@ k_x_c2r(c2<R>* __restrict__ data, const c2<R>* __restrict__ nyq, long nlines,
   const int l = threadIdx.x / T, t = threadIdx.x % T;
   const long line = (long)blockIdx.x * LPB + l;
   const bool act = line < nlines;
-  c2<R>* g = data + (act ? line : 0) * M;
+  const c2<R>* g = src + (act ? line : 0) * M;
+  c2<R>* gd = dst + (act ? line : 0) * M;
   c2<R> v[E];
   // pre-processing from HBM straight into registers (X_k and X_{M-k} of the line)
 #pragma unroll
@@ -223,59 +178,7 @@ k_x_c2r(c2<R>* __restrict__ data, const c2<R>* __restrict__ nyq, long nlines,
   rfft<R, M, true, 1>(v, t, act, sh + ((plan_np(M) > 1) ? l * M : 0), tw, 2);
 #pragma unroll
   for (int s = 0; s < kOutSlots<M>; ++s)
-    if (act && rfft_out_valid<M>(t, s)) st_nt<R>(g + rfft_out_idx<M>(t, s), v[s]);
-}
-
-// ---------------------------------------------------------------------------
-// x pass, inverse, reduced to weighted sums of squares instead of stored: for
-// the gradient-energy sum of a batch of gradient fields (three per state field,
-// lines_per_field lines each), w = w0 for state field 0 and w1 for the others.
-// Block partials (fixed order) in part[blockIdx.x].
-// ---------------------------------------------------------------------------
-template <typename R, int NX>
-__global__ void __launch_bounds__(x_lines<R>(NX / 2) * plan_T(NX / 2))
-k_x_c2r_sumsq(const c2<R>* __restrict__ data, const c2<R>* __restrict__ nyq, long nlines, long lines_per_field,
-              double w0, double w1, const c2<R>* __restrict__ tw, double* __restrict__ part) {
-  constexpr int M = NX / 2, T = plan_T(M), E = plan_E(M);
-  constexpr int LPB = x_lines<R>(M), NT = LPB * T;
-  __shared__ c2<R> sh[(plan_np(M) > 1) ? LPB * M : 1];
-  __shared__ double red[NT / 64 + 1];
-  const int l = threadIdx.x / T, t = threadIdx.x % T;
-  double acc = 0.0;
-  const long ngroups = (nlines + LPB - 1) / LPB;
-  for (long grp = blockIdx.x; grp < ngroups; grp += gridDim.x) {
-    const long line = grp * LPB + l;
-    const bool act = line < nlines;
-    const c2<R>* g = data + (act ? line : 0) * M;
-    c2<R> v[E];
-#pragma unroll
-    for (int s = 0; s < kInSlots<M>; ++s) {
-      if (!(act && rfft_in_valid<M>(t, s))) continue;
-      const int k = rfft_in_idx<M>(t, s);
-      if (k == 0) {
-        const R a0 = g[0].x, xn = nyq[line].x;
-        v[s] = mk<R>(a0 + xn, a0 - xn);
-      } else {
-        v[s] = c2r_pre<R>(g[k], g[M - k], tw[k]);
-      }
-    }
-    rfft<R, M, true, 1>(v, t, act, sh + ((plan_np(M) > 1) ? l * M : 0), tw, 2);
-    double q = 0.0;
-#pragma unroll
-    for (int s = 0; s < kOutSlots<M>; ++s)
-      if (act && rfft_out_valid<M>(t, s)) q += (double)v[s].x * v[s].x + (double)v[s].y * v[s].y;
-    if (act) acc += ((line / lines_per_field) / 3 == 0 ? w0 : w1) * q;
-    __syncthreads();  // the next group reuses the exchange tile
-  }
-  // block reduction in a fixed order
-  for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double sum = 0.0;
-    for (int w = 0; w < (NT + 63) / 64; ++w) sum += red[w];
-    part[blockIdx.x] = sum;
-  }
+    if (act && rfft_out_valid<M>(t, s)) st_nt<R>(gd + rfft_out_idx<M>(t, s), v[s]);
 }
 
 }  // namespace pf

@@ -13,8 +13,8 @@
 
 #include "../../include/pf.h"
 #include "pf_internal.hpp"
+#include "pf_faithful.hpp"
 #include "pf_fused.hpp"
-#include "pf_step_kernels.hpp"
 
 namespace pf {
 double kaxis(int m, int n, bool zero_nyquist);
@@ -107,100 +107,6 @@ __global__ void __launch_bounds__(NB) k_voronoi_state(Geo g, const double* __res
 }
 
 // ---------------------------------------------------------------------------
-// Loops 5-10, faithful form (src/var_diff.f90:685-905), FP64, O(var^2).
-// Reads the real state bank (c, eta_i); writes df_dc, df_dphi_i, mob_c.
-// ---------------------------------------------------------------------------
-// gamma_ij of src/var_diff.f90:206-218 (the matrix pf_gamma builds): sigma_1
-// between two distinct matrix grains, sigma_2 between a grain and the
-// precipitate field eta_var (index mat), 0 on the diagonal.  Selected from (i, j)
-// instead of loaded: the same double values, without 2 V^2 loads per point.
-__device__ __forceinline__ double gam_ij(const UCoef& u, int mat, int i, int j) {
-  return (i == j) ? 0.0 : ((i == mat || j == mat) ? u.s2g : u.s1g);
-}
-
-template <bool DIAG>
-__global__ void __launch_bounds__(NB)
-k_nl_faithful(Geo g, UCoef u, const double* __restrict__ st,
-              double* __restrict__ dfdc, double* __restrict__ dfdphi, double* __restrict__ mob,
-              double* __restrict__ part) {
-  extern __shared__ double sh[];  // var * NB values, then NB reduction scratch
-  double* red = sh + (long)g.var * NB;
-  const int V = g.var, mat = V - 1;
-  double a_ch = 0.0, a_eta = 0.0, cmax = 0.0, cmin = 1.0, pmin = 1.0, p3 = 0.0;
-  for (long base = (long)blockIdx.x * NB; base < g.P; base += (long)gridDim.x * NB) {
-    const long t = base + threadIdx.x;
-    const bool ok = t < g.P;
-    __syncthreads();
-    for (int i = 0; i < V; ++i) sh[i * NB + threadIdx.x] = ok ? st[(long)(i + 1) * g.P + t] : 0.0;
-    __syncthreads();
-    if (!ok) continue;
-    const double* ph = sh + threadIdx.x;
-    const double con = st[t];
-    // loop 5
-    double fe = 0.0;
-    for (int i = 0; i < V; ++i) {
-      const double fi = ph[i * NB], fi2 = fi * fi;
-      fe = (fe - 0.5 * fi2) + 0.25 * (fi2 * fi2);
-      for (int j = i + 1; j < V; ++j) {
-        const double fj = ph[j * NB];
-        fe = fe + ((gam_ij(u, mat, i, j) * fi2) * (fj * fj));
-      }
-    }
-    // loop 6
-    double num = 0.0, den = 0.0;
-    for (int i = 0; i < V; ++i) {
-      const double f2 = ph[i * NB] * ph[i * NB], f4 = f2 * f2;
-      if (i < mat) num = num + f4;
-      den = den + f4;
-    }
-    const double hm = num / den, hp = 1.0 - hm;
-    const double dm = con - u.cm, dp = con - u.cp;
-    const double fch = (hm * u.am) * (dm * dm) + (hp * u.ap) * (dp * dp);
-    dfdc[t] = ((2.0 * hm) * u.am) * dm + ((2.0 * hp) * u.ap) * dp;
-    // loops 7-9
-    const double fm = u.am * (dm * dm), fp = u.ap * (dp * dp);
-    const double fv = ph[mat * NB], fv2 = fv * fv, fv4 = fv2 * fv2;
-    const double t2v = (4.0 * (fv2 * fv)) * (den - fv4);
-    const double den2 = den * den;
-    double ps = 0.0;
-    for (int i = 0; i < V; ++i) {
-      const double fi = ph[i * NB];
-      const double term1 = (fi * fi) * fi - fi;
-      double term2 = 0.0;
-      for (int j = 0; j < V; ++j) {
-        if (j == i) continue;
-        const double fj = ph[j * NB];
-        term2 = term2 + ((2.0 * gam_ij(u, mat, i, j)) * fi) * (fj * fj);
-      }
-      const double term4 = (i < mat) ? (((4.0 * ((fi * fi) * fi)) * fv4) * (fm - fp)) / den2
-                                     : (t2v * (fp - fm)) / den2;
-      dfdphi[(long)i * g.P + t] = (term1 + term2) + term4;
-      ps = ps + fi * fi;
-    }
-    // loop 10: mob_c = D_bulk(var) + 2(1 - sum phi^2) D_gb, D_bulk(var) = D_L
-    mob[t] = u.D + ((2.0 * (1.0 - ps)) * u.Dgb);
-    if (DIAG) {
-      a_ch += fch;
-      a_eta += fe;
-      if (fv > p3) p3 = fv;
-      if (con <= cmin) cmin = con;
-      if (con > cmax) cmax = con;
-      if (ps < pmin) pmin = ps;
-    }
-  }
-  if (DIAG) {
-    __syncthreads();
-    const double s0 = block_sum<NB>(a_ch, red), s1 = block_sum<NB>(a_eta, red);
-    const double e0 = block_ext<NB, true>(cmax, red), e1 = block_ext<NB, false>(cmin, red);
-    const double e2 = block_ext<NB, false>(pmin, red), e3 = block_ext<NB, true>(p3, red);
-    if (threadIdx.x == 0) {
-      double* o = part + (long)blockIdx.x * NPART_NL;
-      o[0] = s0; o[1] = s1; o[2] = e0; o[3] = e1; o[4] = e2; o[5] = e3;
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
 // Loops 5-10, reduced form: O(var) per point using the block structure of gamma
 // (sigma_1 between matrix grains, sigma_2 between a grain and eta_var,
 // src/var_diff.f90:206-218).  In place on the real work bank:
@@ -276,121 +182,6 @@ k_nl_reduced(Geo g, UCoef u, R* __restrict__ w, R* __restrict__ mobd, double* __
 }
 
 // ---------------------------------------------------------------------------
-// Faithful k-space kernels (FP64).  One block per (ky, kz, field) row, threads
-// over kx in [0, M] (kx = M: Nyquist plane).  Grid-stride over rows.
-// ---------------------------------------------------------------------------
-
-#define PF_FAITHFUL_SIZES(X) \
-  X(8) X(12) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(160) X(192) X(256) X(512)
-
-// Loops 1 and 3 (dft_grad_d = dft * kf_d, src/var_diff.f90:577-579, 645-647)
-// fused with the first inverse pass of the gradients: for
-// every z column of state field f, the three gradient spectra i a'_d u^
-// (a' = Nyquist-zeroed wavenumbers) are formed in registers, transformed back
-// along z and stored as gradient fields 3f+d; the spectra themselves are never
-// stored.  NYQ: the Nyquist planes (columns = ky, a'_x = 0).
-template <int NZ, bool NYQ>
-__global__ void __launch_bounds__(col_tile(NZ, sizeof(double2)) * plan_T(NZ))
-k_grad_zinv(Geo g, KTab kt, const double2* __restrict__ src, double2* __restrict__ dst, long W,
-            long tiles_per_field, const double2* __restrict__ tw) {
-  constexpr int E = plan_E(NZ);
-  constexpr int TX = col_tile(NZ, sizeof(double2));
-  __shared__ double2 sh[(plan_np(NZ) > 1) ? NZ * TX : 1];
-  const long f = blockIdx.x / tiles_per_field;
-  const long col0 = (blockIdx.x - f * tiles_per_field) * TX;
-  const int ncol = (int)((W - col0) < TX ? (W - col0) : TX);
-  const int c = threadIdx.x % TX, t = threadIdx.x / TX;
-  const bool act = c < ncol;
-  const long col = col0 + (act ? c : 0);
-  const double ax = NYQ ? kt.axp[g.M] : kt.axp[col % g.M];
-  const double ay = NYQ ? kt.ayp[col] : kt.ayp[col / g.M];
-  const double2* in = src + f * NZ * W + col;
-  double2 u[E], v[E];
-#pragma unroll
-  for (int s = 0; s < kInSlots<NZ>; ++s)
-    if (act && rfft_in_valid<NZ>(t, s)) u[s] = in[(long)rfft_in_idx<NZ>(t, s) * W];
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-#pragma unroll
-    for (int s = 0; s < kInSlots<NZ>; ++s) {
-      if (!(act && rfft_in_valid<NZ>(t, s))) continue;
-      const double a = (d == 0) ? ax : (d == 1) ? ay : kt.azp[rfft_in_idx<NZ>(t, s)];
-      v[s] = make_double2(-(u[s].y * a), u[s].x * a);
-    }
-    if (d > 0) __syncthreads();  // the exchange tile is reused
-    rfft<double, NZ, true, TX>(v, t, act, sh + c, tw);
-    double2* out = dst + (3 * f + d) * NZ * W + col;
-#pragma unroll
-    for (int s = 0; s < kOutSlots<NZ>; ++s)
-      if (act && rfft_out_valid<NZ>(t, s)) out[(long)rfft_out_idx<NZ>(t, s) * W] = v[s];
-  }
-}
-
-
-// loop 11: dft_dummy = kf_sum*dft_df_dc - grad_coeff_c*dft_con*k_cube  (src/var_diff.f90:932-936)
-template <typename R>
-__global__ void k_ghat(Geo g, UCoef u, KTab kt, Bank<R> fhat, int ff, Bank<R> chat, int cf,
-                       Bank<R> out, long nrows) {
-  for (long row = blockIdx.x; row < nrows; row += gridDim.x) {
-    const RowIdx r = row_decode(g, row);
-    for (int kx = threadIdx.x; kx <= g.M; kx += blockDim.x) {
-      const KCoef k = kcoef(kt, kx, r.ky, r.kz);
-      const c2<R> f = *elem(fhat, g, ff, kx, r.ky, r.kz);
-      const c2<R> c = *elem(chat, g, cf, kx, r.ky, r.kz);
-      const double kcr = u.kc * (double)c.x, kci = u.kc * (double)c.y;
-      const double re = -(k.s1 * (double)f.y) - (-(kci * k.k3));
-      const double im = (k.s1 * (double)f.x) - (kcr * k.k3);
-      *elem(out, g, 0, kx, r.ky, r.kz) = mk<R>((R)re, (R)im);
-    }
-  }
-}
-
-// loop 12: dummy = dummy*(mob_c - D_mean)  (src/var_diff.f90:956)
-__global__ void k_mult_faithful(long P, double D, double* __restrict__ x, const double* __restrict__ mob) {
-  for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < P; t += (long)gridDim.x * blockDim.x)
-    x[t] = x[t] * (mob[t] - D);
-}
-template <typename R>
-__global__ void k_mult(long P, R* __restrict__ x, const R* __restrict__ m) {
-  for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < P; t += (long)gridDim.x * blockDim.x)
-    x[t] = x[t] * m[t];
-}
-
-// loop 13: dft_con = (dft_con + term11 + term33) / term22  (src/var_diff.f90:978-987)
-__global__ void k_ch_faithful(Geo g, UCoef u, KTab kt, Bank<double> st, Bank<double> hhat,
-                              Bank<double> fhat, long nrows) {
-  for (long row = blockIdx.x; row < nrows; row += gridDim.x) {
-    const RowIdx r = row_decode(g, row);
-    for (int kx = threadIdx.x; kx <= g.M; kx += blockDim.x) {
-      const KCoef k = kcoef(kt, kx, r.ky, r.kz);
-      double2* cp = elem(st, g, 0, kx, r.ky, r.kz);
-      const double2 c = *cp, h = *elem(hhat, g, 0, kx, r.ky, r.kz), f = *elem(fhat, g, 0, kx, r.ky, r.kz);
-      const double t11r = -((h.y * u.dt) * k.s1), t11i = (h.x * u.dt) * k.s1;
-      const double t22 = 1.0 + ((u.D * u.dt) * u.kc) * k.k4;
-      const double r33 = (u.D * k.k2) * u.dt;
-      const double nr = (c.x + t11r) + r33 * f.x, ni = (c.y + t11i) + r33 * f.y;
-      *cp = make_double2(nr / t22, ni / t22);
-    }
-  }
-}
-
-// loop 14: dft_dummy = (dft_dummy - mob_phi*t_step*dft_dummy2) / (1 - mob_phi*kappa*t_step*k_sq)
-// (src/var_diff.f90:1019-1027); fields 1..var of the state bank, df_dphi bank 0..var-1.
-__global__ void k_ac_faithful(Geo g, UCoef u, KTab kt, Bank<double> st, Bank<double> dpsi, long nrows) {
-  const double ldt = u.L * u.dt, lkd = (u.L * u.kphi) * u.dt;
-  for (long row = blockIdx.x; row < nrows; row += gridDim.x) {
-    const RowIdx r = row_decode(g, row);  // r.f in [0, var)
-    for (int kx = threadIdx.x; kx <= g.M; kx += blockDim.x) {
-      const KCoef k = kcoef(kt, kx, r.ky, r.kz);
-      double2* sp = elem(st, g, r.f + 1, kx, r.ky, r.kz);
-      const double2 s = *sp, p = *elem(dpsi, g, r.f, kx, r.ky, r.kz);
-      const double t22 = 1.0 - lkd * k.k2;
-      *sp = make_double2((s.x - ldt * p.x) / t22, (s.y - ldt * p.y) / t22);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
 // Reduced k-space update for all fields, in place on S, copy into W for the
 // inverse transform; optional Parseval partial sums of the new state for the
 // next step's f_int.  FP32 form keeps each field's k = 0 mode in FP64 (dc64).
@@ -445,29 +236,6 @@ k_update(Geo g, UCoef u, KTab kt, Bank<R> S, Bank<R> W, Bank<R> H, double* __res
   if (PARSEVAL) {
     const double s = block_sum<NB>(acc, red);
     if (threadIdx.x == 0) part[blockIdx.x] = s * (double)g.P;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// A spectrum in the natural layout (main block, Nyquist planes) -> the
-// column-tile layout of S; the tiles' padding columns are zero.
-// ---------------------------------------------------------------------------
-template <typename R>
-__global__ void __launch_bounds__(NB) k_tile_spectrum(Geo g, const c2<R>* __restrict__ main,
-                                                      const c2<R>* __restrict__ nyq, c2<R>* __restrict__ st, long n) {
-  for (long o = blockIdx.x * (long)blockDim.x + threadIdx.x; o < n; o += (long)gridDim.x * blockDim.x) {
-    const long c = o % g.stx, rest = o / g.stx;
-    const long kz = rest % g.nz, tf = rest / g.nz;
-    const long f = tf / g.stpf, tt = tf % g.stpf;
-    c2<R> v = mk<R>(R(0), R(0));
-    if (tt < g.stm) {
-      const long col = tt * g.stx + c;
-      if (col < (long)g.M * g.ny) v = main[f * g.hmain + kz * ((long)g.M * g.ny) + col];
-    } else {
-      const long col = (tt - g.stm) * g.stx + c;
-      if (col < g.ny) v = nyq[f * g.plane + kz * g.ny + col];
-    }
-    st[o] = v;
   }
 }
 
@@ -555,8 +323,9 @@ struct pf_handle {
   KTabF ktf{};
 
   // faithful (FP64) banks
-  Bank<double> fs{}, fgrad{}, fdfdc{}, fdum{}, fpsi{};
-  double* fmob = nullptr;
+  // fs: the state's F fields and, contiguous after them, the F derivatives
+  // (df_dc, df_dphi_i); fdum: the mobility chain's one field
+  Bank<double> fs{}, fdum{};
   // reduced banks (precision R, stored untyped)
   void *S_main = nullptr, *W_main = nullptr, *W_nyq = nullptr;  // S: column-tile layout
   void *G_main = nullptr, *G_nyq = nullptr, *mob = nullptr;
@@ -676,10 +445,6 @@ void tflush(pf_handle* h) {
 }
 
 unsigned grid_for(long n, long per) { return (unsigned)std::min<long>(kMaxGrid, std::max<long>(1, (n + per - 1) / per)); }
-unsigned row_block(const Geo& g) {
-  int b = ((g.M + 1 + 63) / 64) * 64;
-  return (unsigned)std::min(b, NB);
-}
 
 // Final diag reduction into ddiag record `idx`.
 int diag_final(pf_handle* h, long idx, bool with_nl, bool with_fi, const double* cmean, const float* cmean_f) {
@@ -715,108 +480,6 @@ int ensure_diag(pf_handle* h, long n) {
   int rc = dalloc(h, (void**)&h->ddiag, sizeof(double) * 9 * (size_t)n);
   if (!rc) h->ddiag_cap = n;
   return rc;
-}
-
-// ---------------------------------------------------------------------------
-// Faithful step (FP64): the reference's loop sequence.
-// ---------------------------------------------------------------------------
-int launch_grad_zinv(pf_handle* h) {
-  const Geo& g = h->g;
-  const double2* tw = twiddle_table<double>(g.nz);
-  if (!tw) return fail(PF_EHIP, "twiddle table allocation failed");
-  switch (g.nz) {
-#define PF_CASE(N)                                                                                      \
-  case N: {                                                                                             \
-    constexpr int TX = col_tile(N, sizeof(double2));                                                    \
-    const long Wm = (long)g.M * g.ny, tm = (Wm + TX - 1) / TX, tn = ((long)g.ny + TX - 1) / TX;         \
-    hipLaunchKernelGGL((k_grad_zinv<N, false>), dim3((unsigned)(tm * g.F)), dim3(TX * plan_T(N)), 0,    \
-                       h->s, g, h->kt, h->fs.main, h->fgrad.main, Wm, tm, tw);                           \
-    hipLaunchKernelGGL((k_grad_zinv<N, true>), dim3((unsigned)(tn * g.F)), dim3(TX * plan_T(N)), 0,     \
-                       h->s, g, h->kt, h->fs.nyq, h->fgrad.nyq, (long)g.ny, tn, tw);                     \
-    return 0;                                                                                           \
-  }
-    PF_FAITHFUL_SIZES(PF_CASE)
-#undef PF_CASE
-    default: return fail(PF_EINVAL, "unsupported nz");
-  }
-}
-
-int step_faithful(pf_handle* h, bool diag, long rec) {
-  const Geo& g = h->g;
-  hipStream_t s = h->s;
-  const unsigned rb = row_block(g);
-  int rc;
-  double* st = (double*)h->fs.main;
-  // loops 5-10 (read the real state before it is transformed in place)
-  h->n_part_nl = grid_for(g.P, NB);
-  tbeg(h, ST_NONLINEAR);
-  const size_t shb = sizeof(double) * ((size_t)g.var * NB + NB);
-  if (diag)
-    hipLaunchKernelGGL((k_nl_faithful<true>), dim3(grid_for(g.P, NB)), dim3(NB), shb, s, g, h->u, st,
-                       (double*)h->fdfdc.main, (double*)h->fpsi.main, h->fmob, h->part_nl);
-  else
-    hipLaunchKernelGGL((k_nl_faithful<false>), dim3(grid_for(g.P, NB)), dim3(NB), shb, s, g, h->u, st,
-                       (double*)h->fdfdc.main, (double*)h->fpsi.main, h->fmob, h->part_nl);
-  tend(h);
-  // loops 1-4: F(phi_i), F(c); gradients; f_int
-  tbeg(h, ST_X_R2C);
-  if ((rc = fwd3d<double>(h->fs.main, h->fs.nyq, g.nx, g.ny, g.nz, g.F, 1.0 / (double)(float)g.P, s))) return rc;
-  tend(h);
-  // The gradients (3F inverse transforms) feed nothing but f_int, a summary-row
-  // quantity: they run on the steps whose row is reported.  The state sequence
-  // is the reference's either way.
-  if (diag) {
-    tbeg(h, ST_GRAD);
-    if ((rc = launch_grad_zinv(h))) return rc;
-    // loops 2 and 4 (src/var_diff.f90:620-622, 670-671): inverse y of the 3F
-    // gradient fields, then the inverse x pass summed straight into
-    // f_int = sum 0.5*kappa*|grad u|^2 (the real gradients are never stored)
-    const long M = g.M, nb3 = 3L * g.F;
-    if ((rc = col_pass<double>(g.ny, true, h->fgrad.main, M, (long)g.nz * nb3, s))) return rc;
-    if ((rc = row_pass<double>(g.ny, true, h->fgrad.nyq, (long)g.nz * nb3, s))) return rc;
-    long nblk = 0;
-    if ((rc = x_c2r_sumsq<double>(g.nx, h->fgrad.main, h->fgrad.nyq, (long)g.plane * nb3, g.plane,
-                                  0.5 * h->u.kc, 0.5 * h->u.kphi, h->part_fi,
-                                  2 * std::max(kMaxGrid, kZlineMaxGrid), &nblk, s)))
-      return rc;
-    h->n_part_fi = nblk;
-    tend(h);
-  }
-  if (diag) {
-    tbeg(h, ST_DIAG);
-    diag_final(h, rec, true, true, (const double*)h->fs.main, nullptr);  // Re F(c)(0) = mean(c)
-    tend(h);
-  }
-  // loop 10: F(df_dc)  (F(c) of loop 10 is the same transform as loop 3's; reused)
-  tbeg(h, ST_MOBILITY);
-  if ((rc = fwd3d<double>(h->fdfdc.main, h->fdfdc.nyq, g.nx, g.ny, g.nz, 1, 1.0 / (double)(float)g.P, s))) return rc;
-  // loop 11
-  hipLaunchKernelGGL((k_ghat<double>), dim3(grid_for(g.plane, 1)), dim3(rb), 0, s, g, h->u, h->kt, h->fdfdc, 0,
-                     h->fs, 0, h->fdum, (long)g.plane);
-  if ((rc = inv3d<double>(h->fdum.main, h->fdum.nyq, g.nx, g.ny, g.nz, 1, s))) return rc;
-  // loop 12
-  hipLaunchKernelGGL(k_mult_faithful, dim3(grid_for(g.P, NB)), dim3(NB), 0, s, g.P, h->u.D,
-                     (double*)h->fdum.main, h->fmob);
-  if ((rc = fwd3d<double>(h->fdum.main, h->fdum.nyq, g.nx, g.ny, g.nz, 1, 1.0 / (double)(float)g.P, s))) return rc;
-  tend(h);
-  // loop 13
-  tbeg(h, ST_UPDATE);
-  hipLaunchKernelGGL(k_ch_faithful, dim3(grid_for(g.plane, 1)), dim3(rb), 0, s, g, h->u, h->kt, h->fs, h->fdum,
-                     h->fdfdc, (long)g.plane);
-  tend(h);
-  // loop 14: F(df_dphi_i) (F(phi_i) is loop 1's transform; reused)
-  tbeg(h, ST_Y_FWD);
-  if ((rc = fwd3d<double>(h->fpsi.main, h->fpsi.nyq, g.nx, g.ny, g.nz, g.var, 1.0 / (double)(float)g.P, s))) return rc;
-  tend(h);
-  tbeg(h, ST_UPDATE);
-  hipLaunchKernelGGL(k_ac_faithful, dim3(grid_for((long)g.plane * g.var, 1)), dim3(rb), 0, s, g, h->u, h->kt,
-                     h->fs, h->fpsi, (long)g.plane * g.var);
-  tend(h);
-  // inverse transforms of c (loop 13) and phi_i (loop 14), batched
-  tbeg(h, ST_Z_INV);
-  if ((rc = inv3d<double>(h->fs.main, h->fs.nyq, g.nx, g.ny, g.nz, g.F, s))) return rc;
-  tend(h);
-  return 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -918,49 +581,6 @@ bool xline_supported(const Geo& g) {
     PF_GRID_SIZES(PF_CASE)
 #undef PF_CASE
     default: return false;
-  }
-}
-
-// Fused y pass (k_ypass): main block and Nyquist planes in one launch.
-template <typename R, bool INV>
-int launch_ypass_fused(pf_handle* h, c2<R>* main, c2<R>* nyq, int nf) {
-  const Geo& g = h->g;
-  switch (g.ny) {
-#define PF_CASE(N)                                                                              \
-  case N: {                                                                                     \
-    constexpr int TX = col_tile(N, sizeof(c2<R>));                                              \
-    const long npanels = (long)g.nz * nf, nlines = (long)g.nz * nf;                             \
-    const long tpp = ((long)g.M + TX - 1) / TX;                                                 \
-    /* a multiple of 8 blocks for the XCD order (xcd_block); the extra blocks fall on   */       \
-    /* Nyquist lines past the last one and touch no memory                              */       \
-    const long grid = (tpp * npanels + (nlines + TX - 1) / TX + 7) / 8 * 8;                     \
-    const c2<R>* tw = twiddle_table<R>(N);                                                      \
-    if (!tw) return fail(PF_EHIP, "twiddle table allocation failed");                           \
-    hipLaunchKernelGGL((k_ypass<R, N, INV>), dim3((unsigned)grid), dim3(TX * plan_T(N)), 0, \
-                       h->s, main, nyq, (long)g.M, npanels, nlines, tw, (const Member<R>*)nullptr, 0L); \
-    return 0;                                                                                   \
-  }
-    PF_GRID_SIZES(PF_CASE)
-#undef PF_CASE
-    default: return fail(PF_EINVAL, "unsupported ny");
-  }
-}
-
-// y transform of nf fields of a bank.  FP32: the fused pass.  FP64: the column
-// pass over the main block and the row pass over the Nyquist planes; in FP64 the
-// fused kernel measured 1.10 ms (16 columns per tile) / 0.97 ms (8) per pass at
-// 256^3 x 17 against 0.85 ms for the plain column pass, while in FP32 the two
-// are equal (0.45 ms).
-template <typename R, bool INV>
-int launch_ypass(pf_handle* h, c2<R>* main, c2<R>* nyq, int nf) {
-  if constexpr (sizeof(R) == 8) {
-    const Geo& g = h->g;
-    const long nlines = (long)g.nz * nf;
-    int rc = col_pass<R>(g.ny, INV, main, (long)g.M, nlines, h->s);
-    if (!rc) rc = row_pass<R>(g.ny, INV, nyq, nlines, h->s);
-    return rc;
-  } else {
-    return launch_ypass_fused<R, INV>(h, main, nyq, nf);
   }
 }
 
@@ -1072,8 +692,8 @@ template <bool INV> int ypass_batch(const Geo& g, const Member<float>* mt, long 
   case N: {                                                                                           \
     constexpr int TX = col_tile(N, sizeof(c2<float>));                                                \
     const long ppm = (long)g.nz * g.F, npanels = nmem * ppm, nlines = npanels;                        \
-    const long tpp = ((long)g.M + TX - 1) / TX;                                                       \
-    const long grid = (tpp * npanels + (nlines + TX - 1) / TX + 7) / 8 * 8;                           \
+    const long tiles = nmem * ((ppm * g.M + TX - 1) / TX + (ppm + TX - 1) / TX);                      \
+    const long grid = (tiles + 7) / 8 * 8;                                                            \
     const c2<float>* tw = twiddle_table<float>(N);                                                    \
     if (!tw) return fail(PF_EHIP, "twiddle table set-up failed");                                     \
     hipLaunchKernelGGL((k_ypass<float, N, INV, true>), dim3((unsigned)grid), dim3(TX * plan_T(N)), 0, s, \
@@ -1162,7 +782,7 @@ int step_reduced(pf_handle* h, bool diag, long rec, bool fint_next) {
     tend(h);
   }
   tbeg(h, ST_Y_FWD);
-  if ((rc = launch_ypass<R, false>(h, W.main, W.nyq, g.F))) return rc;
+  if ((rc = y_pass<R>(g.ny, false, W.main, W.nyq, g.M, (long)g.nz * g.F, s))) return rc;
   tend(h);
   tbeg(h, ST_UPDATE);
   long g1 = 0, g2 = 0;
@@ -1177,9 +797,9 @@ int step_reduced(pf_handle* h, bool diag, long rec, bool fint_next) {
     if (rc) return rc;
     tend(h);
     tbeg(h, ST_MOBILITY);
-    if ((rc = launch_ypass<R, true>(h, G.main, G.nyq, 1))) return rc;
+    if ((rc = y_pass<R>(g.ny, true, G.main, G.nyq, g.M, g.nz, s))) return rc;
     if ((rc = launch_xline<R, true>(h, G.main, G.nyq, (R*)h->mob, nullptr, nullptr, false, false))) return rc;
-    if ((rc = launch_ypass<R, false>(h, G.main, G.nyq, 1))) return rc;
+    if ((rc = y_pass<R>(g.ny, false, G.main, G.nyq, g.M, g.nz, s))) return rc;
     tend(h);
     tbeg(h, ST_UPDATE);
     rc = fint_next ? launch_zline<R, ROLE_CMOB, DC, true>(h, S, W, Fc, G, h->part_fi + g1, 0, 1, &g2)
@@ -1190,7 +810,66 @@ int step_reduced(pf_handle* h, bool diag, long rec, bool fint_next) {
   h->fint_ready = fint_next;
   tend(h);
   tbeg(h, ST_Y_INV);
-  if ((rc = launch_ypass<R, true>(h, W.main, W.nyq, g.F))) return rc;
+  if ((rc = y_pass<R>(g.ny, true, W.main, W.nyq, g.M, (long)g.nz * g.F, s))) return rc;
+  tend(h);
+  return 0;
+}
+
+// ---------------------------------------------------------------------------
+// Faithful step (FP64): the reference's loop sequence on the real-space state.
+// Twelve launches: the state's and the derivatives' forward transforms run as one
+// batch of 2F fields, the last forward pass, the k-space loops and the first
+// inverse pass are one kernel (k_zfaithful).
+// ---------------------------------------------------------------------------
+int step_faithful(pf_handle* h, bool diag, long rec) {
+  const Geo& g = h->g;
+  hipStream_t s = h->s;
+  const Bank<double> U = h->fs, D = sub(h->fs, g, g.F), G = h->fdum;
+  const double scale = 1.0 / (double)(float)g.P;
+  int rc;
+  // loops 5-10 (read the real state before it is transformed in place)
+  tbeg(h, ST_NONLINEAR);
+  long nnl = 0;
+  if ((rc = faithful_nonlinear(g, h->u, diag, (const double*)U.main, (double*)D.main, (double*)h->mob, h->part_nl,
+                               kMaxGrid, &nnl, s)))
+    return rc;
+  if (diag) h->n_part_nl = nnl;
+  tend(h);
+  // F(c), F(phi_i), F(df_dc), F(df_dphi_i): x and y
+  tbeg(h, ST_X_R2C);
+  if ((rc = x_r2c<double>(g.nx, U.main, U.main, U.nyq, (long)g.plane * 2 * g.F, scale, s))) return rc;
+  tend(h);
+  tbeg(h, ST_Y_FWD);
+  if ((rc = y_pass<double>(g.ny, false, U.main, U.nyq, g.M, (long)g.nz * 2 * g.F, s))) return rc;
+  tend(h);
+  // z, loop 11's g^ and loop 14; f_int of loops 1-4 on reported steps
+  tbeg(h, ST_UPDATE);
+  long n1 = 0, n2 = 0;
+  if ((rc = faithful_z(FZ_GHAT, diag, g, h->u, h->kt, U, D, G, h->part_fi, 0, 1, kZlineMaxGrid, &n1, s))) return rc;
+  if ((rc = faithful_z(FZ_ETA, diag, g, h->u, h->kt, U, D, G, h->part_fi + n1, 1, g.var, kZlineMaxGrid, &n2, s)))
+    return rc;
+  tend(h);
+  if (diag) {
+    h->n_part_fi = n1 + n2;
+    tbeg(h, ST_DIAG);
+    diag_final(h, rec, true, true, (const double*)U.main, nullptr);  // Re F(c)(0) = mean(c)
+    tend(h);
+  }
+  // loops 11-12: g back in real space, times mob_c - D_mean, forward
+  tbeg(h, ST_MOBILITY);
+  if ((rc = y_pass<double>(g.ny, true, G.main, G.nyq, g.M, g.nz, s))) return rc;
+  if ((rc = launch_xline<double, true>(h, G.main, G.nyq, (double*)h->mob, nullptr, nullptr, false, false))) return rc;
+  if ((rc = y_pass<double>(g.ny, false, G.main, G.nyq, g.M, g.nz, s))) return rc;
+  tend(h);
+  // loop 13
+  tbeg(h, ST_UPDATE);
+  if ((rc = faithful_z(FZ_CMOB, false, g, h->u, h->kt, U, D, G, nullptr, 0, 1, kZlineMaxGrid, nullptr, s))) return rc;
+  tend(h);
+  tbeg(h, ST_Y_INV);
+  if ((rc = y_pass<double>(g.ny, true, U.main, U.nyq, g.M, (long)g.nz * g.F, s))) return rc;
+  tend(h);
+  tbeg(h, ST_X_C2R);
+  if ((rc = x_c2r<double>(g.nx, U.main, U.main, U.nyq, (long)g.plane * g.F, s))) return rc;
   tend(h);
   return 0;
 }
@@ -1259,18 +938,16 @@ std::vector<double> host_means(const double* phi, const double* con, long P, int
 }
 
 // Reduced forms, once W holds the real state (SoA): S <- F(W) with f_trans
-// normalisation (computed in X, then put in the column-tile layout), W <- x-half
+// normalisation (passes in X, the last one into the column-tile layout), W <- x-half
 // lines, dc64 <- the FP64 field means dc.
 template <typename R> int finish_put_reduced(pf_handle* h, const std::vector<double>& dc) {
   const Geo& g = h->g;
-  PF_HIP(hipMemcpyAsync(h->X_main, h->W_main, sizeof(R) * (size_t)g.P * g.F, hipMemcpyDeviceToDevice, h->s));
-  int rc = fwd3d<R>((c2<R>*)h->X_main, (c2<R>*)h->X_nyq, g.nx, g.ny, g.nz, g.F, (R)(1.0 / (double)(float)g.P), h->s);
+  int rc = fwd3d_tiled<R>((const c2<R>*)h->W_main, (c2<R>*)h->X_main, (c2<R>*)h->X_nyq, (c2<R>*)h->S_main, g.nx, g.ny,
+                          g.nz, g.F, (R)(1.0 / (double)(float)g.P), h->s);
   if (rc) return rc;
-  const long nst = g.stpf * g.nz * g.stx * g.F;
-  hipLaunchKernelGGL((k_tile_spectrum<R>), dim3(grid_for(nst, NB)), dim3(NB), 0, h->s, g,
-                     (const c2<R>*)h->X_main, (const c2<R>*)h->X_nyq, (c2<R>*)h->S_main, nst);
   // W <- x-half lines: (1/nx) R2C along x of the real state == z,y-inverse of S
-  rc = x_r2c<R>(g.nx, (c2<R>*)h->W_main, (c2<R>*)h->W_nyq, (long)g.ny * g.nz * g.F, (R)(1.0 / (double)g.nx), h->s);
+  c2<R>* w = (c2<R>*)h->W_main;
+  rc = x_r2c<R>(g.nx, w, w, (c2<R>*)h->W_nyq, (long)g.ny * g.nz * g.F, (R)(1.0 / (double)g.nx), h->s);
   if (rc) return rc;
   PF_HIP(hipMemcpyAsync(h->dc64, dc.data(), sizeof(double) * g.F, hipMemcpyHostToDevice, h->s));
   PF_HIP(hipStreamSynchronize(h->s));
@@ -1411,9 +1088,8 @@ extern "C" int pf_create(const pf_params* p, int nx, int ny, int nz, int var, in
     h->ktf.az = df; h->ktf.azp = df + nz;
   }
   if (mode == PF_MODE_FP64_FAITHFUL) {
-    if ((rc = alloc_bank<double>(h, h->fs, g.F)) || (rc = alloc_bank<double>(h, h->fgrad, 3 * g.F)) ||
-        (rc = alloc_bank<double>(h, h->fdfdc, 1)) || (rc = alloc_bank<double>(h, h->fdum, 1)) ||
-        (rc = alloc_bank<double>(h, h->fpsi, var)) || (rc = dalloc(h, (void**)&h->fmob, sizeof(double) * g.P)))
+    if ((rc = alloc_bank<double>(h, h->fs, 2 * g.F)) || (rc = alloc_bank<double>(h, h->fdum, 1)) ||
+        (rc = dalloc(h, &h->mob, sizeof(double) * g.P)))
       return bail(rc);
   } else if (mode == PF_MODE_FP64_REDUCED) {
     if (!xline_supported<double, false>(g))
@@ -1552,12 +1228,11 @@ extern "C" int pf_put_voronoi(pf_handle* h, int nseeds, int iseed, double c0, do
 }
 
 namespace {
-// Reduced modes: real state of the current step = C2R along x of a copy of W.
+// Reduced modes: real state of the current step = C2R along x of W, into X.
 template <typename R> int real_state_reduced(pf_handle* h) {
   const Geo& g = h->g;
-  PF_HIP(hipMemcpyAsync(h->X_main, h->W_main, sizeof(R) * (size_t)g.P * g.F, hipMemcpyDeviceToDevice, h->s));
-  PF_HIP(hipMemcpyAsync(h->X_nyq, h->W_nyq, sizeof(c2<R>) * (size_t)g.plane * g.F, hipMemcpyDeviceToDevice, h->s));
-  return x_c2r<R>(g.nx, (c2<R>*)h->X_main, (const c2<R>*)h->X_nyq, (long)g.ny * g.nz * g.F, h->s);
+  return x_c2r<R>(g.nx, (const c2<R>*)h->W_main, (c2<R>*)h->X_main, (const c2<R>*)h->W_nyq, (long)g.ny * g.nz * g.F,
+                  h->s);
 }
 }  // namespace
 
@@ -1858,20 +1533,19 @@ extern "C" int pf_diagnose(pf_handle* h, pf_diag* out) {
   const long rows = (long)g.plane * g.F;
   const unsigned gr_nl = grid_for(g.P, NB);
   if (h->mode == PF_MODE_FP64_FAITHFUL) {
-    const size_t shb = sizeof(double) * ((size_t)g.var * NB + NB);
-    hipLaunchKernelGGL((k_nl_faithful<true>), dim3(gr_nl), dim3(NB), shb, s, g, h->u,
-                       (const double*)h->fs.main, (double*)h->fdfdc.main, (double*)h->fpsi.main, h->fmob,
-                       h->part_nl);
-    h->n_part_nl = gr_nl;
-    // f_int by Parseval on a transformed copy of the state (same quantity as loops 1-4)
-    PF_HIP(hipMemcpyAsync(h->fgrad.main, h->fs.main, sizeof(double) * (size_t)g.P * g.F,
-                          hipMemcpyDeviceToDevice, s));
-    if ((rc = fwd3d<double>(h->fgrad.main, h->fgrad.nyq, g.nx, g.ny, g.nz, g.F, 1.0 / (double)(float)g.P, s)))
+    const Bank<double> D = sub(h->fs, g, g.F);  // holds nothing between steps
+    long nnl = 0;
+    if ((rc = faithful_nonlinear(g, h->u, true, (const double*)h->fs.main, (double*)D.main, (double*)h->mob,
+                                 h->part_nl, kMaxGrid, &nnl, s)))
+      return rc;
+    h->n_part_nl = nnl;
+    // f_int by Parseval on the transformed state (same quantity as loops 1-4)
+    if ((rc = fwd3d_split<double>(h->fs.main, D.main, D.nyq, g.nx, g.ny, g.nz, g.F, 1.0 / (double)(float)g.P, s)))
       return rc;
     hipLaunchKernelGGL((k_update<double, false, false, true, false>), dim3(grid_for(rows, 1)), dim3(NB), 0, s, g,
-                       h->u, h->kt, h->fgrad, h->fgrad, h->fgrad, h->dc64, h->part_fi, rows);
+                       h->u, h->kt, D, D, D, h->dc64, h->part_fi, rows);
     h->n_part_fi = grid_for(rows, 1);
-    diag_final(h, 0, true, true, (const double*)h->fgrad.main, nullptr);
+    diag_final(h, 0, true, true, (const double*)D.main, nullptr);
   } else {
     const bool f32 = h->mode == PF_MODE_FP32_MIXED;
     if (f32) {

@@ -98,6 +98,23 @@ __device__ __forceinline__ KCoef kcoef(const KTab& t, int kx, int ky, int kz) {
   return k;
 }
 
+// Parameters of the timestep, gamma as its two values, invP = 1 / (nx ny nz).
+struct UPar {
+  double dt, kphi, kc, D, L, Dgb, am, ap, cm, cp, s1g, s2g, invP;
+};
+
+// One simulation of a batched ensemble (a device table of these drives the
+// BATCH forms of the step kernels: one launch per stage covers every member of
+// one grid shape): its carried spectrum S (column-tile layout, below), work
+// bank W, FP64 k = 0 modes and parameters.
+template <typename R> struct Member {
+  c2<R>* Wm;
+  c2<R>* Wn;
+  c2<R>* S;
+  double* dc64;
+  UPar u;
+};
+
 // A bank of nf fields in the split-Nyquist layout.
 template <typename R> struct Bank {
   c2<R>* main;  // nf * M*ny*nz complex (== nf * nx*ny*nz reals)
