@@ -117,16 +117,17 @@ def roofline_of(stages, steps):
     return name, avg_ms, achieved, st["bytes"]
 
 
-def stage_kernels(n, lines=1, plan=0):
+def stage_kernels(n, lines=1, plan=0, keep="false", zkeep=0):
     """Kernel behind each timed stage of the FP32 step on an n^3 grid, named as
     rocprofv3 prints them (lines: x lines per x-line block; plan: the z
-    transforms' radix plan variant)."""
+    transforms' radix plan variant; keep, zkeep: the cache policy, by the size of
+    the spectra)."""
     return {
-        "nonlinear": [f"pf::k_xline<float, {n}, {lines}, false, false>"],
-        "y_fwd": [f"pf::k_ypass<float, {n}, false, false>"],
-        "kspace_update": [f"pf::k_zline<float, {n}, 0, true, false, false, {plan}>",
-                          f"pf::k_zline<float, {n}, 0, true, true, false, {plan}>"],
-        "y_inv": [f"pf::k_ypass<float, {n}, true, false>"],
+        "nonlinear": [f"pf::k_xline<float, {n}, {lines}, false, false, {keep}, false>"],
+        "y_fwd": [f"pf::k_ypass<float, {n}, false, false, {keep}>"],
+        "kspace_update": [f"pf::k_zline<float, {n}, 0, true, false, false, {plan}, {zkeep}>",
+                          f"pf::k_zline<float, {n}, 0, true, true, false, {plan}, {zkeep}>"],
+        "y_inv": [f"pf::k_ypass<float, {n}, true, false, {keep}>"],
     }
 
 
@@ -135,7 +136,7 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic_fused_kernels_256x17_
 # The sources that decide what the step kernels read and write and how they are
 # launched; the traffic profile records their hash when it is measured.
 KERNEL_SOURCES = [os.path.join(ROOT, "phase-field-microstructure-evolution_amd", "csrc", f)
-                  for f in ("pf_fused.hpp", "pf_kernels.hpp", "pf_fft2.hpp", "pf_fft.hpp", "pf_step_kernels.hpp",
+                  for f in ("pf_fused.hpp", "pf_passes.hpp", "pf_xline_launch.hpp", "pf_zline_launch.hpp", "pf_kernels.hpp", "pf_fft2.hpp", "pf_fft.hpp", "pf_step_kernels.hpp",
                             "pf_step.hip", "pf_tuned.inc")]
 
 

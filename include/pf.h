@@ -111,7 +111,7 @@ int pf_set_graphs(pf_handle* h, int on);
  * per point or per column: the state is unchanged, and the summary energies,
  * which are sums of per-block partials, can change in their last bits.
  *   xline_lines   : x lines per x-line block, 0 = automatic, else 1, 2, 4 or 8
- *   xline_grid    : x-line blocks, 0 = 8192, else 256 .. 16384
+ *   xline_grid    : most x-line blocks, 0 = automatic, else 256 .. 16384
  *   zline_grid    : z-line blocks, 0 = 32768, else 1024 .. 65536
  *   zline_run_rows: main-block rows per XCD run of z-line tiles, -1 = 1, 0 = none, 1 .. 8
  *   zline_plan    : radix sequence of the FP32 z transforms, 0 = default, 1 or 2

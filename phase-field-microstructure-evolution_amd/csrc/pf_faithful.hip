@@ -5,6 +5,7 @@
 #include "../../include/pf.h"
 #include "pf_internal.hpp"
 #include "pf_faithful.hpp"
+#include "pf_nl.hpp"
 #include "pf_passes.hpp"
 
 namespace pf {
@@ -13,19 +14,12 @@ namespace pf {
 // Loops 5-10 (src/var_diff.f90:685-905), O(var^2) per point.
 // Reads the real state bank (c, eta_i); writes df_dc and df_dphi_i (a bank in the
 // same order) and mob_c - D_mean.
-//   gamma_ij of src/var_diff.f90:206-218 (the matrix pf_gamma builds) is sigma_1
-//   between two distinct matrix grains, sigma_2 between a grain and the precipitate
-//   field eta_var (index mat) and 0 on the diagonal: the two values are used
-//   directly, and a row's factor (2 gamma) phi_i, the same product for every j, is
-//   formed once.  Every sum keeps the reference's order over i and j.
 //   A point's order parameters sit in the thread's own LDS column.  The pair sums
 //   read it once per kNlRows rows i rather than once per pair: the LDS traffic of
 //   the O(var^2) loops bounded the kernel.  256^3 x 17: 1.87 -> 0.84 ms, with the
 //   energies 2.49 -> 1.03 ms; 0.84 ms is 5.6 TB/s over the 4.7 GB it moves, the
 //   rate of a plain stream.
 // ---------------------------------------------------------------------------
-constexpr int kNlRows = 4;  // rows i per pass over j
-
 template <bool DIAG>
 __global__ void __launch_bounds__(kNlBlock)
 k_nl_faithful(Geo g, UPar u, const double* __restrict__ st, double* __restrict__ dfd, double* __restrict__ mobd,
@@ -33,112 +27,32 @@ k_nl_faithful(Geo g, UPar u, const double* __restrict__ st, double* __restrict__
   constexpr int NB = kNlBlock;
   extern __shared__ double sh[];  // var * NB values, then NB reduction scratch
   double* red = sh + (long)g.var * NB;
-  const int V = g.var, mat = V - 1;
+  const int V = g.var;
   double* const ph = sh + threadIdx.x;
-  double a_ch = 0.0, a_eta = 0.0, cmax = 0.0, cmin = 1.0, pmin = 1.0, p3 = 0.0;
+  NlDiag d;
+  // cache policy of the state and derivative banks together
+  const bool keep = bank_stays(2ul * (unsigned)g.F * g.P * sizeof(double));
+  auto put = [&](double x, double* p) {
+    if (keep) *p = x;
+    else __builtin_nontemporal_store(x, p);
+  };
   for (long t = (long)blockIdx.x * NB + threadIdx.x; t < g.P; t += (long)gridDim.x * NB) {
+    if (keep) {
 #pragma unroll 8
-    for (int i = 0; i < V; ++i) ph[i * NB] = __builtin_nontemporal_load(st + (long)(i + 1) * g.P + t);
-    const double con = __builtin_nontemporal_load(st + t);
-    // loop 5
-    double fe = 0.0;
-    if (DIAG) {
-      for (int i = 0; i < V; ++i) {
-        const double fi = ph[i * NB], fi2 = fi * fi;
-        fe = (fe - 0.5 * fi2) + 0.25 * (fi2 * fi2);
-        const double g1 = u.s1g * fi2, g2 = u.s2g * fi2;
-#pragma unroll 4
-        for (int j = i + 1; j < mat; ++j) {
-          const double fj = ph[j * NB];
-          fe = fe + g1 * (fj * fj);
-        }
-        if (i < mat) {
-          const double fj = ph[mat * NB];
-          fe = fe + g2 * (fj * fj);
-        }
-      }
+      for (int i = 0; i < V; ++i) ph[i * NB] = st[(long)(i + 1) * g.P + t];
+    } else {
+#pragma unroll 8
+      for (int i = 0; i < V; ++i) ph[i * NB] = __builtin_nontemporal_load(st + (long)(i + 1) * g.P + t);
     }
-    // loop 6
-    double num = 0.0, den = 0.0;
-#pragma unroll 4
-    for (int i = 0; i < V; ++i) {
-      const double f2 = ph[i * NB] * ph[i * NB], f4 = f2 * f2;
-      if (i < mat) num = num + f4;
-      den = den + f4;
-    }
-    const double hm = num / den, hp = 1.0 - hm;
-    const double dm = con - u.cm, dp = con - u.cp;
-    const double fch = (hm * u.am) * (dm * dm) + (hp * u.ap) * (dp * dp);
-    __builtin_nontemporal_store(((2.0 * hm) * u.am) * dm + ((2.0 * hp) * u.ap) * dp, dfd + t);
-    // loops 7-9
-    const double fm = u.am * (dm * dm), fp = u.ap * (dp * dp);
-    const double fv = ph[mat * NB], fv2 = fv * fv, fv4 = fv2 * fv2;
-    const double t2v = (4.0 * (fv2 * fv)) * (den - fv4);
-    const double den2 = den * den;
-    double ps = 0.0;
-    for (int i0 = 0; i0 < mat; i0 += kNlRows) {
-      double fi[kNlRows], ci[kNlRows], term2[kNlRows];
-#pragma unroll
-      for (int r = 0; r < kNlRows; ++r) {
-        fi[r] = (i0 + r < mat) ? ph[(i0 + r) * NB] : 0.0;
-        ci[r] = (2.0 * u.s1g) * fi[r];
-        term2[r] = 0.0;
-      }
-      auto add = [&](int j) {
-        const double fj = ph[j * NB], fj2 = fj * fj;
-#pragma unroll
-        for (int r = 0; r < kNlRows; ++r) term2[r] = term2[r] + ci[r] * fj2;
-      };
-#pragma unroll 4
-      for (int j = 0; j < i0; ++j) add(j);
-#pragma unroll
-      for (int q = 0; q < kNlRows; ++q) {  // the rows' own block: no term j = i
-        const double fj2 = fi[q] * fi[q];
-#pragma unroll
-        for (int r = 0; r < kNlRows; ++r)
-          if (r != q) term2[r] = term2[r] + ci[r] * fj2;
-      }
-#pragma unroll 4
-      for (int j = i0 + kNlRows; j < mat; ++j) add(j);
-#pragma unroll
-      for (int r = 0; r < kNlRows; ++r) {
-        if (i0 + r >= mat) continue;
-        const double f = fi[r];
-        const double term1 = (f * f) * f - f;
-        const double t2 = term2[r] + ((2.0 * u.s2g) * f) * fv2;
-        const double term4 = (((4.0 * ((f * f) * f)) * fv4) * (fm - fp)) / den2;
-        __builtin_nontemporal_store((term1 + t2) + term4, dfd + (long)(i0 + r + 1) * g.P + t);
-        ps = ps + f * f;
-      }
-    }
-    {
-      const double term1 = (fv * fv) * fv - fv, c2 = (2.0 * u.s2g) * fv;
-      double t2 = 0.0;
-#pragma unroll 4
-      for (int j = 0; j < mat; ++j) {
-        const double fj = ph[j * NB];
-        t2 = t2 + c2 * (fj * fj);
-      }
-      const double term4 = (t2v * (fp - fm)) / den2;
-      __builtin_nontemporal_store((term1 + t2) + term4, dfd + (long)V * g.P + t);
-      ps = ps + fv * fv;
-    }
-    // loop 10: mob_c = D_bulk(var) + 2(1 - sum phi^2) D_gb, D_bulk(var) = D_L = D_mean;
-    // loop 12 multiplies by mob_c - D_mean
-    mobd[t] = (u.D + ((2.0 * (1.0 - ps)) * u.Dgb)) - u.D;
-    if (DIAG) {
-      a_ch += fch;
-      a_eta += fe;
-      if (fv > p3) p3 = fv;
-      if (con <= cmin) cmin = con;
-      if (con > cmax) cmax = con;
-      if (ps < pmin) pmin = ps;
-    }
+    const double con = st[t];
+    double mob;
+    nl_point_faithful<DIAG>(u, V, con, ph, NB, [&](int f, double x) { put(x, dfd + (long)f * g.P + t); }, mob, d);
+    mobd[t] = mob;
   }
   if (DIAG) {
-    const double s0 = block_sum<NB>(a_ch, red), s1 = block_sum<NB>(a_eta, red);
-    const double e0 = block_ext<NB, true>(cmax, red), e1 = block_ext<NB, false>(cmin, red);
-    const double e2 = block_ext<NB, false>(pmin, red), e3 = block_ext<NB, true>(p3, red);
+    const double s0 = block_sum<NB>(d.ch, red), s1 = block_sum<NB>(d.eta, red);
+    const double e0 = block_ext<NB, true>(d.cmax, red), e1 = block_ext<NB, false>(d.cmin, red);
+    const double e2 = block_ext<NB, false>(d.pmin, red), e3 = block_ext<NB, true>(d.p3, red);
     if (threadIdx.x == 0) {
       double* o = part + (long)blockIdx.x * 6;
       o[0] = s0; o[1] = s1; o[2] = e0; o[3] = e1; o[4] = e2; o[5] = e3;
@@ -190,7 +104,7 @@ __device__ __forceinline__ KCoefR<double> kcoef_ref(const KCol<double>& c, int k
   return k;
 }
 
-template <int NZ, int ROLE, bool PARS>
+template <int NZ, int ROLE, bool PARS, bool KEEP>
 __global__ void __launch_bounds__(col_tile(NZ, sizeof(double2)) * plan_T(NZ)) __attribute__((amdgpu_waves_per_eu(2)))
 k_zfaithful(Geo g, UPar u, KTab kt, Bank<double> U, Bank<double> D, Bank<double> G, double* __restrict__ part,
             const double2* __restrict__ tw, int f0, int nf, unsigned tm, unsigned tn, unsigned run_tiles) {
@@ -198,6 +112,7 @@ k_zfaithful(Geo g, UPar u, KTab kt, Bank<double> U, Bank<double> D, Bank<double>
   constexpr int TX = col_tile(NZ, sizeof(double2));
   constexpr int NI = kInSlots<NZ>, NO = kOutSlots<NZ>, E = plan_E(NZ);
   constexpr unsigned CB = sizeof(double2);
+  constexpr int AUX = KEEP ? 0 : kBufNT;  // cache policy (bank_stays)
   static_assert(last_pass_in_place<NZ>(), "slot rows of the last pass are t + a per-slot constant");
   constexpr int SHN = (plan_np(NZ) > 1 || !rfft_io_same<NZ>()) ? NZ * TX : 1;
   __shared__ double2 sh[SHN * sizeof(double2) >= 16 * sizeof(double) ? SHN : 16 * sizeof(double) / sizeof(double2)];
@@ -226,10 +141,10 @@ k_zfaithful(Geo g, UPar u, KTab kt, Bank<double> U, Bank<double> D, Bank<double>
       if (act && rfft_in_valid<NZ>(t, s)) {
         const unsigned o = (unsigned)rfft_in_idx<NZ>(0, s) * rowb;
         if constexpr (ROLE == FZ_CMOB) {
-          b[s] = buf_ld<R>(rg, lw, o);
+          b[s] = buf_ld<R, AUX>(rg, lw, o);
         } else {
-          b[s] = buf_ld<R>(rd, lw, o);
-          a[s] = buf_ld<R>(ru, lw, o);
+          b[s] = buf_ld<R, AUX>(rd, lw, o);
+          a[s] = buf_ld<R, AUX>(ru, lw, o);
         }
       }
     if constexpr (ROLE == FZ_CMOB) {
@@ -237,8 +152,8 @@ k_zfaithful(Geo g, UPar u, KTab kt, Bank<double> U, Bank<double> D, Bank<double>
       for (int s = 0; s < NO; ++s)
         if (act && rfft_out_valid<NZ>(t, s)) {
           const unsigned o = (unsigned)rfft_out_idx<NZ>(0, s) * rowb;
-          a[s] = buf_ld<R>(ru, lw, o);
-          fh[s] = buf_ld<R>(rd, lw, o);
+          a[s] = buf_ld<R, AUX>(ru, lw, o);
+          fh[s] = buf_ld<R, AUX>(rd, lw, o);
         }
     }
     const int col = (int)col0 + c;
@@ -301,7 +216,7 @@ k_zfaithful(Geo g, UPar u, KTab kt, Bank<double> U, Bank<double> D, Bank<double>
 #pragma unroll
     for (int s = 0; s < NO; ++s)
       if (act && rfft_out_valid<NZ>(t, s))
-        buf_st<R>(ROLE == FZ_GHAT ? rg : ru, lw, (unsigned)rfft_out_idx<NZ>(0, s) * rowb, a[s]);
+        buf_st<R, AUX>(ROLE == FZ_GHAT ? rg : ru, lw, (unsigned)rfft_out_idx<NZ>(0, s) * rowb, a[s]);
     __syncthreads();
   }
   if (PARS) {
@@ -334,7 +249,7 @@ int faithful_nonlinear(const Geo& g, const UPar& u, bool diag, const double* st,
   return 0;
 }
 
-template <int ROLE, bool PARS>
+template <int ROLE, bool PARS, bool KEEP>
 static int zf_launch(const Geo& g, const UPar& u, const KTab& kt, Bank<double> U, Bank<double> D, Bank<double> G,
                      double* part, int f0, int nf, long max_blocks, long* nblocks, hipStream_t s) {
   const double2* tw = twiddle_table<double>(g.nz);
@@ -348,7 +263,7 @@ static int zf_launch(const Geo& g, const UPar& u, const KTab& kt, Bank<double> U
     /* whole XCD runs of main-block rows (xcd_runs): extra blocks find no tile */                       \
     const long runt = ((long)g.M + TX - 1) / TX, run = 8 * runt;                                        \
     if ((grid + run - 1) / run * run <= max_blocks) grid = (grid + run - 1) / run * run;                \
-    hipLaunchKernelGGL((k_zfaithful<N, ROLE, PARS>), dim3((unsigned)grid), dim3(TX * plan_T(N)), 0, s, g, u, kt, \
+    hipLaunchKernelGGL((k_zfaithful<N, ROLE, PARS, KEEP>), dim3((unsigned)grid), dim3(TX * plan_T(N)), 0, s, g, u, kt, \
                        U, D, G, part, tw, f0, nf, (unsigned)tm, (unsigned)tn, (unsigned)runt);          \
     if (nblocks) *nblocks = grid;                                                                       \
     return 0;                                                                                           \
@@ -359,15 +274,24 @@ static int zf_launch(const Geo& g, const UPar& u, const KTab& kt, Bank<double> U
   }
 }
 
+template <bool KEEP>
+static int zf_role(int role, bool pars, const Geo& g, const UPar& u, const KTab& kt, Bank<double> U, Bank<double> D,
+                   Bank<double> G, double* part, int f0, int nf, long max_blocks, long* nblocks, hipStream_t s) {
+  if (role == FZ_ETA)
+    return pars ? zf_launch<FZ_ETA, true, KEEP>(g, u, kt, U, D, G, part, f0, nf, max_blocks, nblocks, s)
+                : zf_launch<FZ_ETA, false, KEEP>(g, u, kt, U, D, G, part, f0, nf, max_blocks, nblocks, s);
+  if (role == FZ_GHAT)
+    return pars ? zf_launch<FZ_GHAT, true, KEEP>(g, u, kt, U, D, G, part, f0, nf, max_blocks, nblocks, s)
+                : zf_launch<FZ_GHAT, false, KEEP>(g, u, kt, U, D, G, part, f0, nf, max_blocks, nblocks, s);
+  return zf_launch<FZ_CMOB, false, KEEP>(g, u, kt, U, D, G, part, f0, nf, max_blocks, nblocks, s);
+}
+
 int faithful_z(int role, bool pars, const Geo& g, const UPar& u, const KTab& kt, Bank<double> U, Bank<double> D,
                Bank<double> G, double* part, int f0, int nf, long max_blocks, long* nblocks, hipStream_t s) {
-  if (role == FZ_ETA)
-    return pars ? zf_launch<FZ_ETA, true>(g, u, kt, U, D, G, part, f0, nf, max_blocks, nblocks, s)
-                : zf_launch<FZ_ETA, false>(g, u, kt, U, D, G, part, f0, nf, max_blocks, nblocks, s);
-  if (role == FZ_GHAT)
-    return pars ? zf_launch<FZ_GHAT, true>(g, u, kt, U, D, G, part, f0, nf, max_blocks, nblocks, s)
-                : zf_launch<FZ_GHAT, false>(g, u, kt, U, D, G, part, f0, nf, max_blocks, nblocks, s);
-  return zf_launch<FZ_CMOB, false>(g, u, kt, U, D, G, part, f0, nf, max_blocks, nblocks, s);
+  // the state and derivative banks together
+  return bank_stays(2ul * g.F * g.P * sizeof(double))
+             ? zf_role<true>(role, pars, g, u, kt, U, D, G, part, f0, nf, max_blocks, nblocks, s)
+             : zf_role<false>(role, pars, g, u, kt, U, D, G, part, f0, nf, max_blocks, nblocks, s);
 }
 
 }  // namespace pf

@@ -278,16 +278,12 @@ int y_pass(int ny, bool inv, c2<R>* main, c2<R>* nyq, long M, long nlines, hipSt
 #define PF_CASE(N)                                                                                     \
   case N: {                                                                                            \
     constexpr int TX = col_tile(N, sizeof(c2<R>));                                                     \
-    /* a multiple of 8 blocks for the XCD order (xcd_block); the extra blocks fall on Nyquist lines  */ \
-    /* past the last one and touch no memory                                                         */ \
-    const unsigned tiles = ceil_div(M * nlines, TX) + ceil_div(nlines, TX);                            \
-    dim3 grid((tiles + 7) / 8 * 8), block(TX * plan_T(N));                                             \
-    if (inv)                                                                                           \
-      hipLaunchKernelGGL((k_ypass<R, N, true>), grid, block, 0, s, main, nyq, M, nlines, nlines, tw,   \
-                         (const Member<R>*)nullptr, 0L);                                               \
-    else                                                                                               \
-      hipLaunchKernelGGL((k_ypass<R, N, false>), grid, block, 0, s, main, nyq, M, nlines, nlines, tw,  \
-                         (const Member<R>*)nullptr, 0L);                                               \
+    dim3 grid(ypass_grid(ceil_div(M * nlines, TX), ceil_div(nlines, TX))), block(TX * plan_T(N));      \
+    const bool keep = bank_stays(2ul * sizeof(R) * M * N * nlines);                                    \
+    auto kernel = inv ? (keep ? &k_ypass<R, N, true, false, true> : &k_ypass<R, N, true>)              \
+                      : (keep ? &k_ypass<R, N, false, false, true> : &k_ypass<R, N, false>);           \
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, main, nyq, M, nlines, nlines, tw,                    \
+                       (const Member<R>*)nullptr, 0L);                                                 \
     break;                                                                                             \
   }
     PF_GRID_SIZES(PF_CASE)

@@ -30,8 +30,23 @@ template <typename R, bool INV> __device__ __forceinline__ c2<R> mul_mi(c2<R> a)
   return INV ? mk<R>(-a.y, a.x) : mk<R>(a.y, -a.x);
 }
 
-// Streaming global accesses: the fused passes read and write each element of
-// a bank once, so these carry the non-temporal hint (no retention in L2/MALL).
+// Cache policy of the passes over a bank.  Each pass reads and writes every element
+// once, but the next pass reads them again: a bank that fits the 256 MiB last level
+// cache is accessed plainly and stays there from pass to pass, a larger one with the
+// non-temporal hint, which spares the cache a stream it cannot hold.  y pass in
+// place: 160^3 x 9 FP32 (147 MB) 41 us plain, 58 us hinted; 192^3 x 9 (255 MB) 63
+// and 101 us; one FP64 field of 256^3 (134 MB) 37 and 50 us; 256^3 x 17 FP64 (2.3
+// GB) 823 and 765 us; 512 x 128 x 128 x 37 FP32 (1.2 GB) 457 and 427 us.
+// A bank that fits the XCDs' L2s together is hinted too: written plainly it sits
+// there dirty when the pass ends and has to be written back before the next pass,
+// on other XCDs, can start (steps, plain and hinted: 64^3 x 9 FP32, 9 MB, 42.0 and
+// 37.7 us; 160 x 96 x 48 x 6, 18 MB, 66.7 and 55.9 us; 96^3 x 9, 32 MB, 85.3 and
+// 90.6 us).
+constexpr unsigned long kCacheBytes = 256ul << 20, kL2Bytes = 24ul << 20;
+__host__ __device__ __forceinline__ bool bank_stays(unsigned long bytes) {
+  return bytes > kL2Bytes && bytes <= kCacheBytes;
+}
+
 template <typename R> __device__ __forceinline__ c2<R> ld_nt(const c2<R>* p) {
   typedef R N __attribute__((ext_vector_type(2)));
   const N v = __builtin_nontemporal_load(reinterpret_cast<const N*>(p));
@@ -58,6 +73,10 @@ __device__ __forceinline__ BufRes buf_res(const void* base, unsigned bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
 }
 constexpr int kBufNT = 2;
+// Lane offset of a lane without work: past every range (they are below 2^32 - 16
+// bytes), so its loads read 0 and its stores are dropped with no branch around
+// each access.
+constexpr unsigned kBufOut = 0xFFFFFFFFu;
 template <typename R, int AUX = kBufNT> __device__ __forceinline__ c2<R> buf_ld(BufRes r, unsigned voff, unsigned soff) {
   if constexpr (sizeof(R) == 4) {
     typedef unsigned U __attribute__((ext_vector_type(2)));

@@ -97,6 +97,19 @@ __host__ __device__ constexpr int plan_alt(int N, int V, int p) {
       default: return 0;
     }
   }
+  // V = 4 (FP32), 5 (FP64): the x line's plans (its rows are half an axis long), with
+  // 4 threads for the short lengths whose default plan has one or two; in FP64 96
+  // points take 12 threads of 8 values (192^3 x 9: x line 295 -> 266 us), in FP32
+  // the default plan is better (132 against 145 us)
+  if (V == 4 || V == 5) {
+    switch (N) {
+      case 96: { const int r[3] = {8, 4, 3}; return V == 4 ? 0 : p < 3 ? r[p] : 1; }
+      case 16: { const int r[2] = {4, 4}; return p < 2 ? r[p] : 1; }
+      case 24: { const int r[2] = {6, 4}; return p < 2 ? r[p] : 1; }
+      case 32: { const int r[2] = {8, 4}; return p < 2 ? r[p] : 1; }
+      default: return 0;
+    }
+  }
   if (V == 2) {
     switch (N) {
       case 64: { const int r[2] = {4, 16}; return p < 2 ? r[p] : 1; }

@@ -41,21 +41,6 @@ __device__ __forceinline__ double bsum(double v, double* red) {
     for (int i = 0; i < nw; ++i) s += red[i];
   return s;
 }
-template <bool MAX> __device__ __forceinline__ double bext(double v, double* red) {
-  v = wave_ext<MAX>(v);
-  const int w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[w] = v;
-  __syncthreads();
-  double s = v;
-  if (threadIdx.x == 0) {
-    s = red[0];
-    for (int i = 1; i < nw; ++i)
-      if (MAX ? (red[i] > s) : (red[i] < s)) s = red[i];
-  }
-  return s;
-}
-
 // Nonlinear terms for NPT = 1 point or NPT = 2 neighbouring points (x = 2k,
 // 2k+1: the two halves of one complex LDS element per field), reduced O(var)
 // form (gamma block structure of src/var_diff.f90:206-218).  v: field 0 = c,
@@ -170,35 +155,26 @@ __device__ __forceinline__ void nl_points(typename Pts<R, NPT>::T* v, long fs, i
 //   XONLY  : mobility-chain variant for one field: C2R, multiply by mobd, R2C.
 // One job = one (field, line) x transform, done by T = plan_T(M) threads.  The
 // LDS tile is job-major: job j's M complex elements in row j, pitch MP.
-//   * When T divides 64 and the plan has at most two passes (every length but
-//     M = 80 and 96), a job's T threads are
-//     consecutive lanes of one wave (t = tid % T), so the transforms' exchanges
-//     stay inside the wave and need no block barrier (XF_WAVE).  Element k of a
-//     row sits at lds_swz(k) = k + k / 16 (XF_SWZ) and the pitch MP is chosen
-//     from a model of the LDS banks over every access pattern of the kernel
+//   * A job's T threads are lanes of one wave (xline_wave_jobs), so the transforms'
+//     exchanges stay inside the wave and need no block barrier (XF_WAVE).  Element
+//     k of a row sits at lds_swz(k) = k + k / 16 (XF_SWZ) and the pitch MP is
+//     chosen from a model of the LDS banks over every access pattern of the kernel
 //     (exchanges, pairing k with M - k, rows by lanes): the strided exchange
 //     accesses of the T lanes and of the 64 / T jobs of a wave then mostly fall
 //     on distinct banks.
-//   * Otherwise lanes run consecutive jobs (job = tid % njobs) with the odd
-//     pitch MP = M + 1, and each exchange is bracketed by block barriers.
-// Threads beyond the njobs*T that carry the transforms: with wave-local rows
-// they sit in the last wave next to active lanes and skip the transform phases
-// as a whole (one branch, no per-slot predicates, no barrier inside); otherwise
-// they run the same schedule on a spare row njobs, so no slot is predicated.
+// Lanes past the jobs skip the transform phases as a whole (one branch, no
+// per-slot predicates, no barrier inside).
 // A last wave that holds a single job hands it to all its lanes (plan variant
 // 3, where the length has one).
-// Staging and the final store move whole rows, one per wave at a time.  For
-// 256-point rows they also do the real <-> half-complex pairing, a lane taking
-// elements k and M - k together (xline_partner, xline_pair_rows); shorter rows
-// are paired by the transform threads as they load (C2R) and by the store's
-// lanes (R2C), with the Nyquist values staged in LDS.  256-point FP32 rows
-// (kXlineTwiddleRegs) skip the final store's row pass: each job's 16 threads
-// pair their forward transform's outputs by DPP and store them (phase 5).
-// The table W_NX^k, k < NX, is copied to LDS once per block: the pairing reads
-// k < M, the x transforms (length M, stride 2) the rest.
-// Dynamic LDS: (rows*MP + NX) complex (+ njobs + 1 reals for the Nyquist values
-// of rows the staging does not pair) + 16 doubles, rows = njobs (+1 for the
-// spare row without wave-local rows).
+// Staging and the final store move whole rows, one or more per wave at a time, and
+// do the real <-> half-complex pairing, a lane taking elements k and M - k
+// together.  256-point FP32 rows (kXlineTwiddleRegs) skip the final store's row
+// pass: each job's 16 threads pair their forward transform's outputs by DPP and
+// store them (phase 5).
+// The table W_NX^k, k < NX, is copied to LDS once per block for the x transforms
+// (length M, stride 2).
+// Dynamic LDS: (njobs*MP + NX) complex; the block's diagnostics take six doubles per
+// wave of it at the end.
 // ---------------------------------------------------------------------------
 // Threads per x-line block: FP32 blocks may use 1024 threads, which a 512^3 grid
 // with 37 fields needs (37 transforms x 16 threads); FP64 blocks stop at 512
@@ -207,35 +183,31 @@ template <typename R> constexpr int kXlineMaxThreads = sizeof(R) == 4 ? 1024 : 5
 // FP64 blocks of 512-point lines may use 640 threads (37 fields x 16), 3 waves
 // per SIMD at most, which their registers allow.
 template <typename R, int NX> constexpr int kXlineMaxThreadsN = (sizeof(R) == 8 && NX >= 512) ? 640 : kXlineMaxThreads<R>;
-// Minimum waves per SIMD asked of the register allocator.  FP32: 5 (at most 102
-// VGPRs; the 256-point kernel takes 92, so 5 three-wave blocks fit a CU's
-// SIMDs with room for a sixth).  FP64: 3 (the 256-point kernel takes 141 VGPRs
-// with no spills).
-template <typename R> constexpr int kXlineWaves = sizeof(R) == 4 ? 5 : 3;
-// 512-point FP32 lines keep their last transform pass's twiddles in registers
-// (kXlineTwiddleRegs): at most 128 VGPRs, which 1024-thread blocks need anyway.
-template <typename R, int NX> constexpr int kXlineWavesN = (sizeof(R) == 4 && NX >= 512) ? 4 : kXlineWaves<R>;
-// Rows each wave keeps in flight when staging a line group.
-constexpr int kXlineRows = 2;
-
-// Wave-local rows for one- and two-pass plans whose T divides 64; the three-pass
-// plan of 96 points spilled 15 VGPRs per lane that way and ran 19% slower at
-// 192^3, so it keeps block barriers, as does 80 (T = 10).
-__host__ __device__ constexpr bool xline_wave_local(int M) { return 64 % plan_T(M) == 0 && plan_np(M) <= 2; }
+// Minimum waves per SIMD asked of the register allocator.  FP32: 6 for 128- and
+// 160-point lines, which then take up to 79 VGPRs without spills (160^3 x 9: 114 ->
+// 102 us against asking for 5); 5 for the others (at 192 points 6 spilled 4 VGPRs,
+// 192^3 x 9 145 -> 185 us; at 256 points 23, 512 -> 694 us); 4 for 512-point lines, which keep their last transform pass's
+// twiddles in registers (kXlineTwiddleRegs), at most 128 VGPRs, which 1024-thread
+// blocks need anyway.  FP64: 3 (the 256-point kernel takes 167 VGPRs).
+template <typename R, int NX>
+constexpr int kXlineWavesN = sizeof(R) == 8 ? 3 : NX >= 512 ? 4 : (NX >= 128 && NX < 192) ? 6 : 5;
+// The x line's transform plan: variant 4 or 5 where it has one, else the default.
+__host__ __device__ constexpr int xline_plan(int cbytes) { return cbytes == 16 ? 5 : 4; }
+__host__ __device__ constexpr int xline_T(int M, int cbytes) { return plan_T(M, xline_plan(cbytes)); }
+// A job's T threads are lanes of one wave: 64 / T jobs a wave, the lanes past them idle.
+__host__ __device__ constexpr int xline_wave_jobs(int M, int cbytes) { return 64 / xline_T(M, cbytes); }
 // FP64 rows of 256 points are not padded: a 16-byte access serves 16 lanes a
 // cycle, which are one job's T = 16 threads in the exchanges and consecutive
 // elements in the row-wise phases, so the rows need no skew; unpadded, 37 fields
 // fit one block's LDS (148 KiB of rows).
 __host__ __device__ constexpr bool xline_plain_rows(int M, int cbytes) { return cbytes == 16 && M >= 256; }
 __host__ __device__ constexpr int xline_xf(int M, int cbytes) {
-  return xline_wave_local(M) ? (XF_WAVE | (xline_plain_rows(M, cbytes) ? 0 : XF_SWZ)) : 0;
+  return XF_WAVE | (xline_plain_rows(M, cbytes) ? 0 : XF_SWZ);
 }
-__host__ __device__ constexpr int xline_rows(int M, int njobs) { return njobs + (xline_wave_local(M) ? 0 : 1); }
 // Row pitch in elements of cbytes bytes: the bank-model choices for FP32
 // elements; FP64 rows take the smallest padded pitch (at 512 points they must
 // fit 33 rows of 16-byte elements in LDS).
 __host__ __device__ constexpr int xline_row_pitch(int M, int cbytes) {
-  if (!xline_wave_local(M)) return M | 1;
   if (xline_plain_rows(M, cbytes)) return M;
   if (cbytes != 8) return M + M / 16 + 1;
   switch (M) {  // smallest of the bank model's best choices, >= M + M / 16
@@ -256,87 +228,83 @@ __host__ __device__ constexpr int xline_row_pitch(int M, int cbytes) {
 // the wave issues far fewer transform instructions (at 256^3 x 17, 17 jobs of 8
 // threads: x-line kernel 0.577 -> 0.532 ms).
 __host__ __device__ constexpr bool xline_has_wide(int M) {
-  return xline_wave_local(M) && plan_T(M) < 64 && (M == 64 || M == 128 || M == 256);
+  return M == 64 || M == 128 || M == 256;
 }
 
-// Phases 2 and 3 when the staging did not pair (xline_pair_rows false): the C2R
-// pre-processing from the raw row straight into the transform's input
-// registers, then the inverse transform in place, as xline_fft.
-// The partner of slot s's element k = t + T s (pass 0 has one butterfly per
-// thread, NB = T) is (M - k) mod M = u + T c, u = T - t, c = M / T - 1 - s; for
-// k = 0 this reads element M instead, one past the row (inside the LDS tile,
-// and not used).  In a swizzled row (e + e / 16) its address is a per-lane base,
-// one for each residue of c mod 16 / T, plus a compile-time offset; computed
-// per slot the swizzle took six or seven VALU instructions a slot.
-template <typename R, int M, int V, int XF>
-__device__ __forceinline__ void xline_c2r(c2<R>* v, c2<R>* col, const c2<R>* shw, const R* xn, int t) {
-  constexpr int T = plan_T(M, V);
-  static_assert(PassC<M, 0, V>::NB == T && PassC<M, 0, V>::Q == 1, "pass 0: element t + T s in slot s");
-  constexpr int NR = T < 16 ? 16 / T : 1;
-  const int u = T - t;
-  int mb[NR];
-#pragma unroll
-  for (int r = 0; r < NR; ++r) mb[r] = u + ((u + T * r) >> 4);
-#pragma unroll
-  for (int s = 0; s < kInSlots<M, V>; ++s) {
-    if (!rfft_in_valid<M, V>(t, s)) continue;
-    const int k = rfft_in_idx<M, V>(t, s);
-    const int c = M / T - 1 - s;
-    const int mi = (XF & XF_SWZ) ? mb[c % NR] + T * c + (T < 16 ? c / NR : T * c / 16) : (M - k) % M;
-    // k = 0 pairs with the Nyquist entry (its c2r_pre value is not used)
-    const c2<R> pk = c2r_pre<R>(col[lds_swz<XF>(k)], col[mi], shw[k]);
-    const R a0 = col[0].x;
-    v[s] = (k == 0) ? mk<R>(a0 + *xn, a0 - *xn) : pk;
-  }
-  rfft<R, M, true, 1, V, XF>(v, t, true, col, shw, 2);
-#pragma unroll
-  for (int s = 0; s < kOutSlots<M, V>; ++s)
-    if (rfft_out_valid<M, V>(t, s)) col[lds_swz<XF>(rfft_out_idx<M, V>(t, s))] = v[s];
-}
 // One job's x transform with plan V, in place in its LDS row (phases 3 and 5).
 // No barrier before the write-back: the last Stockham pass leaves each
 // thread's outputs at exactly the elements it loaded as that pass's inputs
 // (out_idx = in_idx when j < NB = LS), so no thread overwrites an element
 // another thread has yet to read.
+// The Nyquist value goes with thread 0, which holds Z_0 = (X_0 + X_M, X_0 - X_M) in
+// slot 0: inverse, xn (0 in the other threads) completes it; forward, X_M = Z_0.x -
+// Z_0.y goes to *wn (null in the other threads) times scale.
 template <typename R, int M, int V, int XF, bool INV, bool TWR = false>
-__device__ __forceinline__ void xline_fft(c2<R>* v, c2<R>* col, const c2<R>* shw, int t,
+__device__ __forceinline__ void xline_fft(c2<R>* v, c2<R>* col, const c2<R>* shw, int t, R xn, c2<R>* wn, R scale,
                                           const c2<R>* twr = nullptr) {
 #pragma unroll
   for (int s = 0; s < kInSlots<M, V>; ++s)
     if (rfft_in_valid<M, V>(t, s)) v[s] = col[lds_swz<XF>(rfft_in_idx<M, V>(t, s))];
+  if (INV) v[0] = mk<R>(v[0].x + xn, v[0].y - xn);
   rfft<R, M, INV, 1, V, XF, TWR>(v, t, true, col, shw, 2, 0, twr);
+  if (!INV && wn) *wn = mk<R>((v[0].x - v[0].y) * scale, R(0));
 #pragma unroll
   for (int s = 0; s < kOutSlots<M, V>; ++s)
     if (rfft_out_valid<M, V>(t, s)) col[lds_swz<XF>(rfft_out_idx<M, V>(t, s))] = v[s];
 }
 
 // The real <-> half-complex pairing couples element k of a row with element
-// M - k.  A lane takes both: pair p < M / 2 is (p, M - p), and p = 0 stands for
-// the two self-coupled entries, 0 (with the Nyquist value) and M / 2.  Each
-// element is then read once and the twiddle of M - p follows from that of p,
-// W_NX^(M-p) = -conj(W_NX^p) (bit for bit: the table is built by exact quadrant
-// symmetries); W_NX^(M/2) = (-0, -1) exactly.
+// M - k, and the moving waves do it: a lane takes both elements of a pair, from
+// HBM when a row is staged and to HBM when it is stored.  Pair p < M / 2 is
+// (p, M - p); p = 0 stands for the two self-coupled entries, 0 (with the Nyquist
+// value) and M / 2.  A pair's sums and its one twiddle product W_NX^p serve both
+// elements (the mirrored element's differ by signs, W_NX^(M-p) = -conj(W_NX^p)),
+// about half the arithmetic of two single elements, and every element is read from
+// LDS once.  With the pairing one element at a time and vector row addresses, and
+// blocks of several line groups: 192^3 x 9 FP32 210 us, 96^3 x 9 30.8, FP64 256^3 x
+// 17 1193, 64^3 x 9 26.3; as it is 145, 24.9, 1043 and 15.6 us.
 template <int M> __device__ __forceinline__ int xline_partner(int p) { return p ? M - p : M / 2; }
-// Where the pairings happen: in the staging and the final store (each wave's
-// lanes pair the row they move), or in the transform threads' loads and the
-// store's lanes, from the raw rows (three LDS reads per element, the Nyquist
-// values in LDS too).  256-point rows are paired by the moving waves (512^3 x
-// 37: x line 15.4 -> 14.7 ms; the kernel is bound by LDS traffic there).  At
-// 128 points and fewer, pairing in the staging made the x line slower (256^3 x
-// 17: 0.532 -> 0.553 ms; 128^3 x 9: 0.061 -> 0.078 ms, half the lanes idle in a
-// 64-point row's pairs) and pairing in the store alone moved it by less than
-// the run-to-run spread.
-__host__ __device__ constexpr bool xline_pair_rows(int M) { return M >= 256; }
+// C2R of a pair: a = X_p, b = X_{M-p} (p = 0: X_0, X_{M/2}) -> Z_p in a, Z_{M-p} in b
+// (p = 0: Z_0 without the Nyquist value X_M, which the transform's thread adds, and
+// Z_{M/2}).  X_0's imaginary part is not used.
+template <typename R> __device__ __forceinline__ void xline_c2r_pair(c2<R>& a, c2<R>& b, c2<R> w, bool p0) {
+  const R ay = p0 ? R(0) : a.y, bx = p0 ? R(0) : b.x, by = p0 ? R(0) : b.y;
+  const R ar = a.x + bx, ai = ay - by, br = a.x - bx, bi = ay + by;
+  const R cr = w.x * br + w.y * bi, ci = w.x * bi - w.y * br;
+  a = mk<R>(ar - ci, ai + cr);
+  b = mk<R>(p0 ? R(2) * b.x : ar + ci, p0 ? R(-2) * b.y : cr - ai);
+}
+// R2C of a pair: a = Z_p, b = Z_{M-p} (p = 0: Z_0, Z_{M/2}) -> X_p in a and
+// X_{M-p} in b (p = 0: X_0, X_{M/2}); hs = scale / 2.
+template <typename R> __device__ __forceinline__ void xline_r2c_pair(c2<R>& a, c2<R>& b, c2<R> w, bool p0, R hs) {
+  const R bx = p0 ? a.x : b.x, by = p0 ? a.y : b.y;
+  const R ar = a.x + bx, ai = a.y - by, br = a.x - bx, bi = a.y + by;
+  const R cr = w.x * br - w.y * bi, ci = w.x * bi + w.y * br;
+  const R mx = hs * (ar - ci), my = hs * (-ai - cr);
+  a = mk<R>(hs * (ar + ci), hs * (ai - cr));
+  b = mk<R>(p0 ? R(2) * hs * b.x : mx, p0 ? R(-2) * hs * b.y : my);
+}
+// Rows of one field that a wave moves at once: rows of M / 2 pairs, as many of the
+// group's LINES as its 64 lanes hold (a power of two; every lane then has a fixed
+// row and pair, the rest of the address is scalar).
+__host__ __device__ constexpr int xline_rows_at_once(int M, int LINES) {
+  int r = 1;
+  while (2 * r <= LINES && 2 * r * (M / 2) <= 64) r *= 2;
+  return r;
+}
+// Row groups whose loads a wave keeps in flight: 2; in FP64 3 for 64 and 128 points
+// (128^3 x 9: 71.0 -> 67.9 us, 256^3 x 17: 1088 -> 1043 us), where that costs no
+// wave per SIMD (at 96 points it did, 192^3 x 9: 338 -> 383 us), and 1 for 256
+// points, two pairs a lane (more spilled: 512 x 128 x 128 x 9 348 -> 414 us).
+__host__ __device__ constexpr int xline_ahead(int M, int cbytes) {
+  return cbytes == 8 ? 2 : (M == 64 || M == 128) ? 3 : M == 256 ? 1 : 2;
+}
 // 256-point FP32 rows: the last transform pass (radix 16, one butterfly per
 // thread) takes its 15 twiddles, the same for every line and both directions,
 // from registers loaded once per block rather than from the LDS table.  Those
 // blocks hold a CU's LDS alone (37 fields: 85 KB), whose traffic bounds them.
 template <typename R, int M>
-constexpr bool kXlineTwiddleRegs = xline_pair_rows(M) && sizeof(R) == 4 && LastPass<M>::Q == 1 && LastPass<M>::LS > 1;
-template <typename R> __device__ __forceinline__ c2<R> xline_mirror_tw(c2<R> w, int p) {
-  return p ? mk<R>(-w.x, w.y) : mk<R>(R(-0.0), R(-1));
-}
-
+constexpr bool kXlineTwiddleRegs = M >= 256 && sizeof(R) == 4 && LastPass<M>::Q == 1 && LastPass<M>::LS > 1;
 // Lane t of a 16-lane row receives x from lane (16 - t) mod 16 of the same row:
 // DPP row_mirror (lane 15 - t) then row_ror:1 (from lane t - 1), register moves
 // with no LDS traffic.
@@ -344,6 +312,19 @@ __device__ __forceinline__ float dpp_partner16(float x) {
   const int m = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x140, 0xF, 0xF, false);
   const int r = __builtin_amdgcn_update_dpp(0, m, 0x121, 0xF, 0xF, false);
   return __builtin_bit_cast(float, r);
+}
+
+// Blocks for ngroups line groups, at most cap: one group each, or an equal number of
+// consecutive groups each.  Every block then has its full share but the last; with
+// a grid cut at cap itself some blocks carry one group more than others or (ranges of
+// ceil(ngroups / cap)) whole XCDs end up without work.  192^3 x 9 in FP32 (18 432
+// groups): 220 us cut at 16 384 blocks, 174 us at 8 192, 129 us with one group
+// each; 160^3 x 9: 103 us at 8 192, 84 us with one group each; 256^3 x 17 (65 536
+// groups): 513 us at 8 192, 506 to 514 us with one or two each.
+constexpr long kXlineGroupCap = 65536;
+inline long xline_grid(long ngroups, long cap) {
+  const long chunk = (ngroups + cap - 1) / cap, grid = (ngroups + chunk - 1) / chunk;
+  return grid < 8 ? grid : (grid + 7) / 8 * 8;  // a multiple of 8 for the XCD order
 }
 
 // BATCH: ngroups counts the line groups of every member in mt (member m owns
@@ -354,63 +335,84 @@ template <typename R> __device__ __forceinline__ const UPar& member_u(const UPar
   return batch ? mt[m].u : u;
 }
 
-template <typename R, int NX, int LINES, bool XONLY, bool BATCH = false>
+// A block's diagnostics from its threads': wave results side by side in red (LDS, free
+// by now), then one thread per value takes the waves' in order.
+__device__ __forceinline__ void diag_partials(double ch, double eta, double cmax, double cmin, double pmin, double p3,
+                                              double* red, int nw, double* __restrict__ part) {
+  const double r0 = wave_sum(ch), r1 = wave_sum(eta);
+  const double r2 = wave_ext<true>(cmax), r3 = wave_ext<false>(cmin);
+  const double r4 = wave_ext<false>(pmin), r5 = wave_ext<true>(p3);
+  if ((threadIdx.x & 63) == 0) {
+    double* o = red + 6 * (threadIdx.x >> 6);
+    o[0] = r0; o[1] = r1; o[2] = r2; o[3] = r3; o[4] = r4; o[5] = r5;
+  }
+  __syncthreads();
+  const int i = threadIdx.x;
+  if (i < 6) {
+    double s = red[i];
+    for (int w = 1; w < nw; ++w) {
+      const double x = red[6 * w + i];
+      s = i < 2 ? s + x : (i == 2 || i == 5) ? (x > s ? x : s) : (x < s ? x : s);
+    }
+    part[(long)blockIdx.x * 6 + i] = s;
+  }
+}
+
+// KEEP: W stays in cache from pass to pass (bank_stays).
+// ROUNDS: the jobs need more threads than a block may have, and the block's waves
+// take them in several rounds (in one loop with the common case its registers
+// spilled: 256^3 x 17 516 -> 684 us).
+template <typename R, int NX, int LINES, bool XONLY, bool BATCH = false, bool KEEP = false, bool ROUNDS = false>
 __global__ void __launch_bounds__((kXlineMaxThreadsN<R, NX>)) __attribute__((amdgpu_waves_per_eu(kXlineWavesN<R, NX>)))
 k_xline(Geo g, UPar u, c2<R>* __restrict__ wm, c2<R>* __restrict__ wn, R* __restrict__ mobd,
         const c2<R>* __restrict__ tw, double* __restrict__ part, long ngroups, int diag, int mob,
         const Member<R>* __restrict__ mt) {
-  constexpr int M = NX / 2, T = plan_T(M);
+  constexpr int M = NX / 2, XV = xline_plan(sizeof(c2<R>)), T = plan_T(M, XV);
   constexpr int MP = xline_row_pitch(M, sizeof(c2<R>)), XF = xline_xf(M, sizeof(c2<R>));
-  constexpr bool WX = xline_wave_local(M), HAVEW = xline_has_wide(M);
+  constexpr bool HAVEW = xline_has_wide(M);
   // the wide plan's variant (3) and threads; the T-thread plan stands in when
   // this length has no wide plan, and that branch is never taken then
-  constexpr int WV = HAVEW ? 3 : 0, TW = plan_T(M, WV), JW = HAVEW ? 64 / T : 1;
-  static_assert(last_pass_in_place<M>(), "the write-backs after the x transforms rely on it");
+  constexpr int WV = HAVEW ? 3 : XV, TW = plan_T(M, WV), JW = xline_wave_jobs(M, sizeof(c2<R>));
+  static_assert(last_pass_in_place<M, XV>(), "the write-backs after the x transforms rely on it");
   extern __shared__ unsigned char smem[];
   const int F = XONLY ? 1 : g.F;
   const int njobs = F * LINES;
   c2<R>* sh = reinterpret_cast<c2<R>*>(smem);
-  const int rows = xline_rows(M, njobs);
-  constexpr bool PP = xline_pair_rows(M), TR = kXlineTwiddleRegs<R, M>;
-  c2<R>* shw = sh + (long)rows * MP;  // W_NX^k, k < NX
-  R* shn = reinterpret_cast<R*>(shw + NX);  // Nyquist values (without PP)
-  double* red = reinterpret_cast<double*>(smem + (((sizeof(c2<R>) * ((size_t)rows * MP + NX) +
-                                                    (PP ? 0 : sizeof(R) * (njobs + 1))) + 15) & ~(size_t)15));
+  constexpr bool TR = kXlineTwiddleRegs<R, M>;
+  c2<R>* shw = sh + (long)njobs * MP;  // W_NX^k, k < NX
   const int nt = blockDim.x, nw = nt >> 6;
-  constexpr int PPL = (M / 2 + 63) / 64;  // element pairs per lane when a wave moves a row
-  constexpr int KPL = (M + 63) / 64;      // row elements per lane when a wave moves a row
+  constexpr int H = M / 2, PPL = (H + 63) / 64;  // pairs of a row, and per lane
+  constexpr int RP = xline_rows_at_once(M, LINES), NA = xline_ahead(M, sizeof(c2<R>));
+  const int npieces = F * (LINES / RP);
   for (int k = threadIdx.x; k < NX; k += nt) shw[k] = tw[k];
-  __syncthreads();  // the staging of the first line group reads the table
+  if constexpr (TR) __syncthreads();
   c2<R> twr[TR ? LastPass<M>::r - 1 : 1];
-  if constexpr (TR) last_pass_twiddles<R, M>(twr, threadIdx.x % T, shw, 2);
+  if constexpr (TR) last_pass_twiddles<R, M>(twr, (threadIdx.x & 63) % T, shw, 2);
   const R scale = (R)u.invP;
   double a_ch = 0.0, a_eta = 0.0;
   R cmax = 0, cmin = 1, pmin = 1, p3 = 0;
-  c2<R> v[plan_E(M) > plan_E(M, WV) ? plan_E(M) : plan_E(M, WV)];
+  c2<R> v[plan_E(M, XV) > plan_E(M, WV) ? plan_E(M, XV) : plan_E(M, WV)];
 
-  const long lb = xcd_block(blockIdx.x, gridDim.x);
-  const long chunk = (ngroups + gridDim.x - 1) / gridDim.x;
-  const long lg_end = ((lb + 1) * chunk < ngroups) ? (lb + 1) * chunk : ngroups;
-  for (long lg = lb * chunk; lg < lg_end; ++lg) {
+  // each block takes the same number of consecutive line groups (xline_grid)
+  const unsigned lb = (unsigned)xcd_block(blockIdx.x, gridDim.x);
+  const unsigned chunk = ((unsigned)ngroups + gridDim.x - 1) / gridDim.x;
+  const unsigned lg0 = lb * chunk, lg1 = lg0 + chunk < (unsigned)ngroups ? lg0 + chunk : (unsigned)ngroups;
+  for (long lg = lg0; lg < lg1; ++lg) {
     // Per-thread indices are recomputed each iteration from an opaque copy of
     // the thread id: hoisted, the addresses derived from them stayed live across
     // the loop (and the transforms' twiddles, read from global memory, too),
     // 126 VGPRs at 256^3 x 17; recomputed, with the twiddles from LDS, 90.
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
-    const int lane = tid & 63, wv = tid >> 6;
-    const int job = WX ? tid / T : tid % njobs, tq = WX ? tid % T : tid / njobs;
-    // threads beyond the njobs*T run the same schedule on a spare row, so the
-    // transform phases carry no per-slot predicates
-    const bool act = WX ? job < njobs : tq < T;
-    const int t = act ? tq : tq % T;
-    __builtin_assume(t >= 0 && t < T);
-    const int row = act ? job : njobs;
-    c2<R>* col = sh + row * MP;
+    const int lane = tid & 63;
+    // the wave's number, uniform: the rows a wave moves then have scalar addresses
+    const int wv = __builtin_amdgcn_readfirstlane(tid) >> 6;
+    const int t = lane % T;
+    const bool lact = 64 % T == 0 || lane < JW * T;
     // the lone job of the last wave (njobs = 1 mod 64 / T) goes to the whole
     // wave; the condition is uniform over the wave (a scalar branch)
-    const bool wide = HAVEW && njobs % JW == 1 &&
-                      (__builtin_amdgcn_readfirstlane(tid) >> 6) == (njobs - 1) / JW;
+    const bool wide_any = HAVEW && njobs % JW == 1;
+    const auto is_wide = [&](int jr) { return wide_any && jr + wv * JW == njobs - 1; };
     long L0 = lg * LINES, m = 0;
     c2<R>* wmm = wm;
     c2<R>* wnn = wn;
@@ -422,89 +424,72 @@ k_xline(Geo g, UPar u, c2<R>* __restrict__ wm, c2<R>* __restrict__ wn, R* __rest
       wnn = mt[m].Wn;
     }
     const UPar& uu = member_u<R>(u, mt, m, BATCH);
-    if constexpr (PP) {
-      // 1. half lines of every field -> LDS rows, with the C2R pre-processing:
-      //    wave w stages rows w, w + nw, ... (coalesced along k, and along M - k
-      //    in descending order), kXlineRows rows per batch in flight
-      for (int jb0 = wv; jb0 < njobs; jb0 += kXlineRows * nw) {
-        c2<R> ta[kXlineRows][PPL], tb[kXlineRows][PPL];
-        R xn[kXlineRows];
+    // the Nyquist entry of this thread's job in round jr (thread 0 of a job takes it)
+    const auto nyq = [&](int jr, int ln, int lt) -> c2<R>* {
+      const bool wide = is_wide(jr);
+      const int jn = wide ? njobs - 1 : jr + wv * JW + ln / T, fn = jn / LINES;
+      const bool has = wide ? ln == 0 : lact && lt == 0 && jn < njobs;
+      return has ? wnn + (long)fn * g.plane + L0 + (jn - fn * LINES) : nullptr;
+    };
+    R xn = R(0);
+    if (const c2<R>* p = nyq(0, lane, t)) xn = p->x;
+    // this lane's row within a wave's row group and its pairs' elements
+    const int sub = H >= 64 ? 0 : lane / H, p0 = H >= 64 ? lane : lane - sub * H;
+    const bool mine = H >= 64 || sub < RP;
+    // 1. half lines of every field -> LDS rows, with the C2R pre-processing: wave w
+    //    stages row groups w, w + nw, ... (coalesced along k, and along M - k in
+    //    descending order), NA of them in flight
+    c2<R> w[PPL];  // a lane's pairs, and so their twiddles, are the same in every row
 #pragma unroll
-        for (int r = 0; r < kXlineRows; ++r) {
-          const int jb = jb0 + r * nw;
-          if (jb < njobs) {
-            const int f = jb / LINES, l = jb - f * LINES;
-            const c2<R>* src = wmm + (long)f * g.hmain + (L0 + l) * M;
+    for (int i = 0; i < PPL; ++i) w[i] = tw[p0 + 64 * i];
+    for (int j0 = wv; j0 < npieces; j0 += NA * nw) {
+      c2<R> ta[NA][PPL], tb[NA][PPL];
 #pragma unroll
-            for (int j = 0; j < PPL; ++j) {
-              const int p = lane + 64 * j;
-              if ((M / 2) % 64 == 0 || p < M / 2) {
-                ta[r][j] = ld_nt<R>(src + p);
-                tb[r][j] = ld_nt<R>(src + xline_partner<M>(p));
-              }
-            }
-            xn[r] = (lane == 0) ? wnn[(long)f * g.plane + L0 + l].x : R(0);
-          }
-        }
+      for (int r = 0; r < NA; ++r) {
+        const int j = j0 + r * nw;
+        if (j < npieces) {
+          const int f = j / (LINES / RP), l = (j - f * (LINES / RP)) * RP;
+          const c2<R>* src = wmm + (long)f * g.hmain + (L0 + l) * M;
+          if (mine) {
 #pragma unroll
-        for (int r = 0; r < kXlineRows; ++r) {
-          const int jb = jb0 + r * nw;
-          if (jb < njobs) {
-            c2<R>* rw = sh + jb * MP;
-#pragma unroll
-            for (int j = 0; j < PPL; ++j) {
-              const int p = lane + 64 * j;
-              if ((M / 2) % 64 == 0 || p < M / 2) {
-                const c2<R> a = ta[r][j], b = tb[r][j], w = shw[p];
-                rw[lds_swz<XF>(p)] = p ? c2r_pre<R>(a, b, w) : mk<R>(a.x + xn[r], a.x - xn[r]);
-                rw[lds_swz<XF>(xline_partner<M>(p))] = c2r_pre<R>(b, p ? a : b, xline_mirror_tw<R>(w, p));
-              }
+            for (int i = 0; i < PPL; ++i) {
+              const int p = p0 + 64 * i;
+              const c2<R>*a = src + (sub * M + p), *b = src + (sub * M + xline_partner<M>(p));
+              ta[r][i] = KEEP ? *a : ld_nt<R>(a);
+              tb[r][i] = KEEP ? *b : ld_nt<R>(b);
             }
           }
         }
       }
-    } else {
-      // 1. half lines of every field -> LDS rows: wave w stages rows w, w + nw,
-      //    ... (coalesced along k), kXlineRows rows per batch in flight
-      for (int jb0 = wv; jb0 < njobs; jb0 += kXlineRows * nw) {
-        c2<R> tmp[kXlineRows][KPL];
 #pragma unroll
-        for (int r = 0; r < kXlineRows; ++r) {
-          const int jb = jb0 + r * nw;
-          if (jb < njobs) {
-            const int f = jb / LINES, l = jb - f * LINES;
-            const c2<R>* src = wmm + (long)f * g.hmain + (L0 + l) * M;
+      for (int r = 0; r < NA; ++r) {
+        const int j = j0 + r * nw;
+        if (j < npieces && mine) {
+          c2<R>* rw = sh + (j * RP + sub) * MP;
 #pragma unroll
-            for (int kk = 0; kk < KPL; ++kk)
-              if (M % 64 == 0 || lane + 64 * kk < M) tmp[r][kk] = ld_nt<R>(src + lane + 64 * kk);
+          for (int i = 0; i < PPL; ++i) {
+            const int p = p0 + 64 * i;
+            xline_c2r_pair<R>(ta[r][i], tb[r][i], w[i], p == 0);
+            rw[lds_swz<XF>(p)] = ta[r][i];
+            rw[lds_swz<XF>(xline_partner<M>(p))] = tb[r][i];
           }
         }
-#pragma unroll
-        for (int r = 0; r < kXlineRows; ++r) {
-          const int jb = jb0 + r * nw;
-          if (jb < njobs) {
-#pragma unroll
-            for (int kk = 0; kk < KPL; ++kk)
-              if (M % 64 == 0 || lane + 64 * kk < M) sh[jb * MP + lds_swz<XF>(lane + 64 * kk)] = tmp[r][kk];
-          }
-        }
-      }
-      for (int i = tid; i < njobs; i += nt) {
-        const int f = i / LINES, l = i - f * LINES;
-        shn[i] = wnn[(long)f * g.plane + L0 + l].x;
       }
     }
     __syncthreads();
-    // 2-3. (C2R pre-processing and) inverse x transform of each job; real
-    //      pairs z[n] = (x[2n], x[2n+1])
-    if (wide) {
-      if (TW == 64 || lane < TW) {
-        if constexpr (PP) xline_fft<R, M, WV, XF, true>(v, sh + (njobs - 1) * MP, shw, lane);
-        else xline_c2r<R, M, WV, XF>(v, sh + (njobs - 1) * MP, shw, shn + njobs - 1, lane);
+    // 2-3. inverse x transform of each job; real pairs z[n] = (x[2n], x[2n+1]).
+    for (int jr = 0; jr < (ROUNDS ? njobs : 1); jr += ROUNDS ? nw * JW : 1) {
+      const int job = jr + wv * JW + lane / T;
+      if (jr > 0) {
+        const c2<R>* p = nyq(jr, lane, t);
+        xn = p ? p->x : R(0);
       }
-    } else if (!WX || act) {
-      if constexpr (PP) xline_fft<R, M, 0, XF, true, TR>(v, col, shw, t, twr);
-      else xline_c2r<R, M, 0, XF>(v, col, shw, shn + row, t);
+      if (is_wide(jr)) {
+        if (TW == 64 || lane < TW)
+          xline_fft<R, M, WV, XF, true>(v, sh + (njobs - 1) * MP, shw, lane, xn, nullptr, scale);
+      } else if (lact && job < njobs) {
+        xline_fft<R, M, XV, XF, true, TR>(v, sh + job * MP, shw, t, xn, nullptr, scale, twr);
+      }
     }
     __syncthreads();
     // 4. pointwise: point x of line l is component x%2 of element x/2 of row
@@ -553,78 +538,72 @@ k_xline(Geo g, UPar u, c2<R>* __restrict__ wm, c2<R>* __restrict__ wn, R* __rest
     //    come by DPP instead of a write-back and a second read of the row (512^3
     //    x 37: x line 13.5-13.8 -> 13.0-13.1 ms).  The lone wide job, if any,
     //    still goes through its row and phase 6.
-    const bool wide_any = HAVEW && njobs % JW == 1;
-    if (wide) {
-      if (TW == 64 || lane < TW) xline_fft<R, M, WV, XF, false>(v, sh + (njobs - 1) * MP, shw, lane);
-    } else if (!WX || act) {
-      if constexpr (TR) {
-        static_assert(T == 16 && kInSlots<M> == 16 && kOutSlots<M> == 16, "16 threads, 16 slots a job");
+    for (int jr = 0; jr < (ROUNDS ? njobs : 1); jr += ROUNDS ? nw * JW : 1) {
+      // recomputed rather than kept in registers through the phases between
+      int tn = threadIdx.x;
+      asm volatile("" : "+v"(tn));
+      const int ln = tn & 63, lt = ln % T, job = jr + wv * JW + ln / T;
+      c2<R>* const wnj = nyq(jr, ln, lt);
+      if (is_wide(jr)) {
+        if (TW == 64 || ln < TW)
+          xline_fft<R, M, WV, XF, false>(v, sh + (njobs - 1) * MP, shw, ln, R(0), wnj, scale);
+      } else if (lact && job < njobs) {
+        c2<R>* const col = sh + job * MP;
+        if constexpr (TR) {
+          static_assert(T == 16 && kInSlots<M> == 16 && kOutSlots<M> == 16, "16 threads, 16 slots a job");
 #pragma unroll
-        for (int s = 0; s < 16; ++s) v[s] = col[lds_swz<XF>(rfft_in_idx<M>(t, s))];
-        rfft<R, M, false, 1, 0, XF, true>(v, t, true, col, shw, 2, 0, twr);
-        const int f = job / LINES, l = job - f * LINES;
-        c2<R>* dst = wmm + (long)f * g.hmain + (L0 + l) * M;
-        const R hs = R(0.5) * scale;
+          for (int s = 0; s < 16; ++s) v[s] = col[lds_swz<XF>(rfft_in_idx<M>(lt, s))];
+          rfft<R, M, false, 1, 0, XF, true>(v, lt, true, col, shw, 2, 0, twr);
+          const int f = job / LINES, l = job - f * LINES;
+          c2<R>* dst = wmm + (long)f * g.hmain + (L0 + l) * M;
+          const R hs = R(0.5) * scale;
 #pragma unroll
-        for (int s = 0; s < 16; ++s) {
-          const int k = rfft_out_idx<M>(t, s);  // t + 16 s
-          const c2<R> src = v[15 - s];
-          c2<R> pr = mk<R>(dpp_partner16(src.x), dpp_partner16(src.y));
-          if (t == 0) pr = v[(16 - s) % 16];
-          st_nt<R>(dst + k, r2c_post<R>(v[s], pr, shw[k], hs));
+          for (int s = 0; s < 16; ++s) {
+            const int k = rfft_out_idx<M>(lt, s);  // t + 16 s
+            const c2<R> src = v[15 - s];
+            c2<R> pr = mk<R>(dpp_partner16(src.x), dpp_partner16(src.y));
+            if (lt == 0) pr = v[(16 - s) % 16];
+            const c2<R> x = r2c_post<R>(v[s], pr, shw[k], hs);
+            if constexpr (KEEP) dst[k] = x;
+            else st_nt<R>(dst + k, x);
+          }
+          if (lt == 0) *wnj = mk<R>((v[0].x - v[0].y) * scale, R(0));
+        } else {
+          xline_fft<R, M, XV, XF, false, TR>(v, col, shw, lt, R(0), wnj, scale, twr);
         }
-        if (t == 0) wnn[(long)f * g.plane + L0 + l] = mk<R>((v[0].x - v[0].y) * scale, R(0));
-      } else {
-        xline_fft<R, M, 0, XF, false, TR>(v, col, shw, t, twr);
       }
     }
     __syncthreads();
-    // 6. R2C post-processing and store, one row per wave: coalesced along k, or
-    //    with the pairs (p, M - p) of 1 per lane, along k and M - k (with TR only
+    // 6. R2C post-processing and store, the row groups and pairs of 1 (with TR only
     //    the wide job's row)
     const R hs = R(0.5) * scale;
-    for (int jb = wv; jb < njobs; jb += nw) {
-      if (TR && !(wide_any && jb == njobs - 1)) continue;
-      const int f = jb / LINES, l = jb - f * LINES;
+#pragma unroll
+    for (int i = 0; i < PPL; ++i) w[i] = shw[p0 + 64 * i];
+    for (int j = wv; j < npieces; j += nw) {
+      if (TR && !(wide_any && j == njobs - 1)) continue;
+      const int f = j / (LINES / RP), l = (j - f * (LINES / RP)) * RP;
       c2<R>* dst = wmm + (long)f * g.hmain + (L0 + l) * M;
-      const c2<R>* rw = sh + jb * MP;
-      if constexpr (PP) {
+      const c2<R>* rw = sh + (j * RP + sub) * MP;
+      if (!mine) continue;
 #pragma unroll
-        for (int j = 0; j < PPL; ++j) {
-          const int p = lane + 64 * j;
-          if ((M / 2) % 64 == 0 || p < M / 2) {
-            const int q = xline_partner<M>(p);
-            const c2<R> a = rw[lds_swz<XF>(p)], b = rw[lds_swz<XF>(q)], w = shw[p];
-            st_nt<R>(dst + p, r2c_post<R>(a, p ? b : a, w, hs));
-            st_nt<R>(dst + q, r2c_post<R>(b, p ? a : b, xline_mirror_tw<R>(w, p), hs));
-          }
-        }
-      } else {
-#pragma unroll
-        for (int kk = 0; kk < KPL; ++kk) {
-          const int k = lane + 64 * kk;
-          if (M % 64 == 0 || k < M)
-            st_nt<R>(dst + k, r2c_post<R>(rw[lds_swz<XF>(k)], rw[lds_swz<XF>((M - k) % M)], shw[k], hs));
+      for (int i = 0; i < PPL; ++i) {
+        const int p = p0 + 64 * i, q = xline_partner<M>(p);
+        c2<R> a = rw[lds_swz<XF>(p)], b = rw[lds_swz<XF>(q)];
+        xline_r2c_pair<R>(a, b, w[i], p == 0, hs);
+        if constexpr (KEEP) {
+          dst[sub * M + p] = a;
+          dst[sub * M + q] = b;
+        } else {
+          st_nt<R>(dst + (sub * M + p), a);
+          st_nt<R>(dst + (sub * M + q), b);
         }
       }
-    }
-    for (int i = tid; i < njobs; i += nt) {
-      if (TR && !(wide_any && i == njobs - 1)) continue;
-      const int f = i / LINES, l = i - f * LINES;
-      const c2<R> z0 = sh[i * MP];
-      wnn[(long)f * g.plane + L0 + l] = mk<R>((z0.x - z0.y) * scale, R(0));
     }
     __syncthreads();
   }
-  const int tid = threadIdx.x;
   if (!XONLY && diag) {
-    const double s0 = bsum(a_ch, red), s1 = bsum(a_eta, red);
-    const double e0 = bext<true>((double)cmax, red), e1 = bext<false>((double)cmin, red);
-    const double e2 = bext<false>((double)pmin, red), e3 = bext<true>((double)p3, red);
-    if (tid == 0) {
-      double* o = part + (long)blockIdx.x * 6;
-      o[0] = s0; o[1] = s1; o[2] = e0; o[3] = e1; o[4] = e2; o[5] = e3;
-    }
+    diag_partials(a_ch, a_eta, (double)cmax, (double)cmin, (double)pmin, (double)p3, reinterpret_cast<double*>(smem),
+                  nw, part);
   }
 }
 
@@ -682,10 +661,13 @@ __device__ __forceinline__ ZCo zco(const UPar& u) {
   return ZCo{(u.D * u.dt) * u.kc, u.D * u.dt, (u.L * u.kphi) * u.dt, u.L * u.dt, u.dt, u.kc, u.kphi};
 }
 
+// KEEP: cache policy (bank_stays): 0 = every bank streamed, 1 = W (and X, Y) stays,
+// S streamed, 2 = both stay.  A template parameter: with the accesses of both
+// policies behind a uniform branch the kernel spilled.
 // BATCH (ROLE_REG only): the fields f0 .. f0 + nf - 1 run over every member in
 // mt, g.F per member, each with its own S, W, k = 0 modes and parameters; S, W
 // and dc64 are unused.
-template <typename R, int NZ, int ROLE, bool DC64, bool PARSEVAL, bool BATCH = false, int V = 0>
+template <typename R, int NZ, int ROLE, bool DC64, bool PARSEVAL, bool BATCH = false, int V = 0, int KEEP = 0>
 __global__ void __launch_bounds__(col_tile(NZ, sizeof(c2<R>)) * plan_T(NZ, V))
 __attribute__((amdgpu_waves_per_eu(kZlineWavesN<R, NZ, V, PARSEVAL>)))
 k_zline(Geo g, UPar u, KTab kt, Bank<R> S, Bank<R> W, Bank<R> X, Bank<R> Y,
@@ -695,6 +677,7 @@ k_zline(Geo g, UPar u, KTab kt, Bank<R> S, Bank<R> W, Bank<R> X, Bank<R> Y,
   constexpr int TX = col_tile(NZ, sizeof(c2<R>));
   constexpr int NI = kInSlots<NZ, V>, NO = kOutSlots<NZ, V>, E = plan_E(NZ, V);
   constexpr unsigned CB = sizeof(c2<R>);
+  constexpr int AUXW = KEEP ? 0 : kBufNT, AUXS = KEEP == 2 ? 0 : kBufNT;
   static_assert(last_pass_in_place<NZ, V>(), "slot rows of the last pass are t + a per-slot constant");
   // the exchange tile (up to 64 KiB), which after the tile loop holds the
   // block reduction's 16 doubles
@@ -745,11 +728,11 @@ k_zline(Geo g, UPar u, KTab kt, Bank<R> S, Bank<R> W, Bank<R> X, Bank<R> Y,
 #pragma unroll
     for (int s = 0; s < NI; ++s)
       if (act && rfft_in_valid<NZ, V>(t, s))
-        v[s] = buf_ld<R>((ROLE == ROLE_CMOB) ? ry : rw, lw, (unsigned)rfft_in_idx<NZ, V>(0, s) * rowb);
+        v[s] = buf_ld<R, AUXW>((ROLE == ROLE_CMOB) ? ry : rw, lw, (unsigned)rfft_in_idx<NZ, V>(0, s) * rowb);
 #pragma unroll
     for (int s = 0; s < NO; ++s)
       if (act && rfft_out_valid<NZ, V>(t, s)) {
-        sv[s] = buf_ld<R>(rs, ls, (unsigned)(rfft_out_idx<NZ, V>(0, s) * TX) * CB);
+        sv[s] = buf_ld<R, AUXS>(rs, ls, (unsigned)(rfft_out_idx<NZ, V>(0, s) * TX) * CB);
         if constexpr (ROLE == ROLE_CMOB) xv[s] = buf_ld<R, 0>(rx, lw, (unsigned)rfft_out_idx<NZ, V>(0, s) * rowb);
       }
     const long col = col0 + c;
@@ -823,7 +806,6 @@ k_zline(Geo g, UPar u, KTab kt, Bank<R> S, Bank<R> W, Bank<R> X, Bank<R> Y,
       for (int s = 0; s < NO; ++s) {
         if (!(act && rfft_out_valid<NZ, V>(t, s))) continue;
         const R m2 = v[s].x * v[s].x + v[s].y * v[s].y;
-        const int e = rfft_out_idx<NZ, V>(t, s);
         const int ez = rfft_out_idx<NZ, V>(tz, s);
         const R zp = (2 * ez == NZ) ? R(0) : (R)az_of(ez, NZ, kt.uz);  // a'_z: a_z zeroed at Nyquist
         pa1 += m2;
@@ -847,7 +829,7 @@ k_zline(Geo g, UPar u, KTab kt, Bank<R> S, Bank<R> W, Bank<R> X, Bank<R> Y,
 #pragma unroll
     for (int s = 0; s < NO; ++s)
       if (act && rfft_out_valid<NZ, V>(t, s))
-        buf_st<R>((ROLE == ROLE_GHAT) ? ry : rw, lw, (unsigned)rfft_out_idx<NZ, V>(0, s) * rowb, v[s]);
+        buf_st<R, AUXW>((ROLE == ROLE_GHAT) ? ry : rw, lw, (unsigned)rfft_out_idx<NZ, V>(0, s) * rowb, v[s]);
     __syncthreads();
   }
   if (PARSEVAL) {

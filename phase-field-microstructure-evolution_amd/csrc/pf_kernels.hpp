@@ -123,9 +123,17 @@ k_x_r2c(const c2<R>* src, c2<R>* dst, c2<R>* __restrict__ nyq, long nlines,
   const c2<R>* gs = src + l0 * M;
   c2<R>* g = dst + l0 * M;
   c2<R> v[E];
+  // bank_stays: an in-place pass also finds its input in cache
+  const bool keep = bank_stays((unsigned long)nlines * M * sizeof(c2<R>));
+  if (keep && src == dst) {
 #pragma unroll
-  for (int s = 0; s < kInSlots<M>; ++s)
-    if (act && rfft_in_valid<M>(t, s)) v[s] = ld_nt<R>(gs + (long)l * M + rfft_in_idx<M>(t, s));
+    for (int s = 0; s < kInSlots<M>; ++s)
+      if (act && rfft_in_valid<M>(t, s)) v[s] = gs[(long)l * M + rfft_in_idx<M>(t, s)];
+  } else {
+#pragma unroll
+    for (int s = 0; s < kInSlots<M>; ++s)
+      if (act && rfft_in_valid<M>(t, s)) v[s] = ld_nt<R>(gs + (long)l * M + rfft_in_idx<M>(t, s));
+  }
   c2<R>* line = sh + l * M;
   rfft<R, M, false, 1>(v, t, act, line, tw, 2);
   __syncthreads();
@@ -137,7 +145,9 @@ k_x_r2c(const c2<R>* src, c2<R>* dst, c2<R>* __restrict__ nyq, long nlines,
   for (int i = threadIdx.x; i < nl * M; i += NT) {
     const int ll = i / M, k = i - ll * M;
     const c2<R>* z = sh + ll * M;
-    st_nt<R>(g + i, r2c_post<R>(z[k], z[(M - k) % M], tw[k], hs));
+    const c2<R> x = r2c_post<R>(z[k], z[(M - k) % M], tw[k], hs);
+    if (keep) g[i] = x;
+    else st_nt<R>(g + i, x);
   }
   if (threadIdx.x < nl) {
     const c2<R> z0 = sh[threadIdx.x * M];
@@ -176,9 +186,16 @@ k_x_c2r(const c2<R>* src, c2<R>* dst, const c2<R>* __restrict__ nyq, long nlines
     }
   }
   rfft<R, M, true, 1>(v, t, act, sh + ((plan_np(M) > 1) ? l * M : 0), tw, 2);
+  // an in-place pass over a bank that stays in cache (bank_stays) leaves it there
+  if (src == dst && bank_stays((unsigned long)nlines * M * sizeof(c2<R>))) {
 #pragma unroll
-  for (int s = 0; s < kOutSlots<M>; ++s)
-    if (act && rfft_out_valid<M>(t, s)) st_nt<R>(gd + rfft_out_idx<M>(t, s), v[s]);
+    for (int s = 0; s < kOutSlots<M>; ++s)
+      if (act && rfft_out_valid<M>(t, s)) gd[rfft_out_idx<M>(t, s)] = v[s];
+  } else {
+#pragma unroll
+    for (int s = 0; s < kOutSlots<M>; ++s)
+      if (act && rfft_out_valid<M>(t, s)) st_nt<R>(gd + rfft_out_idx<M>(t, s), v[s]);
+  }
 }
 
 }  // namespace pf

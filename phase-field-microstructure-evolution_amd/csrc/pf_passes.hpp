@@ -21,12 +21,16 @@ namespace pf {
 //                   TX, or no multiple of it, carry no padding columns
 //   Nyquist planes: columns are the lines, NY contiguous elements each.
 // A wave's lanes run along whichever of the two is contiguous.  The Nyquist tiles,
-// whose LDS exchanges run at a stride, come first, so that they end under the rest.
-// Accesses go through buffer descriptors (one lane offset, uniform row offsets).
+// whose LDS exchanges run at a stride, come first, so that they end under the rest
+// (ypass_grid blocks).
 // BATCH: the W banks of every member in mt, ppm panels (and Nyquist lines) per
 // member; main and nyq are unused.
 // ---------------------------------------------------------------------------
-template <typename R, int NY, bool INV, bool BATCH = false>
+// The grid: an eighth of each kind's tiles (rounded up) per XCD.
+inline unsigned ypass_grid(long tmain, long tnyq) { return (unsigned)(8 * ((tmain + 7) / 8 + (tnyq + 7) / 8)); }
+
+// KEEP: the bank stays in cache from pass to pass (bank_stays).
+template <typename R, int NY, bool INV, bool BATCH = false, bool KEEP = false>
 __global__ void __launch_bounds__(col_tile(NY, sizeof(c2<R>)) * plan_T(NY))
 k_ypass(c2<R>* __restrict__ main, c2<R>* __restrict__ nyq, long M, long npanels, long nlines,
         const c2<R>* __restrict__ tw, const Member<R>* __restrict__ mt, long ppm) {
@@ -37,9 +41,12 @@ k_ypass(c2<R>* __restrict__ main, c2<R>* __restrict__ nyq, long M, long npanels,
   const unsigned m = (unsigned)M, np = (unsigned)(BATCH ? ppm : npanels), nl = (unsigned)(BATCH ? ppm : nlines);
   const unsigned nmem = BATCH ? (unsigned)(npanels / ppm) : 1u;
   const unsigned tmain = (np * m + TX - 1) / TX, tnyq = (nl + TX - 1) / TX;  // tiles per member
-  unsigned b = (unsigned)xcd_block(blockIdx.x, gridDim.x);
-  const bool isn = b < tnyq * nmem;
-  if (!isn) b -= tnyq * nmem;
+  // XCD x (blocks x, x + 8, ...) takes every eighth Nyquist tile, then one
+  // contiguous range of main-block tiles (their 128-byte pieces of the same rows
+  // are read by one XCD at about the same time).
+  const unsigned x = blockIdx.x % 8, i = blockIdx.x / 8, nq = (tnyq * nmem + 7) / 8;
+  const bool isn = i < nq;
+  unsigned b = isn ? i * 8 + x : x * (gridDim.x / 8 - nq) + (i - nq);
   c2<R>* base = isn ? nyq : main;
   if constexpr (BATCH) {
     const unsigned mem = b / (isn ? tnyq : tmain);
@@ -67,15 +74,33 @@ k_ypass(c2<R>* __restrict__ main, c2<R>* __restrict__ nyq, long M, long npanels,
     es = CB;
     voff = (c * NY + t) * CB;
   }
+  // a bank that stays in cache: plain accesses through a buffer descriptor, lanes
+  // without a column out of its range; a streamed one: hinted accesses by pointer
+  // (256^3 x 17 FP32: 428 us by pointer, 438 us through the descriptor)
   const BufRes rb = buf_res(base, left < 0xFFFFFFF0ul ? (unsigned)left : 0xFFFFFFF0u);
+  c2<R>* const gp = reinterpret_cast<c2<R>*>(reinterpret_cast<char*>(base) + voff);
+  const unsigned ee = es / CB;
   c2<R> v[E];
+  if constexpr (KEEP) {
+    if (!act) voff = kBufOut;
 #pragma unroll
-  for (int s = 0; s < kInSlots<NY>; ++s)
-    if (act && rfft_in_valid<NY>(t, s)) v[s] = buf_ld<R>(rb, voff, (unsigned)rfft_in_idx<NY>(0, s) * es);
-  rfft<R, NY, INV, (int)TX>(v, t, act, sh + c, tw);
+    for (int s = 0; s < kInSlots<NY>; ++s)
+      if (rfft_in_valid<NY>(t, s)) v[s] = buf_ld<R, 0>(rb, voff, (unsigned)rfft_in_idx<NY>(0, s) * es);
+  } else {
 #pragma unroll
-  for (int s = 0; s < kOutSlots<NY>; ++s)
-    if (act && rfft_out_valid<NY>(t, s)) buf_st<R>(rb, voff, (unsigned)rfft_out_idx<NY>(0, s) * es, v[s]);
+    for (int s = 0; s < kInSlots<NY>; ++s)
+      if (act && rfft_in_valid<NY>(t, s)) v[s] = ld_nt<R>(gp + (unsigned long)rfft_in_idx<NY>(0, s) * ee);
+  }
+  rfft<R, NY, INV, (int)TX>(v, t, KEEP || act, sh + c, tw);
+  if constexpr (KEEP) {
+#pragma unroll
+    for (int s = 0; s < kOutSlots<NY>; ++s)
+      if (rfft_out_valid<NY>(t, s)) buf_st<R, 0>(rb, voff, (unsigned)rfft_out_idx<NY>(0, s) * es, v[s]);
+  } else {
+#pragma unroll
+    for (int s = 0; s < kOutSlots<NY>; ++s)
+      if (act && rfft_out_valid<NY>(t, s)) st_nt<R>(gp + (unsigned long)rfft_out_idx<NY>(0, s) * ee, v[s]);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -111,7 +136,7 @@ k_zpass(c2<R>* near, c2<R>* nearn, c2<R>* far, c2<R>* farn, unsigned M, unsigned
   const unsigned long fmain = (unsigned long)f * M * ny * NZ, fplane = (unsigned long)f * ny * NZ;
   const unsigned nrow = W * CB;
   const BufRes rn = buf_res((isn ? nearn + fplane : near + fmain) + col0, (unsigned)NZ * nrow);
-  const unsigned noff = (t * W + c) * CB;
+  const unsigned noff = act ? (t * W + c) * CB : kBufOut;
   unsigned foff, frow;
   BufRes rf = rn;
   if constexpr (FAR == FAR_SPLIT) {
@@ -121,33 +146,50 @@ k_zpass(c2<R>* near, c2<R>* nearn, c2<R>* far, c2<R>* farn, unsigned M, unsigned
   } else if constexpr (FAR == FAR_TILED) {
     rf = buf_res(far + ((unsigned long)f * tpf + tt) * (NZ * TX), NZ * TX * CB);
     frow = TX * CB;
-    foff = threadIdx.x * CB;
+    foff = act ? threadIdx.x * CB : kBufOut;
   } else {
     const unsigned long half = fmain + fplane;
     const unsigned col = act ? col0 + c : 0u;
     const unsigned ky = isn ? col : col / M, kx = isn ? M : col - ky * M;
     rf = buf_res(far + half, (M + 1) * ny * NZ * CB);
     frow = (FAR == FAR_XFAST ? ny * (M + 1) : 1u) * CB;
-    foff = (FAR == FAR_XFAST ? ky * (M + 1) + kx : (kx * ny + ky) * NZ) * CB + t * frow;
+    foff = act ? (FAR == FAR_XFAST ? ky * (M + 1) + kx : (kx * ny + ky) * NZ) * CB + t * frow : kBufOut;
   }
-  // dense layouts: rows are no whole cache lines, so neighbouring tiles (XFAST)
-  // or slots (ZFAST) share lines and the accesses keep them in L2
+  // near: the scratch bank (or the bank itself), by bank_stays; far: dense layouts
+  // have rows of no whole cache lines, neighbouring tiles (XFAST) or slots (ZFAST)
+  // share lines and the accesses keep them in L2; the carried spectrum's tiles are
+  // streamed
+  const bool keep = bank_stays((unsigned long)nf * M * ny * NZ * CB);
   constexpr int AUXF = (FAR == FAR_XFAST || FAR == FAR_ZFAST) ? 0 : kBufNT;
+  constexpr bool NEARIN = !INV, NEAROUT = INV || FAR == FAR_SPLIT;
   c2<R> v[E];
+  if (NEARIN && keep) {
 #pragma unroll
-  for (int s = 0; s < kInSlots<NZ>; ++s)
-    if (act && rfft_in_valid<NZ>(t, s)) {
-      const unsigned i = (unsigned)rfft_in_idx<NZ>(0, s);
-      v[s] = INV ? buf_ld<R, AUXF>(rf, foff, i * frow) : buf_ld<R>(rn, noff, i * nrow);
-    }
-  rfft<R, NZ, INV, (int)TX>(v, t, act, sh + c, tw);
+    for (int s = 0; s < kInSlots<NZ>; ++s)
+      if (rfft_in_valid<NZ>(t, s)) v[s] = buf_ld<R, 0>(rn, noff, (unsigned)rfft_in_idx<NZ>(0, s) * nrow);
+  } else {
 #pragma unroll
-  for (int s = 0; s < kOutSlots<NZ>; ++s)
-    if (act && rfft_out_valid<NZ>(t, s)) {
-      const unsigned i = (unsigned)rfft_out_idx<NZ>(0, s);
-      if (INV) buf_st<R>(rn, noff, i * nrow, v[s]);
-      else buf_st<R, AUXF>(rf, foff, i * frow, v[s]);
-    }
+    for (int s = 0; s < kInSlots<NZ>; ++s)
+      if (rfft_in_valid<NZ>(t, s)) {
+        const unsigned i = (unsigned)rfft_in_idx<NZ>(0, s);
+        v[s] = NEARIN ? buf_ld<R>(rn, noff, i * nrow) : buf_ld<R, AUXF>(rf, foff, i * frow);
+      }
+  }
+  rfft<R, NZ, INV, (int)TX>(v, t, true, sh + c, tw);
+  if (NEAROUT && keep) {
+#pragma unroll
+    for (int s = 0; s < kOutSlots<NZ>; ++s)
+      if (rfft_out_valid<NZ>(t, s))
+        buf_st<R, 0>(INV ? rn : rf, INV ? noff : foff, (unsigned)rfft_out_idx<NZ>(0, s) * (INV ? nrow : frow), v[s]);
+  } else {
+#pragma unroll
+    for (int s = 0; s < kOutSlots<NZ>; ++s)
+      if (rfft_out_valid<NZ>(t, s)) {
+        const unsigned i = (unsigned)rfft_out_idx<NZ>(0, s);
+        if (INV) buf_st<R>(rn, noff, i * nrow, v[s]);
+        else buf_st<R, AUXF>(rf, foff, i * frow, v[s]);
+      }
+  }
 }
 
 }  // namespace pf

@@ -15,6 +15,7 @@
 #include "pf_internal.hpp"
 #include "pf_faithful.hpp"
 #include "pf_fused.hpp"
+#include "pf_launch.hpp"
 
 namespace pf {
 double kaxis(int m, int n, bool zero_nyquist);
@@ -29,11 +30,6 @@ static const char* kStageNames[NSTAGE] = {
 
 constexpr int NB = 256;        // block size of pointwise kernels
 constexpr int NPART_NL = 6;    // f_ch, f_eta, c_max, c_min, phi_min, phi_3
-constexpr long kMaxGrid = 8192;
-// The z-line kernel streams four banks with short (TX-column) row segments;
-// more resident tiles per CU keep more rows in flight (measured 2.5% faster
-// at 32768 than at 8192 blocks, 256^3 x 17 fields).
-constexpr long kZlineMaxGrid = 32768;
 // Largest grids a tuning may ask for (the block-partial buffers are sized for them).
 constexpr long kXlineGridCap = 16384;
 constexpr long kZlineGridCap = 65536;
@@ -489,154 +485,6 @@ int ensure_diag(pf_handle* h, long n) {
 #define PF_GRID_SIZES(X) \
   X(8) X(12) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(160) X(192) X(256) X(512)
 
-// Lines per x-line block: the smallest of 1, 2, 4, 8 that gives the block's
-// transforms at least two waves of work (F*LINES*T >= 128 threads).  Small
-// blocks keep several of them resident per CU, which is what hides the
-// latency of each block's staging and barriers: at 256^3 x 17 fields one
-// line per block (3 waves, 19 KB of LDS) runs 1.6x faster than two.
-constexpr int kXlineMinThreads = 128;
-// LDS one x-line block may take (gfx950: 160 KiB per workgroup); above 64 KiB
-// the kernel is opted in with hipFuncAttributeMaxDynamicSharedMemorySize.
-constexpr size_t kXlineMaxLds = 160 * 1024;
-
-template <typename R, int NX, int LINES, bool XONLY>
-bool xline_fits(const Geo& g, long* nt_out, size_t* shb_out) {
-  constexpr int M = NX / 2, T = plan_T(M);
-  const int F = XONLY ? 1 : g.F;
-  if (g.plane % LINES) return false;
-  const long jobs = (long)F * LINES;
-  const long MP = xline_row_pitch(M, sizeof(c2<R>));
-  long need = std::max<long>(64, (jobs * T + 63) / 64 * 64);
-  const size_t body = sizeof(c2<R>) * ((size_t)xline_rows(M, (int)jobs) * MP + NX) +
-                      (xline_pair_rows(M) ? 0 : sizeof(R) * (size_t)(jobs + 1));
-  const size_t shb = ((body + 15) & ~(size_t)15) + 16 * sizeof(double);
-  if (need > kXlineMaxThreadsN<R, NX> || shb > kXlineMaxLds) return false;
-  *nt_out = need;
-  *shb_out = shb;
-  return true;
-}
-
-template <typename R, int NX, int LINES, bool XONLY>
-int launch_xline_n(pf_handle* h, c2<R>* wm, c2<R>* wn, R* mobd, double* part, long* grid_out, bool diag,
-                   bool mob, long nt, size_t shb) {
-  const Geo& g = h->g;
-  const long ngroups = g.plane / LINES;
-  const long cap = (!XONLY && h->tune.xline_grid > 0) ? h->tune.xline_grid : kMaxGrid;
-  long grid = std::min<long>(ngroups, cap);
-  if (grid >= 8) grid -= grid % 8;
-  const c2<R>* tw = twiddle_table<R>(NX);
-  if (!tw) return fail(PF_EHIP, "twiddle table set-up failed");
-  if (shb > 65536 &&
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&k_xline<R, NX, LINES, XONLY>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)shb) != hipSuccess)
-    return fail(PF_EHIP, "x-line kernel: " + std::to_string(shb) + " bytes of LDS refused");
-  hipLaunchKernelGGL((k_xline<R, NX, LINES, XONLY>), dim3((unsigned)grid), dim3((unsigned)nt), shb, h->s, g, h->u,
-                     wm, wn, mobd, tw, part, ngroups, (int)diag, (int)mob, (const Member<R>*)nullptr);
-  if (grid_out) *grid_out = grid;
-  return 0;
-}
-
-template <typename R, bool XONLY>
-int launch_xline(pf_handle* h, c2<R>* wm, c2<R>* wn, R* mobd, double* part, long* grid_out, bool diag,
-                 bool mob) {
-  long nt = 0;
-  size_t shb = 0;
-  const long F = XONLY ? 1 : h->g.F;
-  switch (h->g.nx) {
-#define PF_TRY(N, L)                                                                                     \
-  if (xline_fits<R, N, L, XONLY>(h->g, &nt, &shb))                                                       \
-    return launch_xline_n<R, N, L, XONLY>(h, wm, wn, mobd, part, grid_out, diag, mob, nt, shb);
-#define PF_CASE(N)                                                                                       \
-  case N: {                                                                                              \
-    const long T = plan_T(N / 2);                                                                        \
-    int want = 1;                                                                                        \
-    while (want < 8 && F * want * T < kXlineMinThreads) want *= 2;                                       \
-    const int tl = XONLY ? 0 : h->tune.xline_lines;                                                      \
-    if (tl > 0) want = tl;                                                                               \
-    if (want >= 8) { PF_TRY(N, 8) }                                                                      \
-    if (want >= 4 && want < 8) { PF_TRY(N, 4) }                                                          \
-    if (want >= 2 && want < 4) { PF_TRY(N, 2) }                                                          \
-    if (tl == 0 || want == 1) { PF_TRY(N, 1) }                                                           \
-    return fail(PF_ENOTIMPL, "x-line kernel: " + std::to_string(F) + " fields of length " #N " in " +    \
-                                 std::to_string(want) + "-line blocks exceed one block's threads or LDS"); \
-  }
-    PF_GRID_SIZES(PF_CASE)
-#undef PF_CASE
-#undef PF_TRY
-    default: return fail(PF_EINVAL, "unsupported nx");
-  }
-}
-
-// Whether some x-line block shape fits this grid (checked at pf_create, so
-// that an unsupported combination fails there rather than at the first step).
-template <typename R, bool XONLY>
-bool xline_supported(const Geo& g) {
-  long nt = 0;
-  size_t shb = 0;
-  switch (g.nx) {
-#define PF_CASE(N)                                                                                 \
-  case N:                                                                                          \
-    return xline_fits<R, N, 8, XONLY>(g, &nt, &shb) || xline_fits<R, N, 4, XONLY>(g, &nt, &shb) ||   \
-           xline_fits<R, N, 2, XONLY>(g, &nt, &shb) || xline_fits<R, N, 1, XONLY>(g, &nt, &shb);
-    PF_GRID_SIZES(PF_CASE)
-#undef PF_CASE
-    default: return false;
-  }
-}
-
-// The z-line's plan variant: the tuned one for the FP32 update of every field
-// (ROLE_REG), the default for FP64 and for the mobility chain's roles.
-template <typename R, int ROLE> int zline_plan_of(const pf_handle* h, int n) {
-  if (sizeof(R) != 4 || ROLE != ROLE_REG || h->tune.zline_plan <= 0) return 0;
-  return plan_alt(n, h->tune.zline_plan, 0) != 0 ? h->tune.zline_plan : 0;
-}
-
-template <typename R, int ROLE, bool DC64, bool PARSEVAL>
-int launch_zline(pf_handle* h, Bank<R> S, Bank<R> W, Bank<R> X, Bank<R> Y, double* part, int f0, int nf,
-                 long* grid_out) {
-  const Geo& g = h->g;
-  switch (g.nz) {
-#define PF_CASE(N)                                                                                   \
-  case N: {                                                                                          \
-    constexpr int TX = col_tile(N, sizeof(c2<R>));                                                 \
-    const long tm = ((long)g.M * g.ny + TX - 1) / TX, tn = ((long)g.ny + TX - 1) / TX;               \
-    const long cap = h->tune.zline_grid > 0 ? h->tune.zline_grid : kZlineMaxGrid;                    \
-    long grid = std::min<long>((tm + tn) * nf, cap);                                                 \
-    /* whole XCD runs of main-block rows (xcd_runs): extra blocks find no tile */                    \
-    const long rows = h->tune.zline_run_rows < 0 ? 1 : h->tune.zline_run_rows;                      \
-    const long runt = rows * (((long)g.M + TX - 1) / TX), run = 8 * runt;                           \
-    if (run > 0 && (grid + run - 1) / run * run <= cap) grid = (grid + run - 1) / run * run;        \
-    const c2<R>* tw = twiddle_table<R>(N);                                                           \
-    if (!tw) return fail(PF_EHIP, "twiddle table set-up failed");                                    \
-    const int plan = zline_plan_of<R, ROLE>(h, N);                                                   \
-    if constexpr (sizeof(R) == 4 && ROLE == ROLE_REG && plan_alt(N, 1, 0) != 0) {                    \
-      if (plan == 1) {                                                                               \
-        hipLaunchKernelGGL((k_zline<R, N, ROLE, DC64, PARSEVAL, false, 1>), dim3((unsigned)grid),    \
-                           dim3(TX * plan_T(N, 1)), 0, h->s, g, h->u, h->kt, S, W, X, Y, h->dc64, part, \
-                           tw, f0, nf, tm, tn, runt, (const Member<R>*)nullptr);                     \
-        if (grid_out) *grid_out = grid;                                                              \
-        return 0;                                                                                    \
-      }                                                                                              \
-      if (plan == 2) {                                                                               \
-        hipLaunchKernelGGL((k_zline<R, N, ROLE, DC64, PARSEVAL, false, 2>), dim3((unsigned)grid),    \
-                           dim3(TX * plan_T(N, 2)), 0, h->s, g, h->u, h->kt, S, W, X, Y, h->dc64, part, \
-                           tw, f0, nf, tm, tn, runt, (const Member<R>*)nullptr);                     \
-        if (grid_out) *grid_out = grid;                                                              \
-        return 0;                                                                                    \
-      }                                                                                              \
-    }                                                                                                \
-    hipLaunchKernelGGL((k_zline<R, N, ROLE, DC64, PARSEVAL>), dim3((unsigned)grid),                  \
-                       dim3(TX * plan_T(N)), 0, h->s, g, h->u, h->kt, S, W, X, Y, h->dc64, part, tw,      \
-                       f0, nf, tm, tn, runt, (const Member<R>*)nullptr);                             \
-    if (grid_out) *grid_out = grid;                                                                  \
-    return 0;                                                                                        \
-  }
-    PF_GRID_SIZES(PF_CASE)
-#undef PF_CASE
-    default: return fail(PF_EINVAL, "unsupported nz");
-  }
-}
-
 // ---------------------------------------------------------------------------
 // Batched ensemble: one launch per stage over every member of a group (same
 // grid and var, FP32-mixed form, constant mobility), each member's banks and
@@ -644,107 +492,26 @@ int launch_zline(pf_handle* h, Bank<R> S, Bank<R> W, Bank<R> X, Bank<R> Y, doubl
 // arithmetic are those of a single member's step, so each member's result is
 // bit-identical to stepping it alone.
 // ---------------------------------------------------------------------------
-int xline_batch(const Geo& g, const UPar& u, const pf_tuning& tn, const Member<float>* mt, long nmem,
-                hipStream_t s) {
-  long nt = 0;
-  size_t shb = 0;
-  const long cap = tn.xline_grid > 0 ? tn.xline_grid : kMaxGrid;
-  switch (g.nx) {
-#define PF_TRY(N, L)                                                                                   \
-  if (xline_fits<float, N, L, false>(g, &nt, &shb)) {                                                  \
-    const long ngroups = nmem * (g.plane / L);                                                         \
-    long grid = std::min<long>(ngroups, cap);                                                          \
-    if (grid >= 8) grid -= grid % 8;                                                                   \
-    const c2<float>* tw = twiddle_table<float>(N);                                                     \
-    if (!tw) return fail(PF_EHIP, "twiddle table set-up failed");                                      \
-    if (shb > 65536 &&                                                                                 \
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&k_xline<float, N, L, false, true>),         \
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)shb) != hipSuccess)       \
-      return fail(PF_EHIP, "x-line kernel: " + std::to_string(shb) + " bytes of LDS refused");         \
-    hipLaunchKernelGGL((k_xline<float, N, L, false, true>), dim3((unsigned)grid), dim3((unsigned)nt), shb, \
-                       s, g, u, (c2<float>*)nullptr, (c2<float>*)nullptr, (float*)nullptr, tw,         \
-                       (double*)nullptr, ngroups, 0, 0, mt);                                            \
-    return 0;                                                                                          \
-  }
-#define PF_CASE(N)                                                                                     \
-  case N: {                                                                                            \
-    const long T = plan_T(N / 2);                                                                      \
-    int want = 1;                                                                                      \
-    while (want < 8 && g.F * want * T < kXlineMinThreads) want *= 2;                                   \
-    if (tn.xline_lines > 0) want = tn.xline_lines;                                                     \
-    if (want >= 8) { PF_TRY(N, 8) }                                                                    \
-    if (want >= 4 && want < 8) { PF_TRY(N, 4) }                                                        \
-    if (want >= 2 && want < 4) { PF_TRY(N, 2) }                                                        \
-    if (tn.xline_lines == 0 || want == 1) { PF_TRY(N, 1) }                                             \
-    return fail(PF_ENOTIMPL, "x-line kernel: " + std::to_string(g.F) +                                \
-                                 " fields of length " #N " exceed one block's threads or LDS");        \
-  }
-    PF_GRID_SIZES(PF_CASE)
-#undef PF_CASE
-#undef PF_TRY
-    default: return fail(PF_EINVAL, "unsupported nx");
-  }
-}
-
 template <bool INV> int ypass_batch(const Geo& g, const Member<float>* mt, long nmem, hipStream_t s) {
   switch (g.ny) {
 #define PF_CASE(N)                                                                                    \
   case N: {                                                                                           \
     constexpr int TX = col_tile(N, sizeof(c2<float>));                                                \
     const long ppm = (long)g.nz * g.F, npanels = nmem * ppm, nlines = npanels;                        \
-    const long tiles = nmem * ((ppm * g.M + TX - 1) / TX + (ppm + TX - 1) / TX);                      \
-    const long grid = (tiles + 7) / 8 * 8;                                                            \
+    const long grid = ypass_grid(nmem * ((ppm * g.M + TX - 1) / TX), nmem * ((ppm + TX - 1) / TX));   \
     const c2<float>* tw = twiddle_table<float>(N);                                                    \
     if (!tw) return fail(PF_EHIP, "twiddle table set-up failed");                                     \
-    hipLaunchKernelGGL((k_ypass<float, N, INV, true>), dim3((unsigned)grid), dim3(TX * plan_T(N)), 0, s, \
-                       (c2<float>*)nullptr, (c2<float>*)nullptr, (long)g.M, npanels, nlines, tw, mt, ppm); \
+    if (bank_stays(sizeof(float) * (unsigned long)g.P * g.F * nmem))                                  \
+      hipLaunchKernelGGL((k_ypass<float, N, INV, true, true>), dim3((unsigned)grid), dim3(TX * plan_T(N)), 0, s, \
+                         (c2<float>*)nullptr, (c2<float>*)nullptr, (long)g.M, npanels, nlines, tw, mt, ppm); \
+    else                                                                                              \
+      hipLaunchKernelGGL((k_ypass<float, N, INV, true>), dim3((unsigned)grid), dim3(TX * plan_T(N)), 0, s, \
+                         (c2<float>*)nullptr, (c2<float>*)nullptr, (long)g.M, npanels, nlines, tw, mt, ppm); \
     return 0;                                                                                         \
   }
     PF_GRID_SIZES(PF_CASE)
 #undef PF_CASE
     default: return fail(PF_EINVAL, "unsupported ny");
-  }
-}
-
-int zline_batch(const Geo& g, const UPar& u, const pf_tuning& tun, const KTab& kt, const Member<float>* mt,
-                long nmem, hipStream_t s) {
-  const Bank<float> none{nullptr, nullptr};
-  const long cap = tun.zline_grid > 0 ? tun.zline_grid : kZlineMaxGrid;
-  const long rows = tun.zline_run_rows < 0 ? 1 : tun.zline_run_rows;
-  switch (g.nz) {
-#define PF_CASE(N)                                                                                   \
-  case N: {                                                                                          \
-    constexpr int TX = col_tile(N, sizeof(c2<float>));                                             \
-    const long tm = ((long)g.M * g.ny + TX - 1) / TX, tn = ((long)g.ny + TX - 1) / TX;               \
-    const long nf = nmem * g.F;                                                                      \
-    long grid = std::min<long>((tm + tn) * nf, cap);                                                 \
-    const long runt = rows * (((long)g.M + TX - 1) / TX), run = 8 * runt;                            \
-    if (run > 0 && (grid + run - 1) / run * run <= cap) grid = (grid + run - 1) / run * run;        \
-    const c2<float>* tw = twiddle_table<float>(N);                                                   \
-    if (!tw) return fail(PF_EHIP, "twiddle table set-up failed");                                    \
-    const int plan = (tun.zline_plan > 0 && plan_alt(N, tun.zline_plan, 0) != 0) ? tun.zline_plan : 0; \
-    if constexpr (plan_alt(N, 1, 0) != 0) {                                                          \
-      if (plan == 1) {                                                                               \
-        hipLaunchKernelGGL((k_zline<float, N, ROLE_REG, true, false, true, 1>), dim3((unsigned)grid), \
-                           dim3(TX * plan_T(N, 1)), 0, s, g, u, kt, none, none, none, none,          \
-                           (double*)nullptr, (double*)nullptr, tw, 0, (int)nf, tm, tn, runt, mt);     \
-        return 0;                                                                                    \
-      }                                                                                              \
-      if (plan == 2) {                                                                               \
-        hipLaunchKernelGGL((k_zline<float, N, ROLE_REG, true, false, true, 2>), dim3((unsigned)grid), \
-                           dim3(TX * plan_T(N, 2)), 0, s, g, u, kt, none, none, none, none,          \
-                           (double*)nullptr, (double*)nullptr, tw, 0, (int)nf, tm, tn, runt, mt);     \
-        return 0;                                                                                    \
-      }                                                                                              \
-    }                                                                                                \
-    hipLaunchKernelGGL((k_zline<float, N, ROLE_REG, true, false, true>), dim3((unsigned)grid),       \
-                       dim3(TX * plan_T(N)), 0, s, g, u, kt, none, none, none, none, (double*)nullptr, \
-                       (double*)nullptr, tw, 0, (int)nf, tm, tn, runt, mt);                          \
-    return 0;                                                                                        \
-  }
-    PF_GRID_SIZES(PF_CASE)
-#undef PF_CASE
-    default: return fail(PF_EINVAL, "unsupported nz");
   }
 }
 
@@ -757,6 +524,8 @@ int step_reduced(pf_handle* h, bool diag, long rec, bool fint_next) {
   Bank<R> S{(c2<R>*)h->S_main, nullptr}, W{(c2<R>*)h->W_main, (c2<R>*)h->W_nyq};
   Bank<R> G{(c2<R>*)h->G_main, (c2<R>*)h->G_nyq}, Fc{(c2<R>*)h->Fc_main, (c2<R>*)h->Fc_nyq};
   int rc;
+
+  const StepCall sc{g, h->u, h->kt, h->tune};
 
   if (diag && !h->fint_ready) {
     tbeg(h, ST_DIAG);
@@ -771,7 +540,7 @@ int step_reduced(pf_handle* h, bool diag, long rec, bool fint_next) {
   {
     long gr = 0;
     R* md = (R*)h->mob;
-    rc = launch_xline<R, false>(h, W.main, W.nyq, md, h->part_nl, &gr, diag, mob);
+    rc = xline<R>(false, sc, W.main, W.nyq, md, h->part_nl, &gr, diag, mob, s);
     if (rc) return rc;
     if (diag) h->n_part_nl = gr;
   }
@@ -787,24 +556,18 @@ int step_reduced(pf_handle* h, bool diag, long rec, bool fint_next) {
   tbeg(h, ST_UPDATE);
   long g1 = 0, g2 = 0;
   if (!mob) {
-    rc = fint_next ? launch_zline<R, ROLE_REG, DC, true>(h, S, W, W, W, h->part_fi, 0, g.F, &g1)
-                   : launch_zline<R, ROLE_REG, DC, false>(h, S, W, W, W, h->part_fi, 0, g.F, &g1);
-    if (rc) return rc;
+    if ((rc = zline<R>(ROLE_REG, fint_next, sc, S, W, W, W, h->dc64, h->part_fi, 0, g.F, &g1, s))) return rc;
   } else {
-    if ((rc = launch_zline<R, ROLE_GHAT, false, false>(h, S, W, Fc, G, h->part_fi, 0, 1, nullptr))) return rc;
-    rc = fint_next ? launch_zline<R, ROLE_REG, DC, true>(h, S, W, W, W, h->part_fi, 1, g.var, &g1)
-                   : launch_zline<R, ROLE_REG, DC, false>(h, S, W, W, W, h->part_fi, 1, g.var, &g1);
-    if (rc) return rc;
+    if ((rc = zline<R>(ROLE_GHAT, false, sc, S, W, Fc, G, h->dc64, h->part_fi, 0, 1, nullptr, s))) return rc;
+    if ((rc = zline<R>(ROLE_REG, fint_next, sc, S, W, W, W, h->dc64, h->part_fi, 1, g.var, &g1, s))) return rc;
     tend(h);
     tbeg(h, ST_MOBILITY);
     if ((rc = y_pass<R>(g.ny, true, G.main, G.nyq, g.M, g.nz, s))) return rc;
-    if ((rc = launch_xline<R, true>(h, G.main, G.nyq, (R*)h->mob, nullptr, nullptr, false, false))) return rc;
+    if ((rc = xline<R>(true, sc, G.main, G.nyq, (R*)h->mob, nullptr, nullptr, false, false, s))) return rc;
     if ((rc = y_pass<R>(g.ny, false, G.main, G.nyq, g.M, g.nz, s))) return rc;
     tend(h);
     tbeg(h, ST_UPDATE);
-    rc = fint_next ? launch_zline<R, ROLE_CMOB, DC, true>(h, S, W, Fc, G, h->part_fi + g1, 0, 1, &g2)
-                   : launch_zline<R, ROLE_CMOB, DC, false>(h, S, W, Fc, G, h->part_fi + g1, 0, 1, &g2);
-    if (rc) return rc;
+    if ((rc = zline<R>(ROLE_CMOB, fint_next, sc, S, W, Fc, G, h->dc64, h->part_fi + g1, 0, 1, &g2, s))) return rc;
   }
   if (fint_next) h->n_part_fi = g1 + g2;
   h->fint_ready = fint_next;
@@ -858,7 +621,8 @@ int step_faithful(pf_handle* h, bool diag, long rec) {
   // loops 11-12: g back in real space, times mob_c - D_mean, forward
   tbeg(h, ST_MOBILITY);
   if ((rc = y_pass<double>(g.ny, true, G.main, G.nyq, g.M, g.nz, s))) return rc;
-  if ((rc = launch_xline<double, true>(h, G.main, G.nyq, (double*)h->mob, nullptr, nullptr, false, false))) return rc;
+  if ((rc = xline<double>(true, StepCall{g, h->u, h->kt, h->tune}, G.main, G.nyq, (double*)h->mob, nullptr, nullptr, false,
+                          false, s))) return rc;
   if ((rc = y_pass<double>(g.ny, false, G.main, G.nyq, g.M, g.nz, s))) return rc;
   tend(h);
   // loop 13
@@ -982,32 +746,11 @@ const TunedShape kTuned[] = {
     {0, 0, 0, 0, -1, {0, 0, 0, -1, 0}},
 };
 
-// Whether the x-line can run blocks of `lines` lines for this handle.
-bool xline_lines_fit(const pf_handle* h, int lines) {
-  const Geo& g = h->g;
-  long nt = 0;
-  size_t shb = 0;
-  const bool f32 = h->mode == PF_MODE_FP32_MIXED;
-  switch (g.nx) {
-#define PF_CASE(N)                                                                                      \
-  case N:                                                                                               \
-    switch (lines) {                                                                                    \
-      case 1: return f32 ? xline_fits<float, N, 1, false>(g, &nt, &shb) : xline_fits<double, N, 1, false>(g, &nt, &shb); \
-      case 2: return f32 ? xline_fits<float, N, 2, false>(g, &nt, &shb) : xline_fits<double, N, 2, false>(g, &nt, &shb); \
-      case 4: return f32 ? xline_fits<float, N, 4, false>(g, &nt, &shb) : xline_fits<double, N, 4, false>(g, &nt, &shb); \
-      case 8: return f32 ? xline_fits<float, N, 8, false>(g, &nt, &shb) : xline_fits<double, N, 8, false>(g, &nt, &shb); \
-      default: return false;                                                                            \
-    }
-    PF_GRID_SIZES(PF_CASE)
-#undef PF_CASE
-    default: return false;
-  }
-}
-
 int check_tuning(const pf_handle* h, const pf_tuning& t) {
   if (!(t.xline_lines == 0 || t.xline_lines == 1 || t.xline_lines == 2 || t.xline_lines == 4 || t.xline_lines == 8))
     return fail(PF_EINVAL, "xline_lines must be 0, 1, 2, 4 or 8");
-  if (t.xline_lines > 0 && !xline_lines_fit(h, t.xline_lines))
+  if (t.xline_lines > 0 && !(h->mode == PF_MODE_FP32_MIXED ? xline_accepts<float>(h->g, t.xline_lines)
+                                                            : xline_accepts<double>(h->g, t.xline_lines)))
     return fail(PF_EINVAL, "x-line blocks of " + std::to_string(t.xline_lines) + " lines do not fit this grid");
   if (t.xline_grid != 0 && (t.xline_grid < 256 || t.xline_grid > kXlineGridCap))
     return fail(PF_EINVAL, "xline_grid must be 0 or in [256, " + std::to_string(kXlineGridCap) + "]");
@@ -1092,12 +835,12 @@ extern "C" int pf_create(const pf_params* p, int nx, int ny, int nz, int var, in
         (rc = dalloc(h, &h->mob, sizeof(double) * g.P)))
       return bail(rc);
   } else if (mode == PF_MODE_FP64_REDUCED) {
-    if (!xline_supported<double, false>(g))
+    if (!xline_accepts<double>(g, 0))
       return bail(fail(PF_ENOTIMPL, "FP64 reduced form: " + std::to_string(g.F) + " fields of " +
                                         std::to_string(nx) + "-point x lines exceed one block's threads or LDS"));
     if ((rc = alloc_reduced<double>(h))) return bail(rc);
   } else {
-    if (!xline_supported<float, false>(g))
+    if (!xline_accepts<float>(g, 0))
       return bail(fail(PF_ENOTIMPL, "FP32-mixed form: " + std::to_string(g.F) + " fields of " +
                                         std::to_string(nx) + "-point x lines exceed one block's threads or LDS"));
     if ((rc = alloc_reduced<float>(h))) return bail(rc);
@@ -1371,9 +1114,10 @@ int step_group(const Group& gr) {
   pf_handle* h0 = gr.mem[0];
   const Geo& g = h0->g;
   const long nmem = (long)gr.mem.size();
-  int rc = xline_batch(g, h0->u, h0->tune, gr.table, nmem, h0->s);
+  const StepCall call{g, h0->u, h0->kt, h0->tune};
+  int rc = xline_batch(call, gr.table, nmem, h0->s);
   if (!rc) rc = ypass_batch<false>(g, gr.table, nmem, h0->s);
-  if (!rc) rc = zline_batch(g, h0->u, h0->tune, h0->kt, gr.table, nmem, h0->s);
+  if (!rc) rc = zline_batch(call, gr.table, nmem, h0->s);
   if (!rc) rc = ypass_batch<true>(g, gr.table, nmem, h0->s);
   return rc;
 }

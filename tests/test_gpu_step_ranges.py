@@ -1,0 +1,85 @@
+"""The step kernels where their choices by size change, on the GPU.
+
+  * Fields beyond what one round of an x-line block's waves takes: the smallest
+    such count and the largest accepted one, against the oracle.
+  * Spectra below, within and above the sizes that stay in the last-level cache
+    (24 to 256 MiB): one member and a batch of equal ones take different sides of
+    that rule and agree bit for bit; FP64 forms on the cached side against the
+    oracle.
+
+Tolerances: those of the short runs against the oracle (1e-13 for FP64, 2e-6 for
+FP32: 30 times the largest differences measured over the parity shapes)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+PRM = dict(t_step=0.005, grad_coeff_phi=1.0, grad_coeff_c=0.8, D_gb=0.0)
+TOL = {"fp64_reduced": 1e-13, "fp64_faithful": 1e-13, "fp32_mixed": 2e-6}
+
+
+def _run(pf, oracle, shape, var, mode, steps, tuning=None):
+    phi, con = pf.ic_voronoi(*shape, var, var + 3)
+    with pf.Simulation(pf.make_params(**PRM), *shape, var, mode) as sim:
+        if tuning:
+            sim.set_tuning(**tuning)
+        sim.put_state(phi, con)
+        rows = sim.step(steps, diag_every=1)
+        gphi, gcon = sim.get_state()
+    od = oracle.run(oracle.make_params(**PRM), phi, con, steps)  # advances phi, con
+    tol = TOL[mode]
+    err = max(np.abs(gphi - phi).max(), np.abs(gcon - con).max())
+    print(f"{mode} {shape} x {var + 1}: {err:.2e}", flush=True)
+    assert err <= tol
+    for d, o in zip(rows, od):
+        scale = abs(o["f_int"]) + abs(o["f_ch"]) + abs(o["f_eta"]) + 1.0
+        for k in ("f_int", "f_ch", "f_eta", "e_tot"):
+            assert abs(d[k] - o[k]) <= tol * scale, k
+
+
+@pytest.mark.parametrize("mode,shape,var", [("fp64_reduced", (160, 8, 8), 48), ("fp64_reduced", (160, 8, 8), 50),
+                                            ("fp64_reduced", (192, 8, 8), 40), ("fp64_reduced", (192, 8, 12), 63),
+                                            ("fp64_reduced", (64, 8, 8), 128), ("fp64_reduced", (32, 8, 8), 256),
+                                            ("fp32_mixed", (160, 8, 8), 96), ("fp32_mixed", (160, 8, 8), 101),
+                                            ("fp32_mixed", (48, 8, 8), 256)])
+def test_more_fields_than_one_round_of_a_block(pf, oracle, mode, shape, var):
+    _run(pf, oracle, shape, var, mode, 3)
+
+
+@pytest.mark.parametrize("lines", [1, 2])
+def test_lines_per_block_beyond_its_threads(pf, oracle, lines):
+    """25 FP64 fields of 160 points in 2-line blocks: 50 lines, two more than one
+    round of a block's waves."""
+    _run(pf, oracle, (160, 8, 8), 24, "fp64_reduced", 3, dict(xline_lines=lines))
+
+
+@pytest.mark.parametrize("members", [3, 14, 28])
+def test_batch_on_the_other_side_of_the_cache_rule(pf, members):
+    """A member's spectrum is 9.3 MiB: alone it is streamed, in a batch of 3 and 14
+    (28 and 130 MiB) it stays cached, in one of 28 (260 MiB) it does not fit."""
+    n, var = 64, 8
+    p = pf.make_params(**PRM)
+    phi, con = pf.ic_voronoi(n, n, n, var, 12)
+    with pf.Simulation(p, n, n, n, var, "fp32_mixed") as one:
+        one.put_state(phi, con)
+        one.step(4)
+        want = one.get_state()
+    sims = [pf.Simulation(p, n, n, n, var, "fp32_mixed") for _ in range(members)]
+    try:
+        for s in sims:
+            s.put_state(phi, con)
+        pf.ensemble_step(sims, 4)
+        for s in (sims[0], sims[-1]):
+            got = s.get_state()
+            assert all(np.array_equal(a, b) for a, b in zip(got, want))
+    finally:
+        for s in sims:
+            s.close()
+
+
+@pytest.mark.parametrize("mode,shape,var", [("fp64_reduced", (64, 64, 64), 11), ("fp64_reduced", (64, 64, 64), 63),
+                                            ("fp64_faithful", (64, 64, 64), 5), ("fp32_mixed", (64, 64, 64), 24)])
+def test_spectra_that_stay_cached(pf, oracle, mode, shape, var):
+    """24.8, 132 and (faithful: the spectra of the state and of its driving forces)
+    24.8 MiB in FP64, 25.8 MiB in FP32."""
+    _run(pf, oracle, shape, var, mode, 2)
