@@ -11,6 +11,7 @@
 // so each field's half spectrum crosses HBM 10 times per step (x: 2, y: 2+2,
 // z: 4 including S), against 17 for separate transform and pointwise passes.
 #pragma once
+#include "pf_nl.hpp"
 #include "pf_passes.hpp"
 
 namespace pf {
@@ -186,9 +187,9 @@ template <typename R, int NX> constexpr int kXlineMaxThreadsN = (sizeof(R) == 8 
 // Minimum waves per SIMD asked of the register allocator.  FP32: 6 for 128- and
 // 160-point lines, which then take up to 79 VGPRs without spills (160^3 x 9: 114 ->
 // 102 us against asking for 5); 5 for the others (at 192 points 6 spilled 4 VGPRs,
-// 192^3 x 9 145 -> 185 us; at 256 points 23, 512 -> 694 us); 4 for 512-point lines, which keep their last transform pass's
-// twiddles in registers (kXlineTwiddleRegs), at most 128 VGPRs, which 1024-thread
-// blocks need anyway.  FP64: 3 (the 256-point kernel takes 167 VGPRs).
+// 192^3 x 9 145 -> 185 us; at 256 points 23, 512 -> 694 us); 4 for 512-point lines,
+// which keep their last transform pass's twiddles in registers (kXlineTwiddleRegs), at
+// most 128 VGPRs, which 1024-thread blocks need anyway.  FP64: 3 (the 256-point kernel takes 167 VGPRs).
 template <typename R, int NX>
 constexpr int kXlineWavesN = sizeof(R) == 8 ? 3 : NX >= 512 ? 4 : (NX >= 128 && NX < 192) ? 6 : 5;
 // The x line's transform plan: variant 4 or 5 where it has one, else the default.
@@ -362,14 +363,26 @@ __device__ __forceinline__ void diag_partials(double ch, double eta, double cmax
 // ROUNDS: the jobs need more threads than a block may have, and the block's waves
 // take them in several rounds (in one loop with the common case its registers
 // spilled: 256^3 x 17 516 -> 684 us).
-template <typename R, int NX, int LINES, bool XONLY, bool BATCH = false, bool KEEP = false, bool ROUNDS = false>
-__global__ void __launch_bounds__((kXlineMaxThreadsN<R, NX>)) __attribute__((amdgpu_waves_per_eu(kXlineWavesN<R, NX>)))
+// FAITH: the faithful step's x pass (FP64, var <= kNlRegs, LINES * NX threads).  The
+// bank has 2F fields.  The real state's R2C goes back to fields 0 .. F-1, the
+// derivatives' (in the reference's operation order) to F .. 2F-1.  mob here says that
+// the state comes real rather than as x-half lines.  A thread takes its point's values
+// into registers, so that the state's rows can be transformed in place before the
+// derivatives are written over them: with rows of their own the derivatives left two
+// blocks a CU, 256^3 x 17 4.3 ms.  The separate x inverse, pointwise and x forward
+// kernels moved seven banks of F, this pass three (a
+// step of 256 x 128 x 128 x 17: 1.98 -> 1.61 ms).  At 256 points the live values take
+// 208 VGPRs, two waves per SIMD.
+template <typename R, int NX, int LINES, bool XONLY, bool BATCH = false, bool KEEP = false, bool ROUNDS = false,
+          bool FAITH = false>
+__global__ void __launch_bounds__((FAITH ? 512 : kXlineMaxThreadsN<R, NX>))
+__attribute__((amdgpu_waves_per_eu(FAITH && NX >= 256 ? 2 : kXlineWavesN<R, NX>)))
 k_xline(Geo g, UPar u, c2<R>* __restrict__ wm, c2<R>* __restrict__ wn, R* __restrict__ mobd,
         const c2<R>* __restrict__ tw, double* __restrict__ part, long ngroups, int diag, int mob,
         const Member<R>* __restrict__ mt) {
   constexpr int M = NX / 2, XV = xline_plan(sizeof(c2<R>)), T = plan_T(M, XV);
   constexpr int MP = xline_row_pitch(M, sizeof(c2<R>)), XF = xline_xf(M, sizeof(c2<R>));
-  constexpr bool HAVEW = xline_has_wide(M);
+  constexpr bool HAVEW = !FAITH && xline_has_wide(M);
   // the wide plan's variant (3) and threads; the T-thread plan stands in when
   // this length has no wide plan, and that branch is never taken then
   constexpr int WV = HAVEW ? 3 : XV, TW = plan_T(M, WV), JW = xline_wave_jobs(M, sizeof(c2<R>));
@@ -439,9 +452,17 @@ k_xline(Geo g, UPar u, c2<R>* __restrict__ wm, c2<R>* __restrict__ wn, R* __rest
     // 1. half lines of every field -> LDS rows, with the C2R pre-processing: wave w
     //    stages row groups w, w + nw, ... (coalesced along k, and along M - k in
     //    descending order), NA of them in flight
+    const bool real = FAITH && mob;
     c2<R> w[PPL];  // a lane's pairs, and so their twiddles, are the same in every row
 #pragma unroll
     for (int i = 0; i < PPL; ++i) w[i] = tw[p0 + 64 * i];
+    if (real) {
+      for (int f = wv; f < F; f += nw) {
+        const c2<R>* src = wmm + (long)f * g.hmain + L0 * M;
+        for (int e = lane; e < LINES * M; e += 64)
+          sh[(f * LINES + e / M) * MP + lds_swz<XF>(e % M)] = src[e];
+      }
+    } else
     for (int j0 = wv; j0 < npieces; j0 += NA * nw) {
       c2<R> ta[NA][PPL], tb[NA][PPL];
 #pragma unroll
@@ -478,6 +499,7 @@ k_xline(Geo g, UPar u, c2<R>* __restrict__ wm, c2<R>* __restrict__ wn, R* __rest
     }
     __syncthreads();
     // 2-3. inverse x transform of each job; real pairs z[n] = (x[2n], x[2n+1]).
+    if (!real)
     for (int jr = 0; jr < (ROUNDS ? njobs : 1); jr += ROUNDS ? nw * JW : 1) {
       const int job = jr + wv * JW + lane / T;
       if (jr > 0) {
@@ -498,7 +520,19 @@ k_xline(Geo g, UPar u, c2<R>* __restrict__ wm, c2<R>* __restrict__ wn, R* __rest
     //    points of one element: one pass instead of two for the first wave
     //    (measured 0.645 -> 0.616 ms); otherwise one point per thread (pairs
     //    measured 4% slower at 128^3, where the points fit one pass anyway).
-    if (!XONLY && LINES * NX > nt) {
+    R pf[FAITH ? kNlRegs : 1], pc = R(0), pv = R(0);  // FAITH: the thread's point
+    R* pt = nullptr;
+    if constexpr (FAITH) {
+      if (tid < LINES * NX) {
+        constexpr long fs = 2L * LINES * MP;
+        const int l = tid / NX, x = tid - l * NX;
+        pt = reinterpret_cast<R*>(sh) + 2L * ((long)l * MP + lds_swz<XF>(x >> 1)) + (x & 1);
+        pc = pt[0];
+        pv = pt[g.var * fs];
+#pragma unroll
+        for (int i = 0; i < kNlRegs; ++i) pf[i] = i < g.var - 1 ? pt[(i + 1) * fs] : R(0);
+      }
+    } else if (!XONLY && LINES * NX > nt) {
       constexpr long fs = (long)LINES * MP;  // field stride in complex elements
       for (int p = tid; p < LINES * M; p += nt) {
         const int l = p / M, k = p - l * M;
@@ -530,74 +564,95 @@ k_xline(Geo g, UPar u, c2<R>* __restrict__ wm, c2<R>* __restrict__ wn, R* __rest
       }
     }
     __syncthreads();
-    // 5. forward x transform of each job.  With TR (256-point FP32 rows, 16
-    //    threads a job, one 16-lane DPP row each) a job's threads also do its R2C
-    //    post-processing and store: after the last pass thread t holds
-    //    Z[t + 16 s] in slot s, whose partner Z[M - t - 16 s] is slot 15 - s of
-    //    thread 16 - t (for t = 0: its own slot (16 - s) mod 16), so the pairs
-    //    come by DPP instead of a write-back and a second read of the row (512^3
-    //    x 37: x line 13.5-13.8 -> 13.0-13.1 ms).  The lone wide job, if any,
-    //    still goes through its row and phase 6.
-    for (int jr = 0; jr < (ROUNDS ? njobs : 1); jr += ROUNDS ? nw * JW : 1) {
-      // recomputed rather than kept in registers through the phases between
-      int tn = threadIdx.x;
-      asm volatile("" : "+v"(tn));
-      const int ln = tn & 63, lt = ln % T, job = jr + wv * JW + ln / T;
-      c2<R>* const wnj = nyq(jr, ln, lt);
-      if (is_wide(jr)) {
-        if (TW == 64 || ln < TW)
-          xline_fft<R, M, WV, XF, false>(v, sh + (njobs - 1) * MP, shw, ln, R(0), wnj, scale);
-      } else if (lact && job < njobs) {
-        c2<R>* const col = sh + job * MP;
-        if constexpr (TR) {
-          static_assert(T == 16 && kInSlots<M> == 16 && kOutSlots<M> == 16, "16 threads, 16 slots a job");
+    const auto forward = [&](const int half) __attribute__((always_inline)) {
+      // 5. forward x transform of each job.  With TR (256-point FP32 rows, 16
+      //    threads a job, one 16-lane DPP row each) a job's threads also do its R2C
+      //    post-processing and store: after the last pass thread t holds
+      //    Z[t + 16 s] in slot s, whose partner Z[M - t - 16 s] is slot 15 - s of
+      //    thread 16 - t (for t = 0: its own slot (16 - s) mod 16), so the pairs
+      //    come by DPP instead of a write-back and a second read of the row (512^3
+      //    x 37: x line 13.5-13.8 -> 13.0-13.1 ms).  The lone wide job, if any,
+      //    still goes through its row and phase 6.
+      for (int jr = 0; jr < (ROUNDS ? njobs : 1); jr += ROUNDS ? nw * JW : 1) {
+        // recomputed rather than kept in registers through the phases between
+        int tn = threadIdx.x;
+        asm volatile("" : "+v"(tn));
+        const int ln = tn & 63, lt = ln % T, job = jr + wv * JW + ln / T;
+        c2<R>* wnj = nyq(jr, ln, lt);
+        if (FAITH && half && wnj) wnj += (long)F * g.plane;
+        if (is_wide(jr)) {
+          if (TW == 64 || ln < TW)
+            xline_fft<R, M, WV, XF, false>(v, sh + (njobs - 1) * MP, shw, ln, R(0), wnj, scale);
+        } else if (lact && job < njobs) {
+          c2<R>* const col = sh + job * MP;
+          if constexpr (TR) {
+            static_assert(T == 16 && kInSlots<M> == 16 && kOutSlots<M> == 16, "16 threads, 16 slots a job");
 #pragma unroll
-          for (int s = 0; s < 16; ++s) v[s] = col[lds_swz<XF>(rfft_in_idx<M>(lt, s))];
-          rfft<R, M, false, 1, 0, XF, true>(v, lt, true, col, shw, 2, 0, twr);
-          const int f = job / LINES, l = job - f * LINES;
-          c2<R>* dst = wmm + (long)f * g.hmain + (L0 + l) * M;
-          const R hs = R(0.5) * scale;
+            for (int s = 0; s < 16; ++s) v[s] = col[lds_swz<XF>(rfft_in_idx<M>(lt, s))];
+            rfft<R, M, false, 1, 0, XF, true>(v, lt, true, col, shw, 2, 0, twr);
+            const int f = job / LINES, l = job - f * LINES;
+            c2<R>* dst = wmm + (long)f * g.hmain + (L0 + l) * M;
+            const R hs = R(0.5) * scale;
 #pragma unroll
-          for (int s = 0; s < 16; ++s) {
-            const int k = rfft_out_idx<M>(lt, s);  // t + 16 s
-            const c2<R> src = v[15 - s];
-            c2<R> pr = mk<R>(dpp_partner16(src.x), dpp_partner16(src.y));
-            if (lt == 0) pr = v[(16 - s) % 16];
-            const c2<R> x = r2c_post<R>(v[s], pr, shw[k], hs);
-            if constexpr (KEEP) dst[k] = x;
-            else st_nt<R>(dst + k, x);
+            for (int s = 0; s < 16; ++s) {
+              const int k = rfft_out_idx<M>(lt, s);  // t + 16 s
+              const c2<R> src = v[15 - s];
+              c2<R> pr = mk<R>(dpp_partner16(src.x), dpp_partner16(src.y));
+              if (lt == 0) pr = v[(16 - s) % 16];
+              const c2<R> x = r2c_post<R>(v[s], pr, shw[k], hs);
+              if constexpr (KEEP) dst[k] = x;
+              else st_nt<R>(dst + k, x);
+            }
+            if (lt == 0) *wnj = mk<R>((v[0].x - v[0].y) * scale, R(0));
+          } else {
+            xline_fft<R, M, XV, XF, false, TR>(v, col, shw, lt, R(0), wnj, scale, twr);
           }
-          if (lt == 0) *wnj = mk<R>((v[0].x - v[0].y) * scale, R(0));
-        } else {
-          xline_fft<R, M, XV, XF, false, TR>(v, col, shw, lt, R(0), wnj, scale, twr);
         }
       }
-    }
-    __syncthreads();
-    // 6. R2C post-processing and store, the row groups and pairs of 1 (with TR only
-    //    the wide job's row)
-    const R hs = R(0.5) * scale;
+      __syncthreads();
+      // 6. R2C post-processing and store, the row groups and pairs of 1 (with TR only
+      //    the wide job's row)
+      const R hs = R(0.5) * scale;
 #pragma unroll
-    for (int i = 0; i < PPL; ++i) w[i] = shw[p0 + 64 * i];
-    for (int j = wv; j < npieces; j += nw) {
-      if (TR && !(wide_any && j == njobs - 1)) continue;
-      const int f = j / (LINES / RP), l = (j - f * (LINES / RP)) * RP;
-      c2<R>* dst = wmm + (long)f * g.hmain + (L0 + l) * M;
-      const c2<R>* rw = sh + (j * RP + sub) * MP;
-      if (!mine) continue;
+      for (int i = 0; i < PPL; ++i) w[i] = shw[p0 + 64 * i];
+      for (int j = wv; j < npieces; j += nw) {
+        if (TR && !(wide_any && j == njobs - 1)) continue;
+        const int f = j / (LINES / RP), l = (j - f * (LINES / RP)) * RP;
+        c2<R>* dst = wmm + (long)(FAITH && half ? F + f : f) * g.hmain + (L0 + l) * M;
+        const c2<R>* rw = sh + (j * RP + sub) * MP;
+        if (!mine) continue;
 #pragma unroll
-      for (int i = 0; i < PPL; ++i) {
-        const int p = p0 + 64 * i, q = xline_partner<M>(p);
-        c2<R> a = rw[lds_swz<XF>(p)], b = rw[lds_swz<XF>(q)];
-        xline_r2c_pair<R>(a, b, w[i], p == 0, hs);
-        if constexpr (KEEP) {
-          dst[sub * M + p] = a;
-          dst[sub * M + q] = b;
-        } else {
-          st_nt<R>(dst + (sub * M + p), a);
-          st_nt<R>(dst + (sub * M + q), b);
+        for (int i = 0; i < PPL; ++i) {
+          const int p = p0 + 64 * i, q = xline_partner<M>(p);
+          c2<R> a = rw[lds_swz<XF>(p)], b = rw[lds_swz<XF>(q)];
+          xline_r2c_pair<R>(a, b, w[i], p == 0, hs);
+          if constexpr (KEEP) {
+            dst[sub * M + p] = a;
+            dst[sub * M + q] = b;
+          } else {
+            st_nt<R>(dst + (sub * M + p), a);
+            st_nt<R>(dst + (sub * M + q), b);
+          }
         }
       }
+    };
+    forward(0);
+    if constexpr (FAITH) {
+      __syncthreads();
+      if (pt) {
+        // not before the state's transforms: the products of these would be held too
+        asm volatile("" : "+v"(pc), "+v"(pv));
+#pragma unroll
+        for (int i = 0; i < kNlRegs; ++i) asm volatile("" : "+v"(pf[i]));
+        constexpr long fs = 2L * LINES * MP;
+        const auto put = [&](int i, R y) { pt[i * fs] = y; };
+        R mo;
+        if (diag) nl_point_regs<true>(uu, g.var, pc, pf, pv, put, mo, a_ch, a_eta, cmax, cmin, pmin, p3);
+        else nl_point_regs<false>(uu, g.var, pc, pf, pv, put, mo, a_ch, a_eta, cmax, cmin, pmin, p3);
+        mobd[L0 * NX + (long)threadIdx.x] = mo;
+      }
+      __syncthreads();
+      forward(1);
     }
     __syncthreads();
   }

@@ -38,6 +38,10 @@ int zline_batch(const StepCall& c, const Member<float>* mt, long nmem, hipStream
 template <typename R>
 int xline(bool xonly, const StepCall& c, c2<R>* wm, c2<R>* wn, R* mobd, double* part, long* nblocks, bool diag,
           bool mob, hipStream_t s);
+// The faithful step's x pass (k_xline's FAITH) on the bank U of 2F fields, whose state
+// is real or x-half lines; var <= kNlRegs.
+int xline_faithful(const StepCall& c, bool real, Bank<double> U, double* mobd, double* part, long* nblocks,
+                   bool diag, hipStream_t s);
 // Whether the x-line takes this grid and field count in blocks of `lines` lines (0:
 // of some number).
 template <typename R> bool xline_accepts(const Geo& g, int lines);

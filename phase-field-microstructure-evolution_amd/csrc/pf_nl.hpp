@@ -122,4 +122,95 @@ __device__ __forceinline__ void nl_point_faithful(const UPar& u, int V, double c
   }
 }
 
+// The same with the order parameters in registers, V <= kNlRegs: f holds the V - 1
+// matrix grains, 0 from there on (terms of 0 that leave the sums as they are, and are
+// skipped four at a time), fv the precipitate's.  Nothing is read after a result is
+// given, so put may overwrite the point's values.
+constexpr int kNlRegs = 16;
+template <bool DIAG, typename Put>
+__device__ __forceinline__ void nl_point_regs(const UPar& u, int V, double con, const double (&f)[kNlRegs], double fv,
+                                              Put put, double& mob, double& ch, double& eta, double& cmax,
+                                              double& cmin, double& pmin, double& p3) {
+  const int mat = V - 1;
+  const double fv2 = fv * fv, fv4 = fv2 * fv2;
+  // loop 5
+  double fe = 0.0;
+  if (DIAG) {
+#pragma unroll
+    for (int i = 0; i < kNlRegs - 1; ++i) {
+      if (i >= mat) break;
+      const double fi2 = f[i] * f[i];
+      fe = (fe - 0.5 * fi2) + 0.25 * (fi2 * fi2);
+      const double g1 = u.s1g * fi2, g2 = u.s2g * fi2;
+#pragma unroll
+      for (int j0 = 0; j0 < kNlRegs; j0 += kNlRows) {
+        if (j0 + kNlRows - 1 <= i || j0 >= mat) continue;
+#pragma unroll
+        for (int j = j0; j < j0 + kNlRows; ++j)
+          if (j > i) fe = fe + g1 * (f[j] * f[j]);
+      }
+      fe = fe + g2 * fv2;
+    }
+    fe = (fe - 0.5 * fv2) + 0.25 * fv4;
+  }
+  // loop 6
+  double num = 0.0;
+#pragma unroll
+  for (int i = 0; i < kNlRegs; ++i) {
+    const double f2 = f[i] * f[i];
+    num = num + f2 * f2;
+  }
+  const double den = num + fv4;
+  const double hm = num / den, hp = 1.0 - hm;
+  const double dm = con - u.cm, dp = con - u.cp;
+  const double fch = (hm * u.am) * (dm * dm) + (hp * u.ap) * (dp * dp);
+  put(0, ((2.0 * hm) * u.am) * dm + ((2.0 * hp) * u.ap) * dp);
+  // loops 7-9
+  const double fm = u.am * (dm * dm), fp = u.ap * (dp * dp);
+  const double t2v = (4.0 * (fv2 * fv)) * (den - fv4);
+  const double den2 = den * den;
+  double ps = 0.0;
+#pragma unroll
+  for (int i0 = 0; i0 < kNlRegs; i0 += kNlRows) {
+    if (i0 >= mat) continue;
+#pragma unroll
+    for (int i = i0; i < i0 + kNlRows; ++i) {
+      if (i >= mat) break;
+      const double fi = f[i], ci = (2.0 * u.s1g) * fi;
+      double t2 = 0.0;
+#pragma unroll
+      for (int j0 = 0; j0 < kNlRegs; j0 += kNlRows) {
+        if (j0 >= mat) continue;
+#pragma unroll
+        for (int j = j0; j < j0 + kNlRows; ++j)
+          if (j != i) t2 = t2 + ci * (f[j] * f[j]);
+      }
+      const double term1 = (fi * fi) * fi - fi;
+      t2 = t2 + ((2.0 * u.s2g) * fi) * fv2;
+      const double term4 = (((4.0 * ((fi * fi) * fi)) * fv4) * (fm - fp)) / den2;
+      put(i + 1, (term1 + t2) + term4);
+      ps = ps + fi * fi;
+    }
+  }
+  {
+    const double term1 = (fv * fv) * fv - fv, c2 = (2.0 * u.s2g) * fv;
+    double t2 = 0.0;
+#pragma unroll
+    for (int j = 0; j < kNlRegs; ++j) t2 = t2 + c2 * (f[j] * f[j]);
+    const double term4 = (t2v * (fp - fm)) / den2;
+    put(V, (term1 + t2) + term4);
+    ps = ps + fv * fv;
+  }
+  // loop 10
+  mob = (u.D + ((2.0 * (1.0 - ps)) * u.Dgb)) - u.D;
+  if (DIAG) {
+    ch += fch;
+    eta += fe;
+    if (fv > p3) p3 = fv;
+    if (con <= cmin) cmin = con;
+    if (con > cmax) cmax = con;
+    if (ps < pmin) pmin = ps;
+  }
+}
+
 }  // namespace pf

@@ -332,6 +332,7 @@ struct pf_handle {
   double* part_fi = nullptr;
   long n_part_nl = 0, n_part_fi = 0;
   bool fint_ready = false;  // part_fi holds f_int of the current state
+  bool fs_half = false;     // faithful: fs holds x-half lines of the state (only within a call)
   double* ddiag = nullptr;  // 9 doubles per record
   long ddiag_cap = 0;
 
@@ -580,28 +581,50 @@ int step_reduced(pf_handle* h, bool diag, long rec, bool fint_next) {
 
 // ---------------------------------------------------------------------------
 // Faithful step (FP64): the reference's loop sequence on the real-space state.
-// Twelve launches: the state's and the derivatives' forward transforms run as one
-// batch of 2F fields, the last forward pass, the k-space loops and the first
-// inverse pass are one kernel (k_zfaithful).
+// The state's and the derivatives' forward transforms run as one batch of 2F fields,
+// the last forward pass, the k-space loops and the first inverse pass are one kernel
+// (k_zfaithful).  Where faithful_halves says so the last inverse pass, the pointwise
+// loops and the first forward pass are one kernel too (k_xline's FAITH), ten launches:
+// the steps of one call leave the state before its last inverse pass, on x-half lines
+// (fs_half), and settle_faithful ends the call with the real state.  Elsewhere the
+// three kernels run: twelve.
 // ---------------------------------------------------------------------------
+// Whether the faithful step's x passes and pointwise loops are one kernel.  Its blocks
+// have a thread per point; with few fields on long lines most of them wait while the
+// transforms run, and the separate kernels are faster (below 13 fields 160 points also
+// take two lines a block).  Steps, us, separate and one:
+// 64^3 x 5 111 and 88, x 17 175 and 151; 96^3 x 5 199 and 219, x 9 280 and 288, x 17
+// 441 and 368; 192 x 96 x 96 x 9 485 and 530, x 17 858 and 733; 256 x 128 x 128 x 9
+// 1124 and 1090, x 17 1983 and 1613; 512 x 64 x 64 x 9 553 and 569, x 17 1010 and 935;
+// 160 x 96 x 96 x 12 551 and 584, x 17 729 and 611.
+bool faithful_halves(const Geo& g) { return g.var <= kNlRegs && (g.nx <= 64 || g.F >= 13); }
+
 int step_faithful(pf_handle* h, bool diag, long rec) {
   const Geo& g = h->g;
   hipStream_t s = h->s;
   const Bank<double> U = h->fs, D = sub(h->fs, g, g.F), G = h->fdum;
-  const double scale = 1.0 / (double)(float)g.P;
   int rc;
-  // loops 5-10 (read the real state before it is transformed in place)
-  tbeg(h, ST_NONLINEAR);
   long nnl = 0;
-  if ((rc = faithful_nonlinear(g, h->u, diag, (const double*)U.main, (double*)D.main, (double*)h->mob, h->part_nl,
-                               kMaxGrid, &nnl, s)))
-    return rc;
+  if (faithful_halves(g)) {
+    // the last inverse pass, loops 5-10 and F(c), F(phi_i), F(df_dc), F(df_dphi_i) along x
+    tbeg(h, ST_NONLINEAR);
+    if ((rc = xline_faithful(StepCall{g, h->u, h->kt, h->tune}, !h->fs_half, U, (double*)h->mob, h->part_nl, &nnl,
+                             diag, s)))
+      return rc;
+    tend(h);
+  } else {
+    // loops 5-10 (read the real state before it is transformed in place)
+    tbeg(h, ST_NONLINEAR);
+    if ((rc = faithful_nonlinear(g, h->u, diag, (const double*)U.main, (double*)D.main, (double*)h->mob, h->part_nl,
+                                 kMaxGrid, &nnl, s)))
+      return rc;
+    tend(h);
+    tbeg(h, ST_X_R2C);
+    if ((rc = x_r2c<double>(g.nx, U.main, U.main, U.nyq, (long)g.plane * 2 * g.F, 1.0 / (double)(float)g.P, s)))
+      return rc;
+    tend(h);
+  }
   if (diag) h->n_part_nl = nnl;
-  tend(h);
-  // F(c), F(phi_i), F(df_dc), F(df_dphi_i): x and y
-  tbeg(h, ST_X_R2C);
-  if ((rc = x_r2c<double>(g.nx, U.main, U.main, U.nyq, (long)g.plane * 2 * g.F, scale, s))) return rc;
-  tend(h);
   tbeg(h, ST_Y_FWD);
   if ((rc = y_pass<double>(g.ny, false, U.main, U.nyq, g.M, (long)g.nz * 2 * g.F, s))) return rc;
   tend(h);
@@ -632,11 +655,33 @@ int step_faithful(pf_handle* h, bool diag, long rec) {
   tbeg(h, ST_Y_INV);
   if ((rc = y_pass<double>(g.ny, true, U.main, U.nyq, g.M, (long)g.nz * g.F, s))) return rc;
   tend(h);
-  tbeg(h, ST_X_C2R);
-  if ((rc = x_c2r<double>(g.nx, U.main, U.main, U.nyq, (long)g.plane * g.F, s))) return rc;
-  tend(h);
+  h->fs_half = faithful_halves(g);
+  if (!h->fs_half) {
+    tbeg(h, ST_X_C2R);
+    if ((rc = x_c2r<double>(g.nx, U.main, U.main, U.nyq, (long)g.plane * g.F, s))) return rc;
+    tend(h);
+  }
   return 0;
 }
+
+// The real state of a faithful handle whose last step left it on x-half lines: what
+// every call that steps ends with, whatever it returns.
+int settle_faithful(pf_handle* h) {
+  if (!h->fs_half) return 0;
+  const Geo& g = h->g;
+  h->fs_half = false;
+  tbeg(h, ST_X_C2R);
+  const int rc = x_c2r<double>(g.nx, h->fs.main, h->fs.main, h->fs.nyq, (long)g.plane * g.F, h->s);
+  tend(h);
+  return rc;
+}
+struct SettleFaithful {  // a call's early returns
+  pf_handle* const* h;
+  size_t n;
+  ~SettleFaithful() {
+    for (size_t i = 0; i < n; ++i) (void)settle_faithful(h[i]);
+  }
+};
 
 template <typename R> int alloc_reduced(pf_handle* h) {
   Geo& g = h->g;
@@ -1023,14 +1068,17 @@ int step_once(pf_handle* h, bool diag, long rec, bool next_diag) {
 int capture_period(pf_handle* h, int de) {
   drop_graph(h);
   const int P = de > 0 ? de : 1;
-  const bool ready0 = h->fint_ready;
+  const bool ready0 = h->fint_ready, half0 = h->fs_half;
   h->fint_ready = (de == 1);
+  // a faithful period starts from x-half lines (replayable)
+  h->fs_half = h->mode == PF_MODE_FP64_FAITHFUL && faithful_halves(h->g);
   h->capturing = true;
   h->cap_step = P;
   int rc = 0;
   if (hipStreamBeginCapture(h->s, hipStreamCaptureModeThreadLocal) != hipSuccess) {
     h->capturing = false;
     h->fint_ready = ready0;
+    h->fs_half = half0;
     h->graphs = false;
     (void)hipGetLastError();
     return 0;
@@ -1044,6 +1092,7 @@ int capture_period(pf_handle* h, int de) {
   const hipError_t e = hipStreamEndCapture(h->s, &graph);
   h->capturing = false;
   h->fint_ready = ready0;
+  h->fs_half = half0;
   if (rc) {
     if (graph) (void)hipGraphDestroy(graph);
     return rc;
@@ -1058,6 +1107,12 @@ int capture_period(pf_handle* h, int de) {
   }
   if (graph) (void)hipGraphDestroy(graph);
   return 0;
+}
+
+// Whether the next step is one a captured period can stand for: a faithful call's
+// first step starts from the real state, the steps after it from x-half lines.
+bool replayable(const pf_handle* h) {
+  return h->mode != PF_MODE_FP64_FAITHFUL || h->fs_half || !faithful_halves(h->g);
 }
 
 // Fewest replays of a period for which a call captures (or reuses) a graph.
@@ -1170,6 +1225,7 @@ extern "C" int pf_ensemble_step(pf_handle* const* hs, int n, int nsteps) {
       h->fint_ready = false;
       h->step += nsteps;
     }
+  const SettleFaithful settle{single.data(), single.size()};
   // members step without diagnostics: a captured one-step period each
   for (pf_handle* h : single) {
     if (nsteps >= kMinGraphReplays && h->graphs && !h->timing && h->gx_key != 0) {
@@ -1179,7 +1235,7 @@ extern "C" int pf_ensemble_step(pf_handle* const* hs, int n, int nsteps) {
   }
   for (int st = 0; st < nsteps; ++st) {
     for (pf_handle* h : single) {
-      if (h->gx && h->gx_key == 0 && !h->timing && nsteps >= kMinGraphReplays) {
+      if (h->gx && h->gx_key == 0 && !h->timing && nsteps >= kMinGraphReplays && replayable(h)) {
         PF_HIP(hipGraphLaunch(h->gx, h->s));
         h->fint_ready = false;
       } else {
@@ -1189,6 +1245,8 @@ extern "C" int pf_ensemble_step(pf_handle* const* hs, int n, int nsteps) {
       h->step += 1;
     }
   }
+  for (pf_handle* h : single)
+    if (const int rc1 = settle_faithful(h)) return rc1;
   PF_HIP(hipGetLastError());
   for (pf_handle* h : single) {
     PF_HIP(hipStreamSynchronize(h->s));
@@ -1207,6 +1265,7 @@ extern "C" int pf_step(pf_handle* h, int nsteps, int diag_every, pf_diag* out) {
   const int de = (out && diag_every > 0) ? diag_every : 0;
   const int P = de > 0 ? de : 1;
   int i = 0;
+  const SettleFaithful settle{&h, 1};
   while (i < nsteps) {
     const long stepno = h->step + 1;
     // replays of whole periods: the steps from i on follow the captured pattern
@@ -1214,7 +1273,7 @@ extern "C" int pf_step(pf_handle* h, int nsteps, int diag_every, pf_diag* out) {
     // faithful form recomputes it, so every step of de = 1 is alike)
     const bool carry = h->mode != PF_MODE_FP64_FAITHFUL;
     long K = 0;
-    if (h->graphs && !h->timing) {
+    if (h->graphs && !h->timing && replayable(h)) {
       if (de == 0 || (de == 1 && !carry)) K = nsteps - i;
       else if (de == 1) K = (i >= 1 && h->fint_ready) ? (nsteps - 1) - i : 0;
       else if (stepno % de == 1 && !h->fint_ready) K = (nsteps - i) / de;
@@ -1239,6 +1298,7 @@ extern "C" int pf_step(pf_handle* h, int nsteps, int diag_every, pf_diag* out) {
     h->step = stepno;
     ++i;
   }
+  if ((rc = settle_faithful(h))) return rc;
   PF_HIP(hipGetLastError());
   std::vector<double> hd;
   if (out && nsteps > 0) {
@@ -1367,7 +1427,9 @@ extern "C" double pf_stage_bytes(pf_handle* h, int stage) {
   const double Bc = 2.0 * (double)(g.M + 1) * g.plane * s; // one half spectrum
   const double F = g.F;
   switch (stage) {
-    case ST_NONLINEAR: return 2.0 * F * Br + (h->p.D_gb != 0.0 ? Br : 0.0);
+    case ST_NONLINEAR:
+      if (h->mode == PF_MODE_FP64_FAITHFUL && faithful_halves(g)) return 3.0 * F * Bc + Br;
+      return 2.0 * F * Br + (h->p.D_gb != 0.0 ? Br : 0.0);
     case ST_X_R2C: return F * (Br + Bc);
     case ST_Y_FWD: case ST_Z_FWD: case ST_Z_INV: case ST_Y_INV: return 2.0 * F * Bc;
     case ST_X_C2R: return F * (Bc + Br);

@@ -42,7 +42,7 @@ template <typename R, int NX> bool xline_fits(const Geo& g, long F, int lines) {
          xline_lds<R, NX>(jobs) + 16 * sizeof(double) <= kXlineMaxLds;
 }
 
-template <typename R, int NX, int LINES, bool XONLY, bool BATCH, bool KEEP, bool ROUNDS>
+template <typename R, int NX, int LINES, bool XONLY, bool BATCH, bool KEEP, bool ROUNDS, bool FAITH = false>
 int xline_one(const StepCall& c, c2<R>* wm, c2<R>* wn, R* mobd, double* part, long ngroups, long waves, bool diag,
               bool mob, const Member<R>* mt, long* nblocks, hipStream_t s) {
   const Geo& g = c.g;
@@ -56,7 +56,7 @@ int xline_one(const StepCall& c, c2<R>* wm, c2<R>* wn, R* mobd, double* part, lo
   const size_t shb = xline_lds<R, NX>((long)(XONLY ? 1 : g.F) * LINES);
   const c2<R>* tw = twiddle_table<R>(NX);
   if (!tw) return fail(PF_EHIP, "twiddle table set-up failed");
-  auto kernel = &k_xline<R, NX, LINES, XONLY, BATCH, KEEP, ROUNDS>;
+  auto kernel = &k_xline<R, NX, LINES, XONLY, BATCH, KEEP, ROUNDS, FAITH>;
   if (shb > 65536 && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)shb) != hipSuccess)
     return fail(PF_EHIP, "x-line kernel: " + std::to_string(shb) + " bytes of LDS refused");
@@ -119,6 +119,36 @@ int xline(bool xonly, const StepCall& c, c2<R>* wm, c2<R>* wn, R* mobd, double* 
           bool mob, hipStream_t s) {
   return xonly ? xline_size<R, true, false>(c, wm, wn, mobd, part, 1, diag, mob, nullptr, nblocks, s)
                : xline_size<R, false, false>(c, wm, wn, mobd, part, 1, diag, mob, nullptr, nblocks, s);
+}
+
+// The faithful step's x pass: a thread per point, one round.
+template <int NX, int LINES>
+int xline_faithful_lines(const StepCall& c, bool real, Bank<double> U, double* mobd, double* part, long* nblocks,
+                         bool diag, hipStream_t s) {
+  const Geo& g = c.g;
+  constexpr int JW = xline_wave_jobs(NX / 2, sizeof(double2));
+  const long jobs = (long)g.F * LINES, ngroups = g.plane / LINES;
+  const long waves = std::max<long>((jobs + JW - 1) / JW, (LINES * NX + 63) / 64);
+  // the state and derivative banks together
+  if (bank_stays(2ul * g.F * g.P * sizeof(double)))
+    return xline_one<double, NX, LINES, false, false, true, false, true>(c, U.main, U.nyq, mobd, part, ngroups, waves,
+                                                                         diag, real, nullptr, nblocks, s);
+  return xline_one<double, NX, LINES, false, false, false, false, true>(c, U.main, U.nyq, mobd, part, ngroups, waves,
+                                                                        diag, real, nullptr, nblocks, s);
+}
+template <int NX>
+int xline_faithful_of(const StepCall& c, bool real, Bank<double> U, double* mobd, double* part, long* nblocks,
+                      bool diag, hipStream_t s) {
+  const Geo& g = c.g;
+  constexpr int JW = xline_wave_jobs(NX / 2, sizeof(double2)), threads = 512;
+  const int want = xline_lines(g.F, NX / 2, sizeof(double2));
+#define PF_TRY(L)                                                                              \
+  if constexpr (L * NX <= threads)                                                             \
+    if (want >= L && xline_fits<double, NX>(g, g.F, L) && (long)g.F * L <= JW * (threads / 64)) \
+      return xline_faithful_lines<NX, L>(c, real, U, mobd, part, nblocks, diag, s);
+  PF_TRY(8) PF_TRY(4) PF_TRY(2) PF_TRY(1)
+#undef PF_TRY
+  return fail(PF_ENOTIMPL, "faithful x line: fields exceed one block");
 }
 
 template <typename R> bool xline_accepts(const Geo& g, int lines) {

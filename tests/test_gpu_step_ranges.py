@@ -83,3 +83,31 @@ def test_spectra_that_stay_cached(pf, oracle, mode, shape, var):
     """24.8, 132 and (faithful: the spectra of the state and of its driving forces)
     24.8 MiB in FP64, 25.8 MiB in FP32."""
     _run(pf, oracle, shape, var, mode, 2)
+
+
+# The faithful form's one-kernel x pass: every x length at its largest field count and
+# either side of the counts and lengths where it takes over from the three kernels.
+@pytest.mark.parametrize("shape,var", [((8, 8, 12), 1), ((12, 8, 8), 2), ((16, 8, 8), 16), ((24, 12, 8), 7),
+                                       ((32, 8, 8), 16), ((48, 8, 8), 5), ((64, 8, 16), 16), ((96, 8, 8), 11),
+                                       ((96, 8, 8), 12), ((128, 8, 8), 16), ((160, 8, 8), 12), ((192, 8, 8), 16),
+                                       ((256, 8, 8), 16), ((512, 8, 8), 16), ((64, 8, 8), 17)])
+def test_faithful_x_pass(pf, oracle, shape, var):
+    _run(pf, oracle, shape, var, "fp64_faithful", 4)
+
+
+@pytest.mark.parametrize("shape,var", [((24, 8, 8), 4), ((256, 8, 8), 13)])
+def test_faithful_calls_of_any_length_agree(pf, shape, var):
+    """Steps in calls of 1, 2 and 5, and in one call by replayed graphs, bit for bit: a
+    call starts from the real state and its later steps from x-half lines."""
+    phi, con = pf.ic_voronoi(*shape, var, var + 3)
+    p = pf.make_params(**dict(PRM, D_gb=0.4))
+    got = []
+    for calls, graphs in (([8], True), ([8], False), ([1] * 8, True), ([2, 5, 1], True)):
+        with pf.Simulation(p, *shape, var, "fp64_faithful") as s:
+            s.set_graphs(graphs)
+            s.put_state(phi, con)
+            for n in calls:
+                s.step(n, diag_every=2)
+            got.append(s.get_state())
+    for g in got[1:]:
+        assert all(np.array_equal(a, b) for a, b in zip(g, got[0]))
