@@ -136,7 +136,8 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic_fused_kernels_256x17_
 # The sources that decide what the step kernels read and write and how they are
 # launched; the traffic profile records their hash when it is measured.
 KERNEL_SOURCES = [os.path.join(ROOT, "phase-field-microstructure-evolution_amd", "csrc", f)
-                  for f in ("pf_fused.hpp", "pf_passes.hpp", "pf_xline_launch.hpp", "pf_zline_launch.hpp", "pf_kernels.hpp", "pf_fft2.hpp", "pf_fft.hpp", "pf_step_kernels.hpp",
+                  for f in ("pf_fused.hpp", "pf_passes.hpp", "pf_xline_launch.hpp", "pf_zline_launch.hpp",
+                            "pf_kernels.hpp", "pf_fft2.hpp", "pf_fft.hpp", "pf_step_kernels.hpp",
                             "pf_step.hip", "pf_tuned.inc")]
 
 
