@@ -49,12 +49,32 @@ __global__ void k_scatter_state(const double* __restrict__ phi, const double* __
     for (int i = 0; i < var; ++i) dst[(long)(i + 1) * P + t] = (R)phi[t * var + i];
   }
 }
+// Bank -> AoS through an LDS tile of kGatherPoints points by kGatherFields fields, so
+// that a point's fields are written in runs of up to 128 bytes: a thread per point
+// stored 8 bytes every 8 var (256^3 x 17 FP32 3.68 -> 0.68 ms, 128^3 x 9 FP64 158 -> 56
+// us, 64^3 x 9 FP32 18.9 -> 8.6 us).
+constexpr int kGatherPoints = 128, kGatherFields = 16;
 template <typename R>
-__global__ void k_gather_state(const R* __restrict__ src, double* __restrict__ phi,
-                               double* __restrict__ con, long P, int var) {
-  for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < P; t += (long)gridDim.x * blockDim.x) {
-    con[t] = (double)src[t];
-    for (int i = 0; i < var; ++i) phi[t * var + i] = (double)src[(long)(i + 1) * P + t];
+__global__ void __launch_bounds__(NB) k_gather_state(const R* __restrict__ src, double* __restrict__ phi,
+                                                     double* __restrict__ con, long P, int var) {
+  constexpr int TP = kGatherPoints, TF = kGatherFields;
+  __shared__ double tile[TF][TP + 1];
+  for (long t0 = (long)blockIdx.x * TP; t0 < P; t0 += (long)gridDim.x * TP) {
+    const int np = (int)min((long)TP, P - t0);
+    if ((int)threadIdx.x < np) con[t0 + threadIdx.x] = (double)src[t0 + threadIdx.x];
+    for (int i0 = 0; i0 < var; i0 += TF) {
+      const int nf = min(TF, var - i0);
+      for (int e = threadIdx.x; e < nf * TP; e += NB) {
+        const int i = e / TP, q = e % TP;
+        if (q < np) tile[i][q] = (double)src[(long)(i0 + i + 1) * P + t0 + q];
+      }
+      __syncthreads();
+      for (int e = threadIdx.x; e < nf * np; e += NB) {
+        const int q = e / nf, i = e - q * nf;
+        phi[(t0 + q) * var + i0 + i] = tile[i][q];
+      }
+      __syncthreads();
+    }
   }
 }
 
@@ -1032,15 +1052,15 @@ extern "C" int pf_get_state(pf_handle* h, double* phi, double* con) {
   double* scon = h->staging + (size_t)g.var * g.P;
   int rc = 0;
   if (h->mode == PF_MODE_FP64_FAITHFUL) {
-    hipLaunchKernelGGL((k_gather_state<double>), dim3(grid_for(g.P, NB)), dim3(NB), 0, h->s,
+    hipLaunchKernelGGL((k_gather_state<double>), dim3(grid_for(g.P, kGatherPoints)), dim3(NB), 0, h->s,
                        (const double*)h->fs.main, sphi, scon, g.P, g.var);
   } else if (h->mode == PF_MODE_FP64_REDUCED) {
     if ((rc = real_state_reduced<double>(h))) return rc;
-    hipLaunchKernelGGL((k_gather_state<double>), dim3(grid_for(g.P, NB)), dim3(NB), 0, h->s,
+    hipLaunchKernelGGL((k_gather_state<double>), dim3(grid_for(g.P, kGatherPoints)), dim3(NB), 0, h->s,
                        (const double*)h->X_main, sphi, scon, g.P, g.var);
   } else {
     if ((rc = real_state_reduced<float>(h))) return rc;
-    hipLaunchKernelGGL((k_gather_state<float>), dim3(grid_for(g.P, NB)), dim3(NB), 0, h->s,
+    hipLaunchKernelGGL((k_gather_state<float>), dim3(grid_for(g.P, kGatherPoints)), dim3(NB), 0, h->s,
                        (const float*)h->X_main, sphi, scon, g.P, g.var);
   }
   PF_HIP(hipGetLastError());

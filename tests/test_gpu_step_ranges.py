@@ -111,3 +111,24 @@ def test_faithful_calls_of_any_length_agree(pf, shape, var):
             got.append(s.get_state())
     for g in got[1:]:
         assert all(np.array_equal(a, b) for a, b in zip(g, got[0]))
+
+
+@pytest.mark.parametrize("mode", ["fp64_faithful", "fp32_mixed"])
+@pytest.mark.parametrize("shape,var", [((12, 12, 12), 1), ((8, 8, 12), 15), ((12, 12, 12), 16), ((8, 12, 12), 17),
+                                       ((12, 12, 12), 33)])
+def test_state_comes_back_point_by_point(pf, mode, shape, var):
+    """put_state then get_state, point counts and field counts around the tiles of 128
+    points by 16 fields: the faithful form's state as it was, FP32 rounded once more by
+    its transforms."""
+    rng = np.random.default_rng(var)
+    n = shape[2], shape[1], shape[0]
+    phi, con = rng.random(n + (var,)), rng.random(n)
+    with pf.Simulation(pf.make_params(**PRM), *shape, var, mode) as s:
+        ref_phi, ref_con = pf.ic_voronoi(*shape, var, var + 3)
+        phi, con = phi.reshape(ref_phi.shape), con.reshape(ref_con.shape)
+        s.put_state(phi, con)
+        gphi, gcon = s.get_state()
+    if mode == "fp64_faithful":
+        assert np.array_equal(gphi, phi) and np.array_equal(gcon, con)
+    else:
+        assert np.abs(gphi - phi).max() <= 2e-6 and np.abs(gcon - con).max() <= 2e-6
