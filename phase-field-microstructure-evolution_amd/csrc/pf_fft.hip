@@ -251,16 +251,18 @@ int x_r2c(int nx, const c2<R>* src, c2<R>* dst, c2<R>* nyq, long nlines, R scale
   return 0;
 }
 
-template <typename R>
-int x_c2r(int nx, const c2<R>* src, c2<R>* dst, const c2<R>* nyq, long nlines, hipStream_t s) {
+namespace {
+// V: plan variant, for the lengths that have it.
+template <typename R, int V>
+int x_c2r_plan(int nx, const c2<R>* src, c2<R>* dst, const c2<R>* nyq, long nlines, hipStream_t s) {
   const c2<R>* tw = twiddle_table<R>(nx);
   if (!tw) return fail(PF_EHIP, "twiddle table set-up failed");
   switch (nx) {
 #define PF_CASE(N)                                                                   \
   case N: {                                                                          \
-    constexpr int LPB = x_lines<R>(N / 2);                                           \
-    hipLaunchKernelGGL((k_x_c2r<R, N>), dim3(ceil_div(nlines, LPB)),                 \
-                       dim3(LPB * plan_T(N / 2)), 0, s, src, dst, nyq, nlines, tw); \
+    constexpr int W = plan_alt(N / 2, V, 0) ? V : 0, LPB = x_lines<R>(N / 2, W);     \
+    hipLaunchKernelGGL((k_x_c2r<R, N, W>), dim3(ceil_div(nlines, LPB)),              \
+                       dim3(LPB * plan_T(N / 2, W)), 0, s, src, dst, nyq, nlines, tw); \
     break;                                                                           \
   }
     PF_GRID_SIZES(PF_CASE)
@@ -268,6 +270,15 @@ int x_c2r(int nx, const c2<R>* src, c2<R>* dst, const c2<R>* nyq, long nlines, h
     default: return fail(PF_EINVAL, "unsupported nx " + std::to_string(nx));
   }
   return 0;
+}
+}  // namespace
+
+template <typename R>
+int x_c2r(int nx, const c2<R>* src, c2<R>* dst, const c2<R>* nyq, long nlines, hipStream_t s) {
+  return x_c2r_plan<R, 0>(nx, src, dst, nyq, nlines, s);
+}
+int x_c2r_as_xline(int nx, const double2* src, double2* dst, const double2* nyq, long nlines, hipStream_t s) {
+  return x_c2r_plan<double, xline_plan(sizeof(double2))>(nx, src, dst, nyq, nlines, s);
 }
 
 template <typename R>

@@ -123,6 +123,8 @@ __host__ __device__ constexpr int plan_alt(int N, int V, int p) {
   }
   return 0;
 }
+// The x line's transform plan: variant 4 or 5 where it has one, else the default.
+__host__ __device__ constexpr int xline_plan(int cbytes) { return cbytes == 16 ? 5 : 4; }
 __host__ __device__ constexpr int plan_rad(int N, int p, int V = 0) {
   if (V > 0 && plan_alt(N, V, 0)) return plan_alt(N, V, p);
   if (plan_fixed(N, 0)) return plan_fixed(N, p);

@@ -192,8 +192,6 @@ template <typename R, int NX> constexpr int kXlineMaxThreadsN = (sizeof(R) == 8 
 // most 128 VGPRs, which 1024-thread blocks need anyway.  FP64: 3 (the 256-point kernel takes 167 VGPRs).
 template <typename R, int NX>
 constexpr int kXlineWavesN = sizeof(R) == 8 ? 3 : NX >= 512 ? 4 : (NX >= 128 && NX < 192) ? 6 : 5;
-// The x line's transform plan: variant 4 or 5 where it has one, else the default.
-__host__ __device__ constexpr int xline_plan(int cbytes) { return cbytes == 16 ? 5 : 4; }
 __host__ __device__ constexpr int xline_T(int M, int cbytes) { return plan_T(M, xline_plan(cbytes)); }
 // A job's T threads are lanes of one wave: 64 / T jobs a wave, the lanes past them idle.
 __host__ __device__ constexpr int xline_wave_jobs(int M, int cbytes) { return 64 / xline_T(M, cbytes); }

@@ -47,6 +47,8 @@ template <typename R>
 int x_r2c(int nx, const c2<R>* src, c2<R>* dst, c2<R>* nyq, long nlines, R scale, hipStream_t s);
 template <typename R>
 int x_c2r(int nx, const c2<R>* src, c2<R>* dst, const c2<R>* nyq, long nlines, hipStream_t s);
+// With the x line's plan: the bits of k_xline's own inverse x transform.
+int x_c2r_as_xline(int nx, const double2* src, double2* dst, const double2* nyq, long nlines, hipStream_t s);
 template <typename R>
 int y_pass(int ny, bool inv, c2<R>* main, c2<R>* nyq, long M, long nlines, hipStream_t s);
 // Copies between device memory and the caller's (pageable) host arrays on

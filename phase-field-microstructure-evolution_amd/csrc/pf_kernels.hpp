@@ -67,8 +67,8 @@ __device__ __forceinline__ long xcd_runs(long b, long nb, long G) {
 // blocks of one wave (e.g. 8 lines of 8 threads at NX = 256), a 16 KiB tile
 // instead of 64 KiB, which held blocks to two per CU; measured for 17 fields at
 // 256^3: R2C 0.90 -> 0.85 ms, C2R 1.19 -> 1.13 ms.  FP32: lines_per_block.
-template <typename R> __host__ __device__ constexpr int x_lines(int M) {
-  return sizeof(R) == 8 ? ((64 / plan_T(M)) > 0 ? 64 / plan_T(M) : 1) : lines_per_block(M);
+template <typename R> __host__ __device__ constexpr int x_lines(int M, int V = 0) {
+  return sizeof(R) == 8 ? ((64 / plan_T(M, V)) > 0 ? 64 / plan_T(M, V) : 1) : lines_per_block(M);
 }
 
 // ---------------------------------------------------------------------------
@@ -158,15 +158,15 @@ k_x_r2c(const c2<R>* src, c2<R>* dst, c2<R>* __restrict__ nyq, long nlines,
 // ---------------------------------------------------------------------------
 // x pass, inverse: half spectrum lines -> real lines (unnormalised); src and dst
 // may be the same memory (one-pass lengths hold a line in one thread, the others
-// pass a barrier between a block's reads and its writes).
+// pass a barrier between a block's reads and its writes).  V: plan variant.
 // ---------------------------------------------------------------------------
-template <typename R, int NX>
-__global__ void __launch_bounds__(x_lines<R>(NX / 2) * plan_T(NX / 2))
+template <typename R, int NX, int V = 0>
+__global__ void __launch_bounds__(x_lines<R>(NX / 2, V) * plan_T(NX / 2, V))
 k_x_c2r(const c2<R>* src, c2<R>* dst, const c2<R>* __restrict__ nyq, long nlines,
         const c2<R>* __restrict__ tw) {
-  constexpr int M = NX / 2, T = plan_T(M), E = plan_E(M);
-  constexpr int LPB = x_lines<R>(M);
-  __shared__ c2<R> sh[(plan_np(M) > 1) ? LPB * M : 1];
+  constexpr int M = NX / 2, T = plan_T(M, V), E = plan_E(M, V);
+  constexpr int LPB = x_lines<R>(M, V);
+  __shared__ c2<R> sh[(plan_np(M, V) > 1) ? LPB * M : 1];
   const int l = threadIdx.x / T, t = threadIdx.x % T;
   const long line = (long)blockIdx.x * LPB + l;
   const bool act = line < nlines;
@@ -175,9 +175,9 @@ k_x_c2r(const c2<R>* src, c2<R>* dst, const c2<R>* __restrict__ nyq, long nlines
   c2<R> v[E];
   // pre-processing from HBM straight into registers (X_k and X_{M-k} of the line)
 #pragma unroll
-  for (int s = 0; s < kInSlots<M>; ++s) {
-    if (!(act && rfft_in_valid<M>(t, s))) continue;
-    const int k = rfft_in_idx<M>(t, s);
+  for (int s = 0; s < kInSlots<M, V>; ++s) {
+    if (!(act && rfft_in_valid<M, V>(t, s))) continue;
+    const int k = rfft_in_idx<M, V>(t, s);
     if (k == 0) {
       const R a0 = g[0].x, xn = nyq[line].x;
       v[s] = mk<R>(a0 + xn, a0 - xn);
@@ -185,16 +185,16 @@ k_x_c2r(const c2<R>* src, c2<R>* dst, const c2<R>* __restrict__ nyq, long nlines
       v[s] = c2r_pre<R>(g[k], g[M - k], tw[k]);
     }
   }
-  rfft<R, M, true, 1>(v, t, act, sh + ((plan_np(M) > 1) ? l * M : 0), tw, 2);
+  rfft<R, M, true, 1, V>(v, t, act, sh + ((plan_np(M, V) > 1) ? l * M : 0), tw, 2);
   // an in-place pass over a bank that stays in cache (bank_stays) leaves it there
   if (src == dst && bank_stays((unsigned long)nlines * M * sizeof(c2<R>))) {
 #pragma unroll
-    for (int s = 0; s < kOutSlots<M>; ++s)
-      if (act && rfft_out_valid<M>(t, s)) gd[rfft_out_idx<M>(t, s)] = v[s];
+    for (int s = 0; s < kOutSlots<M, V>; ++s)
+      if (act && rfft_out_valid<M, V>(t, s)) gd[rfft_out_idx<M, V>(t, s)] = v[s];
   } else {
 #pragma unroll
-    for (int s = 0; s < kOutSlots<M>; ++s)
-      if (act && rfft_out_valid<M>(t, s)) st_nt<R>(gd + rfft_out_idx<M>(t, s), v[s]);
+    for (int s = 0; s < kOutSlots<M, V>; ++s)
+      if (act && rfft_out_valid<M, V>(t, s)) st_nt<R>(gd + rfft_out_idx<M, V>(t, s), v[s]);
   }
 }
 

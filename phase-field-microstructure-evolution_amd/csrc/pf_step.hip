@@ -685,13 +685,15 @@ int step_faithful(pf_handle* h, bool diag, long rec) {
 }
 
 // The real state of a faithful handle whose last step left it on x-half lines: what
-// every call that steps ends with, whatever it returns.
+// every call that steps ends with, whatever it returns.  The transform is the one the
+// next step's k_xline would have done, so a run gives the same bits however it is
+// split into calls, or into runs by checkpoints.
 int settle_faithful(pf_handle* h) {
   if (!h->fs_half) return 0;
   const Geo& g = h->g;
   h->fs_half = false;
   tbeg(h, ST_X_C2R);
-  const int rc = x_c2r<double>(g.nx, h->fs.main, h->fs.main, h->fs.nyq, (long)g.plane * g.F, h->s);
+  const int rc = x_c2r_as_xline(g.nx, h->fs.main, h->fs.main, h->fs.nyq, (long)g.plane * g.F, h->s);
   tend(h);
   return rc;
 }

@@ -95,20 +95,28 @@ def test_faithful_x_pass(pf, oracle, shape, var):
     _run(pf, oracle, shape, var, "fp64_faithful", 4)
 
 
-@pytest.mark.parametrize("shape,var", [((24, 8, 8), 4), ((256, 8, 8), 13)])
+# every x length of the one-kernel x pass, and one of the three kernels
+@pytest.mark.parametrize("shape,var", [((8, 8, 12), 3), ((12, 8, 8), 5), ((16, 8, 8), 4), ((24, 8, 8), 4),
+                                       ((32, 8, 8), 6), ((48, 8, 8), 5), ((64, 8, 8), 4), ((64, 8, 8), 16),
+                                       ((96, 8, 8), 12), ((128, 8, 8), 12), ((160, 8, 8), 13), ((192, 8, 8), 12),
+                                       ((256, 8, 8), 13), ((512, 8, 8), 12), ((96, 8, 8), 4)])
 def test_faithful_calls_of_any_length_agree(pf, shape, var):
-    """Steps in calls of 1, 2 and 5, and in one call by replayed graphs, bit for bit: a
-    call starts from the real state and its later steps from x-half lines."""
+    """Steps in calls of 1, 2 and 5, in one call by replayed graphs, and with a restart
+    in a new handle from the state of the first four, bit for bit: a call starts from
+    the real state and its later steps from x-half lines."""
     phi, con = pf.ic_voronoi(*shape, var, var + 3)
     p = pf.make_params(**dict(PRM, D_gb=0.4))
     got = []
-    for calls, graphs in (([8], True), ([8], False), ([1] * 8, True), ([2, 5, 1], True)):
-        with pf.Simulation(p, *shape, var, "fp64_faithful") as s:
-            s.set_graphs(graphs)
-            s.put_state(phi, con)
-            for n in calls:
-                s.step(n, diag_every=2)
-            got.append(s.get_state())
+    for runs, graphs in (([[8]], True), ([[8]], False), ([[1] * 8], True), ([[2, 5, 1]], True), ([[4], [4]], True)):
+        state = phi, con
+        for calls in runs:
+            with pf.Simulation(p, *shape, var, "fp64_faithful") as s:
+                s.set_graphs(graphs)
+                s.put_state(*state)
+                for n in calls:
+                    s.step(n, diag_every=2)
+                state = s.get_state()
+        got.append(state)
     for g in got[1:]:
         assert all(np.array_equal(a, b) for a, b in zip(g, got[0]))
 
