@@ -126,11 +126,16 @@ __device__ __forceinline__ void nl_point_faithful(const UPar& u, int V, double c
 // matrix grains, 0 from there on (terms of 0 that leave the sums as they are, and are
 // skipped four at a time), fv the precipitate's.  Nothing is read after a result is
 // given, so put may overwrite the point's values.
+//   What is fused into a multiply-add is written out and nothing else is: left to the
+//   compiler, the choice for products that the energies use too differed between the
+//   two values of DIAG, and with it the last bits of the state between runs that report
+//   other steps.
 constexpr int kNlRegs = 16;
 template <bool DIAG, typename Put>
 __device__ __forceinline__ void nl_point_regs(const UPar& u, int V, double con, const double (&f)[kNlRegs], double fv,
                                               Put put, double& mob, double& ch, double& eta, double& cmax,
                                               double& cmin, double& pmin, double& p3) {
+#pragma clang fp contract(off)
   const int mat = V - 1;
   const double fv2 = fv * fv, fv4 = fv2 * fv2;
   // loop 5
@@ -140,31 +145,31 @@ __device__ __forceinline__ void nl_point_regs(const UPar& u, int V, double con, 
     for (int i = 0; i < kNlRegs - 1; ++i) {
       if (i >= mat) break;
       const double fi2 = f[i] * f[i];
-      fe = (fe - 0.5 * fi2) + 0.25 * (fi2 * fi2);
+      fe = fma(0.25, fi2 * fi2, fma(-0.5, fi2, fe));
       const double g1 = u.s1g * fi2, g2 = u.s2g * fi2;
 #pragma unroll
       for (int j0 = 0; j0 < kNlRegs; j0 += kNlRows) {
         if (j0 + kNlRows - 1 <= i || j0 >= mat) continue;
 #pragma unroll
         for (int j = j0; j < j0 + kNlRows; ++j)
-          if (j > i) fe = fe + g1 * (f[j] * f[j]);
+          if (j > i) fe = fma(g1, f[j] * f[j], fe);
       }
-      fe = fe + g2 * fv2;
+      fe = fma(g2, fv2, fe);
     }
-    fe = (fe - 0.5 * fv2) + 0.25 * fv4;
+    fe = fma(0.25, fv4, fma(-0.5, fv2, fe));
   }
   // loop 6
   double num = 0.0;
 #pragma unroll
   for (int i = 0; i < kNlRegs; ++i) {
     const double f2 = f[i] * f[i];
-    num = num + f2 * f2;
+    num = fma(f2, f2, num);
   }
   const double den = num + fv4;
   const double hm = num / den, hp = 1.0 - hm;
   const double dm = con - u.cm, dp = con - u.cp;
-  const double fch = (hm * u.am) * (dm * dm) + (hp * u.ap) * (dp * dp);
-  put(0, ((2.0 * hm) * u.am) * dm + ((2.0 * hp) * u.ap) * dp);
+  const double fch = fma(hm * u.am, dm * dm, (hp * u.ap) * (dp * dp));
+  put(0, fma((2.0 * hm) * u.am, dm, ((2.0 * hp) * u.ap) * dp));
   // loops 7-9
   const double fm = u.am * (dm * dm), fp = u.ap * (dp * dp);
   const double t2v = (4.0 * (fv2 * fv)) * (den - fv4);
@@ -183,26 +188,26 @@ __device__ __forceinline__ void nl_point_regs(const UPar& u, int V, double con, 
         if (j0 >= mat) continue;
 #pragma unroll
         for (int j = j0; j < j0 + kNlRows; ++j)
-          if (j != i) t2 = t2 + ci * (f[j] * f[j]);
+          if (j != i) t2 = fma(ci, f[j] * f[j], t2);
       }
-      const double term1 = (fi * fi) * fi - fi;
-      t2 = t2 + ((2.0 * u.s2g) * fi) * fv2;
+      const double term1 = fma(fi * fi, fi, -fi);
+      t2 = fma((2.0 * u.s2g) * fi, fv2, t2);
       const double term4 = (((4.0 * ((fi * fi) * fi)) * fv4) * (fm - fp)) / den2;
       put(i + 1, (term1 + t2) + term4);
-      ps = ps + fi * fi;
+      ps = fma(fi, fi, ps);
     }
   }
   {
-    const double term1 = (fv * fv) * fv - fv, c2 = (2.0 * u.s2g) * fv;
+    const double term1 = fma(fv2, fv, -fv), c2 = (2.0 * u.s2g) * fv;
     double t2 = 0.0;
 #pragma unroll
-    for (int j = 0; j < kNlRegs; ++j) t2 = t2 + c2 * (f[j] * f[j]);
+    for (int j = 0; j < kNlRegs; ++j) t2 = fma(c2, f[j] * f[j], t2);
     const double term4 = (t2v * (fp - fm)) / den2;
     put(V, (term1 + t2) + term4);
-    ps = ps + fv * fv;
+    ps = fma(fv, fv, ps);
   }
   // loop 10
-  mob = (u.D + ((2.0 * (1.0 - ps)) * u.Dgb)) - u.D;
+  mob = fma(2.0 * (1.0 - ps), u.Dgb, u.D) - u.D;
   if (DIAG) {
     ch += fch;
     eta += fe;

@@ -121,6 +121,32 @@ def test_faithful_calls_of_any_length_agree(pf, shape, var):
         assert all(np.array_equal(a, b) for a, b in zip(g, got[0]))
 
 
+# the x lengths of the one-kernel x pass, then every z length with the three kernels
+# (more order parameters than the one kernel takes)
+@pytest.mark.parametrize("shape,var", [((8, 8, 12), 3), ((12, 8, 8), 5), ((16, 8, 8), 4), ((24, 8, 8), 4),
+                                       ((32, 8, 8), 6), ((48, 8, 8), 5), ((64, 8, 8), 4), ((96, 8, 8), 12),
+                                       ((128, 8, 8), 12), ((160, 8, 8), 13), ((192, 8, 8), 12), ((256, 8, 8), 13),
+                                       ((512, 8, 8), 12)] +
+                         [((24, 8, nz), 17) for nz in (8, 12, 16, 24, 32, 48, 64, 96, 128, 160, 192, 256, 512)])
+def test_faithful_state_does_not_depend_on_the_rows(pf, shape, var):
+    """Steps with no summary row, a row every second step and one every step end in the
+    same bits, and so does a restart after an odd number of steps, whose rows fall on
+    the other steps."""
+    phi, con = pf.ic_voronoi(*shape, var, var + 3)
+    p = pf.make_params(**dict(PRM, D_gb=0.4))
+    got = []
+    for runs, every in (([8], 0), ([8], 1), ([8], 2), ([3, 5], 2)):
+        state = phi, con
+        for n in runs:
+            with pf.Simulation(p, *shape, var, "fp64_faithful") as s:
+                s.put_state(*state)
+                s.step(n, diag_every=every)
+                state = s.get_state()
+        got.append(state)
+    for g in got[1:]:
+        assert all(np.array_equal(a, b) for a, b in zip(g, got[0]))
+
+
 @pytest.mark.parametrize("mode", ["fp64_faithful", "fp32_mixed"])
 @pytest.mark.parametrize("shape,var", [((12, 12, 12), 1), ((8, 8, 12), 15), ((12, 12, 12), 16), ((8, 12, 12), 17),
                                        ((12, 12, 12), 33)])
