@@ -67,8 +67,14 @@ __device__ __forceinline__ long xcd_runs(long b, long nb, long G) {
 // blocks of one wave (e.g. 8 lines of 8 threads at NX = 256), a 16 KiB tile
 // instead of 64 KiB, which held blocks to two per CU; measured for 17 fields at
 // 256^3: R2C 0.90 -> 0.85 ms, C2R 1.19 -> 1.13 ms.  FP32: lines_per_block.
-template <typename R> __host__ __device__ constexpr int x_lines(int M, int V = 0) {
-  return sizeof(R) == 8 ? ((64 / plan_T(M, V)) > 0 ? 64 / plan_T(M, V) : 1) : lines_per_block(M);
+template <typename R> __host__ __device__ constexpr int x_lines(int M) {
+  return sizeof(R) == 8 ? ((64 / plan_T(M)) > 0 ? 64 / plan_T(M) : 1) : lines_per_block(M);
+}
+// Of k_x_c2r: the same, and one wave where the lines go through LDS (FP32, 1 MiB of 24
+// points: 16.6 us with four waves, 15.9 us with one).
+__host__ __device__ constexpr bool x_c2r_staged(int M, int V) { return plan_T(M, V) <= 2; }
+template <typename R> __host__ __device__ constexpr int x_c2r_lines(int M, int V) {
+  return (sizeof(R) == 8 || x_c2r_staged(M, V)) ? 64 / plan_T(M, V) : lines_per_block(M);
 }
 
 // ---------------------------------------------------------------------------
@@ -157,23 +163,43 @@ k_x_r2c(const c2<R>* src, c2<R>* dst, c2<R>* __restrict__ nyq, long nlines,
 
 // ---------------------------------------------------------------------------
 // x pass, inverse: half spectrum lines -> real lines (unnormalised); src and dst
-// may be the same memory (one-pass lengths hold a line in one thread, the others
-// pass a barrier between a block's reads and its writes).  V: plan variant.
+// may be the same memory (a block passes a barrier between its reads and its
+// writes).  V: plan variant.
+// Short lines, of one or two threads, are read and stored through LDS
+// (x_c2r_staged): a wave's access from its registers touches 16 or 32 bytes of each of
+// 64 or 32 lines, and with the streaming hint those of a cache line go to memory one by
+// one.  C2R of a whole transform, 32 x 64 x 48 FP64, 100 MiB: 366 us from registers
+// (285 us with no hint), 116 us through LDS; one field, 0.8 MiB, 17.1 and 16.9 us.
+// From four threads on a wave's access fills 64 bytes and more (96 x 64 x 48, 99 MiB:
+// 120 us).
 // ---------------------------------------------------------------------------
 template <typename R, int NX, int V = 0>
-__global__ void __launch_bounds__(x_lines<R>(NX / 2, V) * plan_T(NX / 2, V))
+__global__ void __launch_bounds__(x_c2r_lines<R>(NX / 2, V) * plan_T(NX / 2, V))
 k_x_c2r(const c2<R>* src, c2<R>* dst, const c2<R>* __restrict__ nyq, long nlines,
         const c2<R>* __restrict__ tw) {
   constexpr int M = NX / 2, T = plan_T(M, V), E = plan_E(M, V);
-  constexpr int LPB = x_lines<R>(M, V);
-  __shared__ c2<R> sh[(plan_np(M, V) > 1) ? LPB * M : 1];
+  constexpr int LPB = x_c2r_lines<R>(M, V), NT = LPB * T;
+  constexpr bool STAGE = x_c2r_staged(M, V);
+  constexpr int MP = STAGE ? M + 1 : M;  // row pitch in LDS: a short row's lanes start in other banks
+  __shared__ c2<R> sh[(STAGE || plan_np(M, V) > 1) ? LPB * MP : 1];
   const int l = threadIdx.x / T, t = threadIdx.x % T;
-  const long line = (long)blockIdx.x * LPB + l;
-  const bool act = line < nlines;
+  const long l0 = (long)blockIdx.x * LPB, line = l0 + l;
+  const int nl = (int)((nlines - l0) < LPB ? (nlines - l0) : LPB);
+  const bool act = l < nl;
   const c2<R>* g = src + (act ? line : 0) * M;
-  c2<R>* gd = dst + (act ? line : 0) * M;
+  c2<R>* row = sh + ((STAGE || plan_np(M, V) > 1) ? l * MP : 0);
   c2<R> v[E];
-  // pre-processing from HBM straight into registers (X_k and X_{M-k} of the line)
+  if constexpr (STAGE) {
+#pragma unroll
+    for (int q = 0; q < M / T; ++q)
+      if (const int i = threadIdx.x + q * NT; i < nl * M) v[q] = src[l0 * M + i];
+#pragma unroll
+    for (int q = 0; q < M / T; ++q)
+      if (const int i = threadIdx.x + q * NT; i < nl * M) sh[i / M * MP + i % M] = v[q];
+    __syncthreads();
+    g = row;
+  }
+  // pre-processing (X_k and X_{M-k} of the line) straight into registers
 #pragma unroll
   for (int s = 0; s < kInSlots<M, V>; ++s) {
     if (!(act && rfft_in_valid<M, V>(t, s))) continue;
@@ -185,9 +211,26 @@ k_x_c2r(const c2<R>* src, c2<R>* dst, const c2<R>* __restrict__ nyq, long nlines
       v[s] = c2r_pre<R>(g[k], g[M - k], tw[k]);
     }
   }
-  rfft<R, M, true, 1, V>(v, t, act, sh + ((plan_np(M, V) > 1) ? l * M : 0), tw, 2);
+  rfft<R, M, true, 1, V>(v, t, act, row, tw, 2);
   // an in-place pass over a bank that stays in cache (bank_stays) leaves it there
-  if (src == dst && bank_stays((unsigned long)nlines * M * sizeof(c2<R>))) {
+  const bool keep = src == dst && bank_stays((unsigned long)nlines * M * sizeof(c2<R>));
+  if constexpr (STAGE) {
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < kOutSlots<M, V>; ++s)
+      if (rfft_out_valid<M, V>(t, s)) row[rfft_out_idx<M, V>(t, s)] = v[s];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < M / T; ++q)
+      if (const int i = threadIdx.x + q * NT; i < nl * M) {
+        const c2<R> x = sh[i / M * MP + i % M];
+        if (keep) dst[l0 * M + i] = x;
+        else st_nt<R>(dst + l0 * M + i, x);
+      }
+    return;
+  }
+  c2<R>* gd = dst + (act ? line : 0) * M;
+  if (keep) {
 #pragma unroll
     for (int s = 0; s < kOutSlots<M, V>; ++s)
       if (act && rfft_out_valid<M, V>(t, s)) gd[rfft_out_idx<M, V>(t, s)] = v[s];

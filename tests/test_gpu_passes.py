@@ -62,3 +62,27 @@ def test_real_arrays_aligned_for_reals_only(pf, prec, layout):
     assert off.data_ptr() % (2 * x.element_size()) != 0
     assert torch.equal(spec[0], spec[1]) and torch.equal(back[0], back[1])
     assert torch.equal(off, x)  # the source is left alone
+
+
+# The inverse x pass takes lines of up to 32 complex points (nx <= 64) through LDS, 64 or
+# 32 of them a block: 1 field of 96 lines, and 7 of 96, end in a part of a block.
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("nx", [8, 12, 16, 24, 32, 48, 64, 96])
+@pytest.mark.parametrize("batch", [1, 7])
+def test_inverse_of_short_lines(pf, prec, nx, batch):
+    """Against numpy, with the tolerances of the device transforms' tests; nothing is
+    written past the last line."""
+    import torch
+    ny, nz = 12, 8
+    dt, ct, p, tol = ((torch.float64, torch.complex128, pf.PREC_FP64, 1e-13) if prec == "fp64"
+                      else (torch.float32, torch.complex64, pf.PREC_FP32, 5e-6))
+    rng = np.random.default_rng(nx + batch)
+    x = rng.standard_normal((batch, nz, ny, nx))
+    spec = torch.tensor(np.fft.rfftn(x, axes=(1, 2, 3)) / (nx * ny * nz)).to(ct).cuda()
+    back = torch.full((x.size + 64,), 7.0, dtype=dt, device="cuda")
+    torch.cuda.synchronize()
+    pf.fft_c2r_device(nx, ny, nz, batch, p, spec.data_ptr(), back.data_ptr(), pf.LAYOUT_XFAST)
+    torch.cuda.synchronize()
+    back = back.cpu().double().numpy()
+    assert np.abs(back[:x.size].reshape(x.shape) - x).max() < tol * np.abs(x).max()
+    assert (back[x.size:] == 7.0).all()
