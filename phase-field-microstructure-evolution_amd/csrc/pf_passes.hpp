@@ -21,13 +21,25 @@ namespace pf {
 //                   TX, or no multiple of it, carry no padding columns
 //   Nyquist planes: columns are the lines, NY contiguous elements each.
 // A wave's lanes run along whichever of the two is contiguous.  The Nyquist tiles,
-// whose LDS exchanges run at a stride, come first, so that they end under the rest
-// (ypass_grid blocks).
+// whose LDS exchanges run against the lanes, come first, so that they end under the
+// rest (ypass_grid blocks).
 // BATCH: the W banks of every member in mt, ppm panels (and Nyquist lines) per
 // member; main and nyq are unused.
 // ---------------------------------------------------------------------------
 // The grid: an eighth of each kind's tiles (rounded up) per XCD.
 inline unsigned ypass_grid(long tmain, long tnyq) { return (unsigned)(8 * ((tmain + 7) / 8 + (tnyq + 7) / 8)); }
+
+// Whether a Nyquist tile exchanges each line in LDS elements of its own rather than in
+// the tile's column order, where the lanes of a line, TX elements apart, share a bank.
+// With more than one exchange, or 16 threads a line and 8-byte elements, the few
+// Nyquist tiles of a small bank otherwise outlast the rest: a y pass of 24 x 512 x 24 x
+// 6 FP32 20.4 us in column order, 11.6 us in rows; 24 x 192 x 24 x 6 11.3 and 7.7, FP64
+// 10.3 and 8.9; 24 x 256 x 24 x 6 FP32 9.9 and 8.2.  Elsewhere it gains nothing, and the
+// second copy of the transform costs the main block's tiles a little (128 x 256 x 64 x 9
+// FP64 48.2 and 49.3 us; where it is used, 128 x 512 x 64 x 9 FP32 52.8 and 53.9).
+template <typename R> __host__ __device__ constexpr bool ypass_own_rows(int NY) {
+  return plan_np(NY) > 2 || (plan_np(NY) == 2 && plan_T(NY) >= 16 && sizeof(R) == 4);
+}
 
 // KEEP: the bank stays in cache from pass to pass (bank_stays).
 template <typename R, int NY, bool INV, bool BATCH = false, bool KEEP = false>
@@ -91,7 +103,8 @@ k_ypass(c2<R>* __restrict__ main, c2<R>* __restrict__ nyq, long M, long npanels,
     for (int s = 0; s < kInSlots<NY>; ++s)
       if (act && rfft_in_valid<NY>(t, s)) v[s] = ld_nt<R>(gp + (unsigned long)rfft_in_idx<NY>(0, s) * ee);
   }
-  rfft<R, NY, INV, (int)TX>(v, t, KEEP || act, sh + c, tw);
+  if (ypass_own_rows<R>(NY) && isn) rfft<R, NY, INV, 1>(v, t, KEEP || act, sh + c * NY, tw);
+  else rfft<R, NY, INV, (int)TX>(v, t, KEEP || act, sh + c, tw);
   if constexpr (KEEP) {
 #pragma unroll
     for (int s = 0; s < kOutSlots<NY>; ++s)

@@ -86,3 +86,32 @@ def test_inverse_of_short_lines(pf, prec, nx, batch):
     back = back.cpu().double().numpy()
     assert np.abs(back[:x.size].reshape(x.shape) - x).max() < tol * np.abs(x).max()
     assert (back[x.size:] == 7.0).all()
+
+
+# The y pass exchanges the Nyquist planes' lines in rows of their own at three-pass
+# lengths (96, 160, 192, 512) and FP32's 256, else (128) in the tile's column order;
+# 40 lines end in a part of a tile, and 30 MiB take the accesses of a cached bank.
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("ny", [96, 128, 160, 192, 256, 512])
+@pytest.mark.parametrize("mib", [0, 30])
+def test_y_pass_over_the_nyquist_planes(pf, prec, ny, mib):
+    """Transform and inverse against numpy, the Nyquist plane on its own scale."""
+    import torch
+    nx, nz = 12, 8
+    dt, ct, p, tol = ((torch.float64, torch.complex128, pf.PREC_FP64, 1e-13) if prec == "fp64"
+                      else (torch.float32, torch.complex64, pf.PREC_FP32, 5e-6))
+    batch = max(5, (mib << 20) // (nx * ny * nz * torch.tensor([], dtype=dt).element_size()))
+    x = np.random.default_rng(ny).standard_normal((batch, nz, ny, nx))
+    ref = np.fft.rfftn(x, axes=(1, 2, 3)) / (nx * ny * nz)
+    dx = torch.tensor(x, dtype=dt).cuda()
+    spec = torch.empty(ref.shape, dtype=ct, device="cuda")
+    torch.cuda.synchronize()
+    pf.fft_r2c_device(nx, ny, nz, batch, p, dx.data_ptr(), spec.data_ptr(), pf.LAYOUT_XFAST, 1.0 / (nx * ny * nz))
+    torch.cuda.synchronize()
+    err = np.abs(spec.cpu().numpy() - ref)
+    assert err.max() < tol * np.abs(ref).max() and err[..., -1].max() < tol * np.abs(ref[..., -1]).max()
+    dx.zero_()
+    torch.cuda.synchronize()
+    pf.fft_c2r_device(nx, ny, nz, batch, p, spec.data_ptr(), dx.data_ptr(), pf.LAYOUT_XFAST)
+    torch.cuda.synchronize()
+    assert np.abs(dx.cpu().double().numpy() - x).max() < tol * np.abs(x).max()
