@@ -261,8 +261,11 @@ int x_c2r_plan(int nx, const c2<R>* src, c2<R>* dst, const c2<R>* nyq, long nlin
 #define PF_CASE(N)                                                                   \
   case N: {                                                                          \
     constexpr int W = plan_alt(N / 2, V, 0) ? V : 0, LPB = x_c2r_lines<R>(N / 2, W); \
-    hipLaunchKernelGGL((k_x_c2r<R, N, W>), dim3(ceil_div(nlines, LPB)),              \
-                       dim3(LPB * plan_T(N / 2, W)), 0, s, src, dst, nyq, nlines, tw); \
+    constexpr bool SHORT = x_c2r_short(N / 2, W);                                    \
+    auto kernel = SHORT && nlines * N * sizeof(R) >= kStageBytes ? &k_x_c2r<R, N, W, SHORT> \
+                                                                 : &k_x_c2r<R, N, W, false>; \
+    hipLaunchKernelGGL(kernel, dim3(ceil_div(nlines, LPB)), dim3(LPB * plan_T(N / 2, W)), 0, s, src, dst, nyq, \
+                       nlines, tw);                                                  \
     break;                                                                           \
   }
     PF_GRID_SIZES(PF_CASE)

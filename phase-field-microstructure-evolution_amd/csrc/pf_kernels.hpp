@@ -70,12 +70,14 @@ __device__ __forceinline__ long xcd_runs(long b, long nb, long G) {
 template <typename R> __host__ __device__ constexpr int x_lines(int M) {
   return sizeof(R) == 8 ? ((64 / plan_T(M)) > 0 ? 64 / plan_T(M) : 1) : lines_per_block(M);
 }
-// Of k_x_c2r: the same, and one wave where the lines go through LDS (FP32, 1 MiB of 24
-// points: 16.6 us with four waves, 15.9 us with one).
-__host__ __device__ constexpr bool x_c2r_staged(int M, int V) { return plan_T(M, V) <= 2; }
+// Of k_x_c2r: the same, and one wave for short lines (FP32, 1 MiB of 24 points: 16.6 us
+// with four waves, 15.9 us with one).
+__host__ __device__ constexpr bool x_c2r_short(int M, int V) { return plan_T(M, V) <= 2; }
 template <typename R> __host__ __device__ constexpr int x_c2r_lines(int M, int V) {
-  return (sizeof(R) == 8 || x_c2r_staged(M, V)) ? 64 / plan_T(M, V) : lines_per_block(M);
+  return (sizeof(R) == 8 || x_c2r_short(M, V)) ? 64 / plan_T(M, V) : lines_per_block(M);
 }
+
+constexpr unsigned long kStageBytes = 2ul << 20;
 
 // ---------------------------------------------------------------------------
 // Real <-> half-complex x lines on a complex FFT of length M = NX/2.
@@ -165,21 +167,21 @@ k_x_r2c(const c2<R>* src, c2<R>* dst, c2<R>* __restrict__ nyq, long nlines,
 // x pass, inverse: half spectrum lines -> real lines (unnormalised); src and dst
 // may be the same memory (a block passes a barrier between its reads and its
 // writes).  V: plan variant.
-// Short lines, of one or two threads, are read and stored through LDS
-// (x_c2r_staged): a wave's access from its registers touches 16 or 32 bytes of each of
+// STAGE: short lines, of one or two threads (x_c2r_short), are read and stored through
+// LDS: a wave's access from its registers touches 16 or 32 bytes of each of
 // 64 or 32 lines, and with the streaming hint those of a cache line go to memory one by
 // one.  C2R of a whole transform, 32 x 64 x 48 FP64, 100 MiB: 366 us from registers
-// (285 us with no hint), 116 us through LDS; one field, 0.8 MiB, 17.1 and 16.9 us.
-// From four threads on a wave's access fills 64 bytes and more (96 x 64 x 48, 99 MiB:
-// 120 us).
+// (285 us with no hint), 116 us through LDS.  From four threads on a wave's access fills
+// 64 bytes and more (96 x 64 x 48, 99 MiB: 120 us).  Less than kStageBytes goes straight
+// from registers, since then the barriers and the way through LDS count (C2R of 24 x 16 x
+// 16 FP32, 1.1 MiB: 15.6 us straight and 16.0 staged, 2 MiB alike, 4 MiB 19.3 and 19.1).
 // ---------------------------------------------------------------------------
-template <typename R, int NX, int V = 0>
+template <typename R, int NX, int V, bool STAGE>
 __global__ void __launch_bounds__(x_c2r_lines<R>(NX / 2, V) * plan_T(NX / 2, V))
 k_x_c2r(const c2<R>* src, c2<R>* dst, const c2<R>* __restrict__ nyq, long nlines,
         const c2<R>* __restrict__ tw) {
   constexpr int M = NX / 2, T = plan_T(M, V), E = plan_E(M, V);
   constexpr int LPB = x_c2r_lines<R>(M, V), NT = LPB * T;
-  constexpr bool STAGE = x_c2r_staged(M, V);
   constexpr int MP = STAGE ? M + 1 : M;  // row pitch in LDS: a short row's lanes start in other banks
   __shared__ c2<R> sh[(STAGE || plan_np(M, V) > 1) ? LPB * MP : 1];
   const int l = threadIdx.x / T, t = threadIdx.x % T;

@@ -64,11 +64,12 @@ def test_real_arrays_aligned_for_reals_only(pf, prec, layout):
     assert torch.equal(off, x)  # the source is left alone
 
 
-# The inverse x pass takes lines of up to 32 complex points (nx <= 64) through LDS, 64 or
-# 32 of them a block: 1 field of 96 lines, and 7 of 96, end in a part of a block.
+# The inverse x pass takes lines of up to 32 complex points (nx <= 64), 64 or 32 of them a
+# block, from 2 MiB on through LDS: 1 field of 96 lines, 7 of 96, and enough for 2.2 MiB
+# end in a part of a block.
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
 @pytest.mark.parametrize("nx", [8, 12, 16, 24, 32, 48, 64, 96])
-@pytest.mark.parametrize("batch", [1, 7])
+@pytest.mark.parametrize("batch", [1, 7, 0])
 def test_inverse_of_short_lines(pf, prec, nx, batch):
     """Against numpy, with the tolerances of the device transforms' tests; nothing is
     written past the last line."""
@@ -76,6 +77,7 @@ def test_inverse_of_short_lines(pf, prec, nx, batch):
     ny, nz = 12, 8
     dt, ct, p, tol = ((torch.float64, torch.complex128, pf.PREC_FP64, 1e-13) if prec == "fp64"
                       else (torch.float32, torch.complex64, pf.PREC_FP32, 5e-6))
+    batch = batch or int(2.2 * 2 ** 20 / (96 * nx * torch.tensor([], dtype=dt).element_size())) | 1
     rng = np.random.default_rng(nx + batch)
     x = rng.standard_normal((batch, nz, ny, nx))
     spec = torch.tensor(np.fft.rfftn(x, axes=(1, 2, 3)) / (nx * ny * nz)).to(ct).cuda()

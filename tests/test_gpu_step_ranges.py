@@ -95,11 +95,13 @@ def test_faithful_x_pass(pf, oracle, shape, var):
     _run(pf, oracle, shape, var, "fp64_faithful", 4)
 
 
-# every x length of the one-kernel x pass, and one of the three kernels
+# every x length of the one-kernel x pass, one of the three kernels, and short lines of
+# more than 2 MiB, whose inverse goes through LDS
 @pytest.mark.parametrize("shape,var", [((8, 8, 12), 3), ((12, 8, 8), 5), ((16, 8, 8), 4), ((24, 8, 8), 4),
                                        ((32, 8, 8), 6), ((48, 8, 8), 5), ((64, 8, 8), 4), ((64, 8, 8), 16),
                                        ((96, 8, 8), 12), ((128, 8, 8), 12), ((160, 8, 8), 13), ((192, 8, 8), 12),
-                                       ((256, 8, 8), 13), ((512, 8, 8), 12), ((96, 8, 8), 4)])
+                                       ((256, 8, 8), 13), ((512, 8, 8), 12), ((96, 8, 8), 4),
+                                       ((24, 64, 48), 4), ((16, 64, 64), 4)])
 def test_faithful_calls_of_any_length_agree(pf, shape, var):
     """Steps in calls of 1, 2 and 5, in one call by replayed graphs, and with a restart
     in a new handle from the state of the first four, bit for bit: a call starts from
