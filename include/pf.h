@@ -133,7 +133,8 @@ int pf_set_timing(pf_handle* h, int on);
 int pf_set_timing_stages(pf_handle* h, unsigned mask);
 int pf_stage_times(pf_handle* h, double* ms, long* count, int n);
 int pf_stage_name(int stage, char* buf, int len);
-/* Algorithmic HBM bytes of one launch of `stage` for this handle's grid. */
+/* Algorithmic HBM bytes of one of the events that pf_stage_times counts for
+ * `stage`, for this handle's grid and form (0: not given). */
 double pf_stage_bytes(pf_handle* h, int stage);
 /* The HIP stream the handle launches on (hipStream_t). */
 void* pf_stream(pf_handle* h);

@@ -1448,14 +1448,22 @@ extern "C" double pf_stage_bytes(pf_handle* h, int stage) {
   const double Br = (double)g.P * s;                       // one real field
   const double Bc = 2.0 * (double)(g.M + 1) * g.plane * s; // one half spectrum
   const double F = g.F;
+  const bool faithful = h->mode == PF_MODE_FP64_FAITHFUL, mob = h->p.D_gb != 0.0;
+  // the faithful form's forward passes take the state and its derivatives together
+  const double fwd = faithful ? 2.0 * F : F;
   switch (stage) {
     case ST_NONLINEAR:
-      if (h->mode == PF_MODE_FP64_FAITHFUL && faithful_halves(g)) return 3.0 * F * Bc + Br;
-      return 2.0 * F * Br + (h->p.D_gb != 0.0 ? Br : 0.0);
-    case ST_X_R2C: return F * (Br + Bc);
-    case ST_Y_FWD: case ST_Z_FWD: case ST_Z_INV: case ST_Y_INV: return 2.0 * F * Bc;
+      if (faithful) return (faithful_halves(g) ? 3.0 * F * Bc : 2.0 * F * Br) + Br;
+      return 2.0 * F * Br + (mob ? Br : 0.0);
+    case ST_X_R2C: return fwd * (Br + Bc);
+    case ST_Y_FWD: return 2.0 * fwd * Bc;
+    case ST_Z_FWD: case ST_Z_INV: case ST_Y_INV: return 2.0 * F * Bc;
     case ST_X_C2R: return F * (Bc + Br);
-    case ST_UPDATE: return 4.0 * F * Bc;
+    // with the mobility chain two events a step, before it (c up to the chain's field,
+    // the etas) and after it (c): half of what they move together
+    case ST_UPDATE:
+      if (faithful) return (5.0 + 3.0 * g.var + 4.0) / 2.0 * Bc;
+      return mob ? (4.0 + 4.0 * g.var + 5.0) / 2.0 * Bc : 4.0 * F * Bc;
     default: return 0.0;
   }
 }
