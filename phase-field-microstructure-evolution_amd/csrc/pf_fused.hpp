@@ -788,7 +788,7 @@ k_zline(Geo g, UPar u, KTab kt, Bank<R> S, Bank<R> W, Bank<R> X, Bank<R> Y,
         sv[s] = buf_ld<R, AUXS>(rs, ls, (unsigned)(rfft_out_idx<NZ, V>(0, s) * TX) * CB);
         if constexpr (ROLE == ROLE_CMOB) xv[s] = buf_ld<R, 0>(rx, lw, (unsigned)rfft_out_idx<NZ, V>(0, s) * rowb);
       }
-    const long col = col0 + c;
+    const long col = act ? col0 + c : 0;  // a padding column's would be past the tables' end
     const int kx = isn ? g.M : (int)(col % g.M);
     const int ky = isn ? (int)col : (int)(col / g.M);
     const KCol<double> kc = kcol<double>(kt, kx, ky);
