@@ -1,9 +1,10 @@
 """The combined passes at their edges, on the GPU.
 
-  * The faithful form's fused kernels at every z length against the oracle: the
-    point loops handle four rows at a time, so var covers every remainder and the
-    smallest (no matrix grain); the x lengths give main-block rows shorter than a
-    y tile, and no multiple of one.
+  * The faithful form's fused kernels at every z length against the oracle; the x
+    lengths give main-block rows shorter than a y tile, and no multiple of one.
+  * The point loops of the three-kernel faithful step (few fields on lines over 64
+    points, or more than 16 order parameters) take four rows at a time: every
+    remainder of var - 1, on either side of it.
   * A device transform from and to real arrays that are aligned for their reals
     only (no complex access is possible there) equals the aligned one bit for bit.
 
@@ -20,7 +21,12 @@ SHAPES = [(8, 12, 8, 1), (12, 8, 12, 2), (16, 16, 16, 3), (24, 12, 24, 4), (48, 
           (8, 8, 256, 3), (8, 8, 512, 2)]
 
 
-@pytest.mark.parametrize("nx,ny,nz,var", SHAPES)
+# the three-kernel step: var - 1 = 3 .. 8 and 16 .. 20 rows
+POINTS = [(96, 8, 8, 4), (96, 8, 12, 5), (128, 8, 8, 6), (96, 12, 8, 8), (160, 8, 8, 9), (24, 8, 8, 17),
+          (16, 8, 12, 18), (64, 8, 8, 19), (32, 8, 8, 20), (8, 8, 8, 21)]
+
+
+@pytest.mark.parametrize("nx,ny,nz,var", SHAPES + POINTS)
 def test_faithful_step_at_every_z_length(pf, oracle, nx, ny, nz, var):
     prm = dict(t_step=0.005, grad_coeff_phi=1.0, grad_coeff_c=0.8, D_gb=0.4)
     phi, con = pf.ic_voronoi(nx, ny, nz, var, 2 * var + 1, iseed=-(nx + nz))

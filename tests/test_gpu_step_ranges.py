@@ -3,9 +3,9 @@
   * Fields beyond what one round of an x-line block's waves takes: the smallest
     such count and the largest accepted one, against the oracle.
   * Spectra below, within and above the sizes that stay in the last-level cache
-    (24 to 256 MiB): one member and a batch of equal ones take different sides of
-    that rule and agree bit for bit; FP64 forms on the cached side against the
-    oracle.
+    (over 24 and up to 256 MiB, counted without their Nyquist planes): one member and a
+    batch of equal ones take different sides of that rule and agree bit for bit; every
+    form on the cached side, with the mobility chain, against the oracle.
 
 Tolerances: those of the short runs against the oracle (1e-13 for FP64, 2e-6 for
 FP32: 30 times the largest differences measured over the parity shapes)."""
@@ -18,15 +18,16 @@ PRM = dict(t_step=0.005, grad_coeff_phi=1.0, grad_coeff_c=0.8, D_gb=0.0)
 TOL = {"fp64_reduced": 1e-13, "fp64_faithful": 1e-13, "fp32_mixed": 2e-6}
 
 
-def _run(pf, oracle, shape, var, mode, steps, tuning=None):
+def _run(pf, oracle, shape, var, mode, steps, tuning=None, dgb=0.0):
     phi, con = pf.ic_voronoi(*shape, var, var + 3)
-    with pf.Simulation(pf.make_params(**PRM), *shape, var, mode) as sim:
+    prm = dict(PRM, D_gb=dgb)
+    with pf.Simulation(pf.make_params(**prm), *shape, var, mode) as sim:
         if tuning:
             sim.set_tuning(**tuning)
         sim.put_state(phi, con)
         rows = sim.step(steps, diag_every=1)
         gphi, gcon = sim.get_state()
-    od = oracle.run(oracle.make_params(**PRM), phi, con, steps)  # advances phi, con
+    od = oracle.run(oracle.make_params(**prm), phi, con, steps)  # advances phi, con
     tol = TOL[mode]
     err = max(np.abs(gphi - phi).max(), np.abs(gcon - con).max())
     print(f"{mode} {shape} x {var + 1}: {err:.2e}", flush=True)
@@ -53,10 +54,11 @@ def test_lines_per_block_beyond_its_threads(pf, oracle, lines):
     _run(pf, oracle, (160, 8, 8), 24, "fp64_reduced", 3, dict(xline_lines=lines))
 
 
-@pytest.mark.parametrize("members", [3, 14, 28])
+@pytest.mark.parametrize("members", [2, 3, 14, 28, 29])
 def test_batch_on_the_other_side_of_the_cache_rule(pf, members):
-    """A member's spectrum is 9.3 MiB: alone it is streamed, in a batch of 3 and 14
-    (28 and 130 MiB) it stays cached, in one of 28 (260 MiB) it does not fit."""
+    """A member's spectrum is 9 MiB: alone and in a batch of 2 it is streamed, in one of
+    3, 14 and 28 (27, 126 and 252 MiB; from 15 on not together with the carried
+    spectrum's) it stays cached, in one of 29 (261 MiB) it does not fit."""
     n, var = 64, 8
     p = pf.make_params(**PRM)
     phi, con = pf.ic_voronoi(n, n, n, var, 12)
@@ -77,12 +79,24 @@ def test_batch_on_the_other_side_of_the_cache_rule(pf, members):
             s.close()
 
 
-@pytest.mark.parametrize("mode,shape,var", [("fp64_reduced", (64, 64, 64), 11), ("fp64_reduced", (64, 64, 64), 63),
-                                            ("fp64_faithful", (64, 64, 64), 5), ("fp32_mixed", (64, 64, 64), 24)])
-def test_spectra_that_stay_cached(pf, oracle, mode, shape, var):
-    """24.8, 132 and (faithful: the spectra of the state and of its driving forces)
-    24.8 MiB in FP64, 25.8 MiB in FP32."""
-    _run(pf, oracle, shape, var, mode, 2)
+# MiB, and what stays: the reduced forms' W (the carried spectrum S has as many), the
+# faithful form's state and derivatives together, and each transform's own fields
+@pytest.mark.parametrize("mode,shape,var,dgb", [
+    ("fp64_reduced", (64, 64, 64), 11, 0.0),   # 24: streamed, the last that is
+    ("fp64_reduced", (64, 64, 64), 12, 0.4),   # 26: W and S
+    ("fp64_reduced", (64, 64, 64), 63, 0.0),   # 128: W and S, the last that are
+    ("fp64_reduced", (64, 64, 64), 79, 0.4),   # 160: W
+    ("fp32_mixed", (64, 64, 64), 24, 0.4),     # 25: W and S
+    ("fp32_mixed", (96, 64, 64), 99, 0.0),     # 150: W
+    ("fp64_faithful", (64, 64, 64), 5, 0.0),   # 24: streamed
+    ("fp64_faithful", (64, 64, 64), 6, 0.4),   # 28: one-kernel x pass
+    ("fp64_faithful", (128, 32, 64), 12, 0.4),  # 52: the same, longer lines
+    ("fp64_faithful", (96, 64, 64), 5, 0.4),   # 36: three kernels
+    ("fp64_faithful", (48, 64, 64), 18, 0.4),  # 57: three kernels
+    ("fp64_reduced", (160, 128, 160), 3, 0.4),  # 100, and the chain's one field of 25
+    ("fp64_faithful", (160, 128, 160), 3, 0.4)])  # 200, and the chain's one field of 25
+def test_spectra_that_stay_cached(pf, oracle, mode, shape, var, dgb):
+    _run(pf, oracle, shape, var, mode, 2 if shape[0] < 160 else 1, dgb=dgb)
 
 
 # The faithful form's one-kernel x pass: every x length at its largest field count and
@@ -92,7 +106,7 @@ def test_spectra_that_stay_cached(pf, oracle, mode, shape, var):
                                        ((96, 8, 8), 12), ((128, 8, 8), 16), ((160, 8, 8), 12), ((192, 8, 8), 16),
                                        ((256, 8, 8), 16), ((512, 8, 8), 16), ((64, 8, 8), 17)])
 def test_faithful_x_pass(pf, oracle, shape, var):
-    _run(pf, oracle, shape, var, "fp64_faithful", 4)
+    _run(pf, oracle, shape, var, "fp64_faithful", 4, dgb=0.4)
 
 
 # every x length of the one-kernel x pass, one of the three kernels, and short lines of
