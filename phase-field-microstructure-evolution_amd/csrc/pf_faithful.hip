@@ -268,7 +268,7 @@ static int zf_launch(const Geo& g, const UPar& u, const KTab& kt, Bank<double> U
     if (nblocks) *nblocks = grid;                                                                       \
     return 0;                                                                                           \
   }
-    PF_FAITHFUL_SIZES(PF_CASE)
+    PF_GRID_SIZES(PF_CASE)
 #undef PF_CASE
     default: return fail(PF_EINVAL, "unsupported nz");
   }

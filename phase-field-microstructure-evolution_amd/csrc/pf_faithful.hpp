@@ -19,7 +19,4 @@ enum { FZ_ETA = 0, FZ_GHAT = 1, FZ_CMOB = 2 };
 int faithful_z(int role, bool pars, const Geo& g, const UPar& u, const KTab& kt, Bank<double> U, Bank<double> D,
                Bank<double> G, double* part, int f0, int nf, long max_blocks, long* nblocks, hipStream_t s);
 
-#define PF_FAITHFUL_SIZES(X) \
-  X(8) X(12) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(160) X(192) X(256) X(512)
-
 }  // namespace pf

@@ -18,9 +18,6 @@
 
 namespace pf {
 
-#define PF_GRID_SIZES(X) \
-  X(8) X(12) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(160) X(192) X(256) X(512)
-
 bool grid_size_supported(int n) {
   switch (n) {
 #define PF_CASE(N) case N:

@@ -100,15 +100,6 @@ __device__ __forceinline__ c2<R> c2r_pre(c2<R> xk, c2<R> xmk, c2<R> wk) {
   const R cr = wk.x * br + wk.y * bi, ci = wk.x * bi - wk.y * br;
   return mk<R>(ar - ci, ai + cr);
 }
-// Z_k for C2R from the half line x (M entries) and the Nyquist real xn.
-template <typename R, int M>
-__device__ __forceinline__ c2<R> c2r_z(const c2<R>* x, R xn, int k, const c2<R>* __restrict__ tw) {
-  if (k == 0) {
-    const R a0 = x[0].x;
-    return mk<R>(a0 + xn, a0 - xn);
-  }
-  return c2r_pre<R>(x[k], x[M - k], tw[k]);
-}
 
 // ---------------------------------------------------------------------------
 // x pass, forward: real lines (NX) -> half spectrum lines (M main + 1 Nyquist).

@@ -123,14 +123,12 @@ __global__ void __launch_bounds__(NB) k_voronoi_state(Geo g, const double* __res
 }
 
 // ---------------------------------------------------------------------------
-// Loops 5-10, reduced form: O(var) per point using the block structure of gamma
-// (sigma_1 between matrix grains, sigma_2 between a grain and eta_var,
-// src/var_diff.f90:206-218).  In place on the real work bank:
-// (c, eta_1..eta_V) -> (df_dc, df_dphi_1..df_dphi_V); optional (m - D_mean).
+// pf_diagnose's pass over the real state (c, eta_1..eta_V) of a reduced form: energies
+// and extrema, O(var) per point using the block structure of gamma (sigma_1 between
+// matrix grains, sigma_2 between a grain and eta_var, src/var_diff.f90:206-218).
 // ---------------------------------------------------------------------------
-template <typename R, bool DIAG, bool MOB, bool WRITE = true>
-__global__ void __launch_bounds__(NB)
-k_nl_reduced(Geo g, UCoef u, R* __restrict__ w, R* __restrict__ mobd, double* __restrict__ part) {
+template <typename R>
+__global__ void __launch_bounds__(NB) k_energies(Geo g, UCoef u, const R* __restrict__ w, double* __restrict__ part) {
   extern __shared__ unsigned char shraw[];
   R* sh = reinterpret_cast<R*>(shraw);
   double* red = reinterpret_cast<double*>(shraw + sizeof(R) * (size_t)g.var * NB + 16);
@@ -153,60 +151,40 @@ k_nl_reduced(Geo g, UCoef u, R* __restrict__ w, R* __restrict__ mobd, double* __
       pair += a * sm;
       sm += a;
       num += a * a;
-      if (DIAG) fe += a * (R(0.25) * a - R(0.5));
+      fe += a * (R(0.25) * a - R(0.5));
     }
     const R fv = ph[mat * NB], av = fv * fv, av2 = av * av;
     const R d4 = num + av2;
     const R hm = num / d4, hp = R(1) - hm;
     const R dm = con - cm, dp = con - cp;
     const R fm = am * (dm * dm), fpp = ap * (dp * dp);
-    if (WRITE) w[t] = R(2) * hm * am * dm + R(2) * hp * ap * dp;
-    const R inv_d4 = R(1) / d4;
-    const R cT4m = R(4) * (fm - fpp) * (av2 * inv_d4) * inv_d4;
-    if (WRITE) {
-      for (int i = 0; i < mat; ++i) {
-        const R fi = ph[i * NB], a = fi * fi;
-        const R ex = s1g * (sm - a) + s2g * av;
-        w[(long)(i + 1) * g.P + t] = fi * (a - R(1)) + R(2) * fi * ex + cT4m * fi * a;
-      }
-      const R T4v = R(4) * fv * av * hm * (fpp - fm) * inv_d4;
-      w[(long)V * g.P + t] = fv * (av - R(1)) + R(2) * fv * s2g * sm + T4v;
-    }
     const R ps = sm + av;
-    if (MOB && WRITE) mobd[t] = R(2) * (R(1) - ps) * (R)u.Dgb;
-    if (DIAG) {
-      fe += av * (R(0.25) * av - R(0.5)) + s1g * pair + s2g * av * sm;
-      a_ch += (double)(hm * fm + hp * fpp);
-      a_eta += (double)fe;
-      const double dfv = fv, dc = con, dps = ps;
-      if (dfv > p3) p3 = dfv;
-      if (dc <= cmin) cmin = dc;
-      if (dc > cmax) cmax = dc;
-      if (dps < pmin) pmin = dps;
-    }
+    fe += av * (R(0.25) * av - R(0.5)) + s1g * pair + s2g * av * sm;
+    a_ch += (double)(hm * fm + hp * fpp);
+    a_eta += (double)fe;
+    const double dfv = fv, dc = con, dps = ps;
+    if (dfv > p3) p3 = dfv;
+    if (dc <= cmin) cmin = dc;
+    if (dc > cmax) cmax = dc;
+    if (dps < pmin) pmin = dps;
   }
-  if (DIAG) {
-    __syncthreads();
-    const double s0 = block_sum<NB>(a_ch, red), s1 = block_sum<NB>(a_eta, red);
-    const double e0 = block_ext<NB, true>(cmax, red), e1 = block_ext<NB, false>(cmin, red);
-    const double e2 = block_ext<NB, false>(pmin, red), e3 = block_ext<NB, true>(p3, red);
-    if (threadIdx.x == 0) {
-      double* o = part + (long)blockIdx.x * NPART_NL;
-      o[0] = s0; o[1] = s1; o[2] = e0; o[3] = e1; o[4] = e2; o[5] = e3;
-    }
+  __syncthreads();
+  const double s0 = block_sum<NB>(a_ch, red), s1 = block_sum<NB>(a_eta, red);
+  const double e0 = block_ext<NB, true>(cmax, red), e1 = block_ext<NB, false>(cmin, red);
+  const double e2 = block_ext<NB, false>(pmin, red), e3 = block_ext<NB, true>(p3, red);
+  if (threadIdx.x == 0) {
+    double* o = part + (long)blockIdx.x * NPART_NL;
+    o[0] = s0; o[1] = s1; o[2] = e0; o[3] = e1; o[4] = e2; o[5] = e3;
   }
 }
 
 // ---------------------------------------------------------------------------
-// Reduced k-space update for all fields, in place on S, copy into W for the
-// inverse transform; optional Parseval partial sums of the new state for the
-// next step's f_int.  FP32 form keeps each field's k = 0 mode in FP64 (dc64).
-// STILED: S is in the column-tile layout (elem_tiled).
+// f_int of a state from its spectrum, by Parseval's sum with the Nyquist-zeroed
+// wavenumbers, one partial per block.  STILED: S is in the column-tile layout
+// (elem_tiled).
 // ---------------------------------------------------------------------------
-template <typename R, bool DC64, bool MOB, bool PARSEVAL, bool UPD, bool STILED = false>
-__global__ void __launch_bounds__(NB)
-k_update(Geo g, UCoef u, KTab kt, Bank<R> S, Bank<R> W, Bank<R> H, double* __restrict__ dc64,
-         double* __restrict__ part, long nrows) {
+template <typename R, bool STILED>
+__global__ void __launch_bounds__(NB) k_fint(Geo g, UCoef u, KTab kt, Bank<R> S, double* __restrict__ part, long nrows) {
   __shared__ double red[NB];
   double acc = 0.0;
   for (long row = blockIdx.x; row < nrows; row += gridDim.x) {
@@ -214,45 +192,14 @@ k_update(Geo g, UCoef u, KTab kt, Bank<R> S, Bank<R> W, Bank<R> H, double* __res
     const double kap = (r.f == 0) ? u.kc : u.kphi;
     for (int kx = threadIdx.x; kx <= g.M; kx += blockDim.x) {
       const KCoef k = kcoef(kt, kx, r.ky, r.kz);
-      c2<R>* sp = STILED ? elem_tiled(S, g, r.f, kx, r.ky, r.kz) : elem(S, g, r.f, kx, r.ky, r.kz);
-      c2<R> sn = *sp;
-      if (UPD) {
-        const c2<R> w = *elem(W, g, r.f, kx, r.ky, r.kz);
-        if (r.f == 0) {
-          const double den = 1.0 + ((u.D * u.dt) * u.kc) * k.k4;
-          const double A = 1.0 / den, B = ((u.D * k.k2) * u.dt) * A;
-          double re = A * (double)sn.x + B * (double)w.x;
-          double im = A * (double)sn.y + B * (double)w.y;
-          if (MOB) {
-            const c2<R> h = *elem(H, g, 0, kx, r.ky, r.kz);
-            const double C = (u.dt * k.s1) * A;
-            re += -C * (double)h.y;
-            im += C * (double)h.x;
-          }
-          sn = mk<R>((R)re, (R)im);
-        } else {
-          const double A = 1.0 / (1.0 - ((u.L * u.kphi) * u.dt) * k.k2);
-          const double B = -(u.L * u.dt) * A;
-          sn = mk<R>((R)(A * (double)sn.x + B * (double)w.x), (R)(A * (double)sn.y + B * (double)w.y));
-        }
-        if (DC64 && kx == 0 && r.ky == 0 && r.kz == 0) {
-          if (r.f != 0) dc64[r.f] = dc64[r.f] - (u.L * u.dt) * (double)w.x;
-          sn = mk<R>((R)dc64[r.f], R(0));
-        }
-        *sp = sn;
-        *elem(W, g, r.f, kx, r.ky, r.kz) = sn;
-      }
-      if (PARSEVAL) {
-        const double wgt = (kx == 0 || kx == g.M) ? 1.0 : 2.0;
-        const double m2 = (double)sn.x * (double)sn.x + (double)sn.y * (double)sn.y;
-        acc += (0.5 * kap) * wgt * k.kp2 * m2;
-      }
+      const c2<R> sn = STILED ? *elem_tiled(S, g, r.f, kx, r.ky, r.kz) : *elem(S, g, r.f, kx, r.ky, r.kz);
+      const double wgt = (kx == 0 || kx == g.M) ? 1.0 : 2.0;
+      const double m2 = (double)sn.x * (double)sn.x + (double)sn.y * (double)sn.y;
+      acc += (0.5 * kap) * wgt * k.kp2 * m2;
     }
   }
-  if (PARSEVAL) {
-    const double s = block_sum<NB>(acc, red);
-    if (threadIdx.x == 0) part[blockIdx.x] = s * (double)g.P;
-  }
+  const double s = block_sum<NB>(acc, red);
+  if (threadIdx.x == 0) part[blockIdx.x] = s * (double)g.P;
 }
 
 // ---------------------------------------------------------------------------
@@ -334,9 +281,7 @@ struct pf_handle {
   long step = 0;  // completed steps
 
   double* dk = nullptr;
-  float* dkf = nullptr;
   KTab kt{};
-  KTabF ktf{};
 
   // faithful (FP64) banks
   // fs: the state's F fields and, contiguous after them, the F derivatives
@@ -402,10 +347,6 @@ struct DeviceGuard {
 };
 
 namespace {
-
-template <typename R> typename KTabOf<R>::T ktab(const pf_handle* h);
-template <> KTab ktab<double>(const pf_handle* h) { return h->kt; }
-template <> KTabF ktab<float>(const pf_handle* h) { return h->ktf; }
 
 int dalloc(pf_handle* h, void** p, size_t bytes) {
   if (bytes == 0) bytes = 16;
@@ -503,9 +444,6 @@ int ensure_diag(pf_handle* h, long n) {
 // Reduced step (fused kernels).  Between steps W holds the x-half-line state
 // (the spectrum S transformed back along z and y), S the full spectrum.
 // ---------------------------------------------------------------------------
-#define PF_GRID_SIZES(X) \
-  X(8) X(12) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(160) X(192) X(256) X(512)
-
 // ---------------------------------------------------------------------------
 // Batched ensemble: one launch per stage over every member of a group (same
 // grid and var, FP32-mixed form, constant mobility), each member's banks and
@@ -551,8 +489,7 @@ int step_reduced(pf_handle* h, bool diag, long rec, bool fint_next) {
   if (diag && !h->fint_ready) {
     tbeg(h, ST_DIAG);
     const long rows = (long)g.plane * g.F;
-    hipLaunchKernelGGL((k_update<R, false, false, true, false, true>), dim3(grid_for(rows, 1)), dim3(NB), 0, s, g,
-                       h->u, h->kt, S, W, G, h->dc64, h->part_fi, rows);
+    hipLaunchKernelGGL((k_fint<R, true>), dim3(grid_for(rows, 1)), dim3(NB), 0, s, g, h->u, h->kt, S, h->part_fi, rows);
     h->n_part_fi = grid_for(rows, 1);
     tend(h);
   }
@@ -888,14 +825,6 @@ extern "C" int pf_create(const pf_params* p, int nx, int ny, int nz, int var, in
     h->kt.ay = d; h->kt.ayp = d + ny; d += 2 * ny;
     h->kt.az = d; h->kt.azp = d + nz;
     h->kt.uz = (2.0 * (std::atan(1.0) * 4.0)) / (double)(float)nz;  // the unit of kaxis
-    std::vector<float> tabf(tab.begin(), tab.end());
-    if ((rc = dalloc(h, (void**)&h->dkf, sizeof(float) * tabf.size()))) return bail(rc);
-    if (hipMemcpy(h->dkf, tabf.data(), sizeof(float) * tabf.size(), hipMemcpyHostToDevice) != hipSuccess)
-      return bail(fail(PF_EHIP, "copy of wavenumber tables failed"));
-    const float* df = h->dkf;
-    h->ktf.ax = df; h->ktf.axp = df + M + 1; df += 2 * (M + 1);
-    h->ktf.ay = df; h->ktf.ayp = df + ny; df += 2 * ny;
-    h->ktf.az = df; h->ktf.azp = df + nz;
   }
   if (mode == PF_MODE_FP64_FAITHFUL) {
     if ((rc = alloc_bank<double>(h, h->fs, 2 * g.F)) || (rc = alloc_bank<double>(h, h->fdum, 1)) ||
@@ -1368,28 +1297,26 @@ extern "C" int pf_diagnose(pf_handle* h, pf_diag* out) {
     // f_int by Parseval on the transformed state (same quantity as loops 1-4)
     if ((rc = fwd3d_split<double>(h->fs.main, D.main, D.nyq, g.nx, g.ny, g.nz, g.F, 1.0 / (double)(float)g.P, s)))
       return rc;
-    hipLaunchKernelGGL((k_update<double, false, false, true, false>), dim3(grid_for(rows, 1)), dim3(NB), 0, s, g,
-                       h->u, h->kt, D, D, D, h->dc64, h->part_fi, rows);
+    hipLaunchKernelGGL((k_fint<double, false>), dim3(grid_for(rows, 1)), dim3(NB), 0, s, g, h->u, h->kt, D, h->part_fi,
+                       rows);
     h->n_part_fi = grid_for(rows, 1);
     diag_final(h, 0, true, true, (const double*)D.main, nullptr);
   } else {
     const bool f32 = h->mode == PF_MODE_FP32_MIXED;
     if (f32) {
       Bank<float> S{(c2<float>*)h->S_main, nullptr};
-      hipLaunchKernelGGL((k_update<float, false, false, true, false, true>), dim3(grid_for(rows, 1)), dim3(NB), 0, s, g,
-                         h->u, h->kt, S, S, S, h->dc64, h->part_fi, rows);
+      hipLaunchKernelGGL((k_fint<float, true>), dim3(grid_for(rows, 1)), dim3(NB), 0, s, g, h->u, h->kt, S, h->part_fi,
+                         rows);
       const size_t shb = sizeof(float) * (size_t)g.var * NB + 16 + sizeof(double) * NB;
       if ((rc = real_state_reduced<float>(h))) return rc;
-      hipLaunchKernelGGL((k_nl_reduced<float, true, false, false>), dim3(gr_nl), dim3(NB), shb, s, g, h->u,
-                         (float*)h->X_main, (float*)nullptr, h->part_nl);
+      hipLaunchKernelGGL((k_energies<float>), dim3(gr_nl), dim3(NB), shb, s, g, h->u, (const float*)h->X_main, h->part_nl);
     } else {
       Bank<double> S{(c2<double>*)h->S_main, nullptr};
-      hipLaunchKernelGGL((k_update<double, false, false, true, false, true>), dim3(grid_for(rows, 1)), dim3(NB), 0, s, g,
-                         h->u, h->kt, S, S, S, h->dc64, h->part_fi, rows);
+      hipLaunchKernelGGL((k_fint<double, true>), dim3(grid_for(rows, 1)), dim3(NB), 0, s, g, h->u, h->kt, S, h->part_fi,
+                         rows);
       const size_t shb = sizeof(double) * (size_t)g.var * NB + 16 + sizeof(double) * NB;
       if ((rc = real_state_reduced<double>(h))) return rc;
-      hipLaunchKernelGGL((k_nl_reduced<double, true, false, false>), dim3(gr_nl), dim3(NB), shb, s, g, h->u,
-                         (double*)h->X_main, (double*)nullptr, h->part_nl);
+      hipLaunchKernelGGL((k_energies<double>), dim3(gr_nl), dim3(NB), shb, s, g, h->u, (const double*)h->X_main, h->part_nl);
     }
     h->n_part_fi = grid_for(rows, 1);
     h->n_part_nl = gr_nl;

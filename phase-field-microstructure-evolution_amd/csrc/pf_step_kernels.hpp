@@ -10,13 +10,6 @@ struct KTab {
   const double *ax, *axp, *ay, *ayp, *az, *azp;
   double uz;  // 2 pi / nz: az[m] = (double)(float)m_s * uz, m_s = m or m - nz
 };
-// The same tables rounded to FP32, for the FP32-mixed update arithmetic.
-struct KTabF {
-  const float *ax, *axp, *ay, *ayp, *az, *azp;
-};
-template <typename R> struct KTabOf;
-template <> struct KTabOf<double> { using T = KTab; };
-template <> struct KTabOf<float> { using T = KTabF; };
 
 // Per-column (kx, ky fixed) partial sums of the wavenumber combinations and the
 // kz-dependent completion, in precision R: s1 = kf_sum/i, k2 = k_sq, k3 =
@@ -26,8 +19,8 @@ template <> struct KTabOf<float> { using T = KTabF; };
 template <typename R> struct KCol {
   R s1, k2, k3, k4, kp2;  // x + y parts
 };
-template <typename R, typename KT>
-__device__ __forceinline__ KCol<R> kcol(const KT& t, int kx, int ky) {
+template <typename R>
+__device__ __forceinline__ KCol<R> kcol(const KTab& t, int kx, int ky) {
   const R ax = t.ax[kx], axp = t.axp[kx], ay = t.ay[ky], ayp = t.ayp[ky];
   const R x2 = ax * ax, y2 = ay * ay;
   KCol<R> c;
@@ -41,20 +34,8 @@ __device__ __forceinline__ KCol<R> kcol(const KT& t, int kx, int ky) {
 template <typename R> struct KCoefR {
   R s1, k2, k3, k4, kp2;
 };
-template <typename R, typename KT>
-__device__ __forceinline__ KCoefR<R> kcoef_col(const KT& t, const KCol<R>& c, int kz) {
-  const R az = t.az[kz], azp = t.azp[kz];
-  const R z2 = az * az;
-  KCoefR<R> k;
-  k.s1 = c.s1 + azp;
-  k.k2 = c.k2 + -z2;
-  k.k3 = c.k3 + -(azp * z2);
-  k.k4 = c.k4 + (z2 * az) * az;
-  k.kp2 = c.kp2 + azp * azp;
-  return k;
-}
 
-// kcoef_col with a_z and a'_z evaluated instead of read from the table.  The
+// The completion, with a_z and a'_z evaluated instead of read from the table.  The
 // table entry is the one product (double)(float)m_s * (2 pi / nz) (kaxis); the
 // product here is kept out of FMA contraction, so it is rounded on its own and
 // equals the table value bit for bit.  The z-line kernel so avoids a load per

@@ -8,9 +8,6 @@
 
 namespace pf {
 
-#define PF_GRID_SIZES(X) \
-  X(8) X(12) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(160) X(192) X(256) X(512)
-
 // Lines per x-line block: the smallest of 1, 2, 4, 8 that gives the block's
 // transforms at least two waves of work (F*LINES*T >= 128 threads) and fills the
 // lanes of a wave that moves rows (xline_rows_at_once: 96 x 96 lines of 64 points x

@@ -8,9 +8,6 @@
 
 namespace pf {
 
-#define PF_GRID_SIZES(X) \
-  X(8) X(12) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(160) X(192) X(256) X(512)
-
 // Cache policy of a pass over banks of nfields fields (k_zline's KEEP).
 template <typename R> int zline_keep(const Geo& g, long nfields) {
   const unsigned long wb = (unsigned long)nfields * g.P * sizeof(R);
