@@ -117,13 +117,32 @@ def roofline_of(stages, steps):
     return name, avg_ms, achieved, st["bytes"]
 
 
-def stage_kernels(n, lines=1, plan=0, keep="false", zkeep=0):
-    """Kernel behind each timed stage of the FP32 step on an n^3 grid, named as
-    rocprofv3 prints them (lines: x lines per x-line block; plan: the z
-    transforms' radix plan variant; keep, zkeep: the cache policy, by the size of
-    the spectra)."""
+def bank_stays(nbytes):
+    """csrc/pf_fft.hpp: whether a bank of fields stays in the last-level cache."""
+    return (24 << 20) < nbytes <= (256 << 20)
+
+
+def auto_xline_lines(n, var):
+    """csrc/pf_xline_launch.hpp: the x line's lines per block where the tuning leaves it."""
+    half = n // 2
+    threads = {16: 4, 24: 4, 32: 4, 48: 4, 64: 8, 80: 10, 96: 8, 128: 8, 256: 16}.get(half, 1)
+    lines = 1
+    while lines < 8 and lines * half <= 64:
+        lines *= 2
+    while lines < 8 and (var + 1) * lines * threads < 128:
+        lines *= 2
+    return lines
+
+
+def stage_kernels(n, var, lines=1, plan=0):
+    """Kernel behind each timed stage of the FP32 step on an n^3 grid of c + var
+    eta, named as rocprofv3 prints them (lines: x lines per x-line block; plan: the
+    z transforms' radix plan variant)."""
+    bank = 4 * n ** 3 * (var + 1)
+    keep = "true" if bank_stays(bank) else "false"
+    zkeep = 0 if keep == "false" else 2 if bank_stays(2 * bank) else 1
     return {
-        "nonlinear": [f"pf::k_xline<float, {n}, {lines}, false, false, {keep}, false>"],
+        "nonlinear": [f"pf::k_xline<float, {n}, {lines}, false, false, {keep}, false, false>"],
         "y_fwd": [f"pf::k_ypass<float, {n}, false, false, {keep}>"],
         "kspace_update": [f"pf::k_zline<float, {n}, 0, true, false, false, {plan}, {zkeep}>",
                           f"pf::k_zline<float, {n}, 0, true, true, false, {plan}, {zkeep}>"],
@@ -131,14 +150,14 @@ def stage_kernels(n, lines=1, plan=0, keep="false", zkeep=0):
     }
 
 
-STAGE_KERNELS = stage_kernels(256)
+STAGE_KERNELS = stage_kernels(256, 16)
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic_fused_kernels_256x17_fp32.md")
 # The sources that decide what the step kernels read and write and how they are
 # launched; the traffic profile records their hash when it is measured.
 KERNEL_SOURCES = [os.path.join(ROOT, "phase-field-microstructure-evolution_amd", "csrc", f)
-                  for f in ("pf_fused.hpp", "pf_passes.hpp", "pf_xline_launch.hpp", "pf_zline_launch.hpp",
-                            "pf_kernels.hpp", "pf_fft2.hpp", "pf_fft.hpp", "pf_step_kernels.hpp",
-                            "pf_step.hip", "pf_tuned.inc")]
+                  for f in ("pf_fused.hpp", "pf_nl.hpp", "pf_passes.hpp", "pf_launch.hpp", "pf_xline_launch.hpp",
+                            "pf_zline_launch.hpp", "pf_kernels.hpp", "pf_fft2.hpp", "pf_fft.hpp",
+                            "pf_step_kernels.hpp", "pf_step.hip", "pf_fft.hip", "pf_tuned.inc")]
 
 
 def kernel_source_sha16():
@@ -402,7 +421,7 @@ def main():
     avg_ms = dom["ms"] / max(dom["count"], 1)
     kbytes = dom["bytes"]
     achieved = kbytes / (avg_ms * 1e-3) / 1e9 if kbytes > 0 else 0.0
-    lines = tuning["xline_lines"] or 1
+    lines = tuning["xline_lines"] or auto_xline_lines(n, var)
     log(f"fp32_mixed: {ms_step:.3f} ms/step, {gpups:.3e} GPUPS; dominant stage {name} "
         f"{avg_ms:.3f} ms avg ({dom['count']} launches timed), {achieved:.0f} GB/s; "
         f"graph replay without events {dt_graph / args.steps * 1e3:.3f} ms/step")
@@ -463,7 +482,7 @@ def main():
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": measured_traffic(name, n, var),
                      "kernel_source_sha16": kernel_source_sha16(),
-                     "stage": name, "kernel": " / ".join(stage_kernels(n, lines, tuning["zline_plan"]).get(name, [name])),
+                     "stage": name, "kernel": " / ".join(stage_kernels(n, var, lines, tuning["zline_plan"]).get(name, [name])),
                      "avg_launch_ms": avg_ms, "algorithmic_bytes_per_launch": kbytes,
                      "stream_reference": {"achieved": stream, "frac": achieved / stream if stream else None,
                                           "kernel": "torch in-place multiply over the same bytes "
