@@ -77,7 +77,8 @@ k_nl_faithful(Geo g, UPar u, const double* __restrict__ st, double* __restrict__
 // Wavenumbers and updates are evaluated in the reference's order
 // (src/var_diff.f90:932-935, 978-987, 1019-1027).
 // A thread holds two columns' worth of values (2 x 64 VGPRs at 256 points): 2
-// waves per SIMD, which the 64 KiB exchange tile allows too.
+// waves per SIMD, which the 64 KiB exchange tile allows too.  FZ_CMOB, one field of
+// F, holds three and spills 15 VGPRs a lane at 128 points, 9 at 32 and 6 at 256.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ KCol<double> kcol_ref(const KTab& t, int kx, int ky) {
 #pragma clang fp contract(off)

@@ -186,8 +186,8 @@ template <typename R> constexpr int kXlineMaxThreads = sizeof(R) == 4 ? 1024 : 5
 template <typename R, int NX> constexpr int kXlineMaxThreadsN = (sizeof(R) == 8 && NX >= 512) ? 640 : kXlineMaxThreads<R>;
 // Minimum waves per SIMD asked of the register allocator.  FP32: 6 for 128- and
 // 160-point lines, which then take up to 79 VGPRs without spills (160^3 x 9: 114 ->
-// 102 us against asking for 5); 5 for the others (at 192 points 6 spilled 4 VGPRs,
-// 192^3 x 9 145 -> 185 us; at 256 points 23, 512 -> 694 us); 4 for 512-point lines,
+// 102 us against asking for 5); 5 for the others (at 192 points it spills 1 VGPR; 6
+// spilled 4, 192^3 x 9 145 -> 185 us; at 256 points 23, 512 -> 694 us); 4 for 512-point lines,
 // which keep their last transform pass's twiddles in registers (kXlineTwiddleRegs), at
 // most 128 VGPRs, which 1024-thread blocks need anyway.  FP64: 3 (the 256-point kernel takes 167 VGPRs).
 template <typename R, int NX>
@@ -369,8 +369,9 @@ __device__ __forceinline__ void diag_partials(double ch, double eta, double cmax
 // derivatives are written over them: with rows of their own the derivatives left two
 // blocks a CU, 256^3 x 17 4.3 ms.  The separate x inverse, pointwise and x forward
 // kernels moved seven banks of F, this pass three (a
-// step of 256 x 128 x 128 x 17: 1.98 -> 1.61 ms).  At 256 points the live values take
-// 208 VGPRs, two waves per SIMD.
+// step of 256 x 128 x 128 x 17: 1.98 -> 1.61 ms).  At 256 and 512 points the live values
+// take 208 and 200 VGPRs, two waves per SIMD; at three waves it spills 38 to 40 VGPRs a
+// lane at 24 points, 8 to 14 at 96, 2 at 48 and 160, none elsewhere.
 template <typename R, int NX, int LINES, bool XONLY, bool BATCH = false, bool KEEP = false, bool ROUNDS = false,
           bool FAITH = false>
 __global__ void __launch_bounds__((FAITH ? 512 : kXlineMaxThreadsN<R, NX>))

@@ -12,6 +12,15 @@ the code-object metadata are checked:
     most 168 VGPRs (3 waves per SIMD);
   * k_zline at 512 points with the 32-thread plan: at most 128 VGPRs, so two
     512-thread blocks share a CU (it spills a few registers by design).
+And for the faithful step and the forms of banks that stay in cache:
+  * k_xline of cached banks, 96 and 160 points: no spills, at most 102 and 80
+    VGPRs (5 and 6 waves per SIMD); 192 points spills 1;
+  * k_xline's FAITH form: at most 168 VGPRs (3 waves) at 64 points, 256 (2 waves)
+    at 256 and 512, without spills; at 24 points, the worst, at most 40;
+  * k_ypass of cached banks at 192 points, with the second copy of its transform:
+    no spills, at most 80 VGPRs (6 waves);
+  * k_zline of cached banks at 64 and 192 points: no spills;
+  * k_zfaithful at 256 points: 2 waves per SIMD, no spills but FZ_CMOB's 6.
 Needs hipcc, not a GPU."""
 import os
 import re
@@ -43,6 +52,24 @@ def resources(tmp_path_factory):
     lines += [YPASS.format(n=n) for n in (256, 512)]
     lines += [ZLINE.format(n=256, p=p, v=0) for p in ("false", "true")]
     lines += [ZLINE.format(n=512, p=p, v=1) for p in ("false", "true")]
+    for n, l in ((96, 2), (160, 1), (192, 1)):
+        lines.append(XLINE.format(n=n).replace("1, false, false>", "%d, false, false, true>" % l))
+    for n, l in ((24, 8), (64, 8), (256, 1), (512, 1)):
+        lines.append(XLINE.format(n=n).replace("1, false, false>", "%d, false, false, false, false, true>" % l)
+                     .replace("float", "double"))
+    lines.append(YPASS.format(n=192).replace("false, false>", "false, false, true>"))
+    lines += [ZLINE.format(n=n, p="true", v=0).replace("false, 0>", "false, 0, %d>" % k) for n, k in ((64, 2), (192, 1))]
+    return _compile(d, lines)
+
+
+@pytest.fixture(scope="module")
+def faithful(tmp_path_factory):
+    if not os.path.exists(HIPCC):
+        pytest.skip("hipcc not available")
+    return _compile(tmp_path_factory.mktemp("res"), ['#include "%s"' % os.path.join(CSRC, "pf_faithful.hip")])
+
+
+def _compile(d, lines):
     src = d / "res.hip"
     src.write_text("\n".join(lines) + "\n")
     asm = d / "res.s"
@@ -87,3 +114,36 @@ def test_zline_registers(resources):
         assert sp == 0 and vg <= 168, (parseval, vg, sp)
         vg, sp = _find(resources, "k_zline", 512, "Li0ELb1E", parseval, "Lb0ELi1E")
         assert vg <= 128, (parseval, vg, sp)
+
+
+def _exact(res, name):
+    hits = [v for k, v in res.items() if k.startswith("_ZN2pf" + name + "E")]
+    assert len(hits) == 1, (name, sorted(res))
+    return hits[0]
+
+
+@pytest.mark.parametrize("n,lines,vgprs,spills", [(96, 2, 102, 0), (160, 1, 80, 0), (192, 1, 102, 1)])
+def test_xline_of_cached_banks(resources, n, lines, vgprs, spills):
+    vg, sp = _exact(resources, "7k_xlineIfLi%dELi%dELb0ELb0ELb1ELb0ELb0E" % (n, lines))
+    assert vg <= vgprs and sp <= spills, (vg, sp)
+
+
+@pytest.mark.parametrize("n,lines,vgprs,spills", [(24, 8, 168, 40), (64, 8, 168, 0), (256, 1, 256, 0), (512, 1, 256, 0)])
+def test_faithful_x_pass(resources, n, lines, vgprs, spills):
+    vg, sp = _exact(resources, "7k_xlineIdLi%dELi%dELb0ELb0ELb0ELb0ELb1E" % (n, lines))
+    assert vg <= vgprs and sp <= spills, (vg, sp)
+
+
+def test_cached_y_and_z(resources):
+    vg, sp = _exact(resources, "7k_ypassIfLi192ELb0ELb0ELb1E")
+    assert vg <= 80 and sp == 0, (vg, sp)
+    for n, keep in ((64, 2), (192, 1)):
+        vg, sp = _exact(resources, "7k_zlineIfLi%dELi0ELb1ELb1ELb0ELi0ELi%dE" % (n, keep))
+        assert vg <= 168 and sp == 0, (n, vg, sp)
+
+
+def test_faithful_z_registers(faithful):
+    for role, pars in ((0, 0), (0, 1), (1, 0), (1, 1), (2, 0)):
+        for keep in (0, 1):
+            vg, sp = _exact(faithful, "11k_zfaithfulILi256ELi%dELb%dELb%dE" % (role, pars, keep))
+            assert vg <= 256 and sp <= (6 if role == 2 else 0), (role, pars, keep, vg, sp)
