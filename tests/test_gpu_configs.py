@@ -142,8 +142,8 @@ def test_c1_reduced_forms_report_nonfinite(pf, mode):
 # ---------------------------------------------------------------------------
 @pytest.mark.parametrize("shape", [(256, 8, 8), (8, 256, 8), (8, 8, 256)], ids=lambda s: "x".join(map(str, s)))
 def test_c2_faithful_256_point_lines_vs_oracle(pf, oracle, shape):
-    """The faithful form's 256-point kernels (k_grad_zinv<256>, k_x_c2r_sumsq at
-    256, the column passes) with 17 fields, D_gb != 0, against the oracle."""
+    """The faithful form's 256-point kernels (k_xline's FAITH form, k_ypass and
+    k_zfaithful at 256) with 17 fields, D_gb != 0, against the oracle."""
     nx, ny, nz = shape
     var = 16
     prm = dict(VOR, D_gb=0.3)
